@@ -180,17 +180,28 @@ mf_status mf_spmv(mf_tiled *t, const double *d_x, const float *d_x32,
                   double *d_y, int mode, void *stream);
 
 /* Stand-alone SpMV kernel of a handle: MF_SPMV_STREAM (nnz-balanced tile
- * ranges, LDS row accumulators; any sparsity; the default), MF_SPMV_ROWGROUP
- * (one row per lane, four tile-rows per wave; regular sparsity) or
- * MF_SPMV_AUTO (the default).
+ * ranges, LDS row accumulators; any sparsity), MF_SPMV_ROWGROUP (one row per
+ * lane, four tile-rows per wave; regular sparsity), MF_SPMV_STRIP (mode 0: a
+ * layout of row strips built with the handle, one row per lane; mode 1 runs
+ * the streamed kernel) or MF_SPMV_AUTO (the default: strips where the handle
+ * has them, else streamed).
  * No reference counterpart (one kernel form there, src/Mille-feuille-cg.h:97-166). */
 #define MF_SPMV_AUTO (-1)
 #define MF_SPMV_STREAM 0
 #define MF_SPMV_ROWGROUP 1
+#define MF_SPMV_STRIP 2
 mf_status mf_tile_set_spmv_kernel(mf_tiled *t, int kind);
 
+/* Sizes of a device handle's row strips: strips of 64 rows (0: the handle has
+ * none), pieces of rows too long for a strip, whether rows are sorted by
+ * length inside windows, and the entry slots (padding included) stored as one
+ * 32-bit word and in full.  No reference counterpart. */
+mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pieces, int *sorted,
+                             int64_t *packed_slots, int64_t *full_slots);
+
 /* Schedule knob for the autotuner: entries per wave of the stand-alone SpMV
- * (its nnz-balanced tile-row ranges are rebuilt; 0 keeps the current value).
+ * (the streamed kernel's nnz-balanced tile-row ranges are rebuilt, and a
+ * handle on strips goes to the streamed kernel; 0 keeps the current value).
  * No reference counterpart (the reference hardcodes its chunking,
  * src/blockspmv_cpu.h:21-31, and its warp budget, src/main-cg.cu:634). */
 mf_status mf_tile_set_schedule(mf_tiled *t, int spmv_wave_nnz);
@@ -432,7 +443,8 @@ typedef struct mf_tune_report {
 /* Stand-alone SpMV schedule of a handle for mf_spmv `mode` (0 or 1, the
  * handle's current levels): the streamed kernel at 384, 512, 768, 1024, 1536
  * and 2048 entries per wave and, on matrices with regular tile-rows, the
- * row-group kernel (value 0).  The fastest is applied with
+ * row-group kernel (value 0), and for mode 0 the strip kernel (value -1) of a
+ * handle that has strips.  The fastest is applied with
  * mf_tile_set_schedule / mf_tile_set_spmv_kernel.  Allocates and frees its
  * own x, x32 and y.
  * No reference counterpart (the reference's warp budget is fixed,

@@ -6,6 +6,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+#include <vector>
+
 #include "mf_internal.h"
 #include "mf_mlp.h"
 
@@ -46,6 +49,27 @@ struct TileView {
   int tilem;
   int tilenum;
   int npad;
+};
+
+// Several device arrays in one allocation (an allocation and its release cost
+// tens to hundreds of microseconds each): add() every array, then alloc().
+class Slab {
+ public:
+  template <typename T>
+  void add(T **p, size_t n) {
+    *p = nullptr;
+    parts_.push_back({(void **)p, bytes_});
+    bytes_ += (n * sizeof(T) + 255) & ~(size_t)255;
+  }
+  mf_status alloc(void **base) {
+    MF_HIP(hipMalloc(base, bytes_ > 0 ? bytes_ : 256));
+    for (auto &q : parts_) *q.first = (char *)*base + q.second;
+    return MF_OK;
+  }
+
+ private:
+  size_t bytes_ = 0;
+  std::vector<std::pair<void **, size_t>> parts_;
 };
 
 inline TileView view_of(const mf_tiled *t) {

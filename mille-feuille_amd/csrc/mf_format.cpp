@@ -57,6 +57,7 @@ mf_status build_tiles_host(mf_tiled *t, int rowA, int colA, const int *rowptr,
   t->tilem = tm;
   t->tilen = tn;
   t->csrsize = nnz;
+  t->low_given = val_low != nullptr;
 
   // Pass 1: distinct tile columns per tile-row.
   std::vector<int> ntiles(tm, 0);

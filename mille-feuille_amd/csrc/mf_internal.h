@@ -43,6 +43,7 @@ mf_status fail(mf_status code, const std::string &msg);
 // Reference-identical Tile_create output plus the handle's device layout.
 struct DeviceLayout {
   int device = -1;
+  void *slab = nullptr;        // one allocation for the arrays from tile_ptr to diag_tile
   int npad = 0;                // padded vector length = 16 * max(tilem, tilen)
   int *tile_ptr = nullptr;     // tilem+1
   int *tile_col = nullptr;     // tilenum
@@ -84,6 +85,81 @@ struct DeviceLayout {
   int spmv_nheavy = 0;
 };
 
+// Row strips (mf_strips.h).
+constexpr int kStripPacked = 0, kStripFull = 1, kStripNear = 2;
+constexpr int kStripLong = 1;  // flags: a lane of the strip holds a row with pieces
+constexpr int kStripLead = 2;  // flags: the rows' diagonals are in the lead arrays
+constexpr int kLongBit = 1 << 30;  // row map: the row's other entries are in pieces
+// Entries per piece of a row longer than a strip takes.
+constexpr int kPieceEntries = 512;
+
+// off: first entry / 128 in the class's arrays; npair: pairs of entries per
+// lane; base: row that packed (near) columns are relative to: column = base +
+// field - 2^23 (2^15).
+struct StripDesc {
+  uint32_t off;
+  uint16_t npair;
+  uint8_t cls;
+  uint8_t flags;
+  float scale;
+  int base;
+};
+
+// A row whose entries are in pieces: its strip lane (64 * strip + lane), first
+// piece and number of pieces.
+struct LongRow {
+  int row, lane, first, n;
+};
+
+// What the class of a row's strip depends on.  lo: exponent of the lowest set
+// bit of its off-diagonal entries, hi: exponent above its largest, so they are
+// integer multiples q of 2^e, |q| <= 127, if e <= lo and hi - e <= 7.
+struct RowInfo {
+  int8_t lo, hi;
+  uint8_t diag;   // has a diagonal entry
+  uint8_t plain;  // bit 0: finite, FP32 payload = (float) value, columns within 2^22 of
+                  // the row; bit 1: columns within kNearCols
+};
+
+constexpr int kNearCols = 31000;
+
+// Host side of the layout: descriptors (strips, then pieces), the row order
+// of sorted layouts and the long rows.
+struct StripPlan {
+  bool ok = false, sorted = false;
+  int nstrips = 0, nmulti = 0;
+  uint64_t npacked = 0, nfull = 0;   // pairs per lane in words; in values (full, near)
+  bool any_full = false, any_near = false;
+  std::vector<StripDesc> desc;
+  std::vector<int> safe;  // per descriptor, a row of it (the column of its padding)
+  std::vector<int> slot, rowmap, long_of, lane_long, piece_long;
+  std::vector<LongRow> lrow;
+};
+
+// Device arrays and sizes; host copies of the descriptors for the solver
+// schedules.
+struct StripLayout {
+  void *slab = nullptr;  // one allocation for the arrays below
+  int nstrips = 0;   // strips of 64 rows (0: the layout was not built)
+  int npieces = 0;   // pieces of long rows, descriptors nstrips ..
+  int nlong = 0;     // rows with pieces, those longer than a piece first
+  int nmulti = 0;    // rows longer than a piece
+  int sorted = 0;    // rows sorted by length inside windows of strips
+  StripDesc *desc = nullptr;
+  uint32_t *words = nullptr;
+  double *vv = nullptr;
+  float *vf = nullptr;
+  int *vc = nullptr;
+  uint16_t *vh = nullptr;
+  double *lead64 = nullptr;
+  float *lead32 = nullptr;
+  int *rowmap = nullptr;
+  int *lane_long = nullptr;
+  LongRow *lrow = nullptr;
+  int *piece_long = nullptr;
+  std::vector<StripDesc> hdesc;
+};
+
 struct Schedule {
   // Contiguous tile-row ranges, one per persistent wave, balanced on nnz
   // (the vector phases' row ownership).
@@ -120,10 +196,12 @@ struct mf_tiled {
   std::vector<unsigned char> blknnznnz, Tile_csr_Col, Blockcsr_Ptr;
   std::vector<double> Blockcsr_Val;
   std::vector<float> Blockcsr_Val_Low;
+  bool low_given = false;  // Blockcsr_Val_Low is the caller's FP32 copy
   // device payload offsets: each tile's entries start at a multiple of 4
   // (entries padded per tile to a multiple of 4), tilenum+1
   std::vector<int> pay_off;
   mf::DeviceLayout dev;
+  mf::StripLayout strips;
   mf::Schedule sched;
   int sched_waves_for = 0;  // wave count the cached schedule was built for
   // device scratch owned by the handle (solver workspace), grown on demand
@@ -137,7 +215,12 @@ mf_status build_tiles_host(mf_tiled *t, int rowA, int colA, const int *rowptr,
                            const int *colidx, const double *val,
                            const float *val_low);
 // Device upload + payload packing (mf_device.hip).
-mf_status upload_tiles(mf_tiled *t, int device);
+mf_status upload_tiles(mf_tiled *t, int device, const int *rowptr);
+// Row strips of an uploaded handle (mf_strips.hip); rowptr: the CSR row
+// pointers the handle was built from.
+mf_status build_strips(mf_tiled *t, const int *rowptr);
+void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info, StripPlan &p);
+void free_strips(mf_tiled *t);
 void free_device(mf_tiled *t);
 // nnz-balanced contiguous tile-row partition for `nwaves` waves.
 std::vector<int> balance_tilerows(const mf_tiled *t, int nwaves);

@@ -62,10 +62,14 @@ __global__ void k_zero_tail(double *y, int from, int to) {
   if (i < to) y[i] = 0.0;
 }
 
+mf_status launch_spmv_strip(const mf_tiled *t, const double *d_x, double *d_y, hipStream_t s);
+
 mf_status launch_spmv(const mf_tiled *t, const double *d_x, const float *d_x32, double *d_y,
                       int mode, hipStream_t s) {
   const TileView A = view_of(t);
-  if (t->dev.spmv_kernel == MF_SPMV_ROWGROUP) {
+  if (mode == kAll64 && t->dev.spmv_kernel == MF_SPMV_STRIP) {
+    MF_TRY(launch_spmv_strip(t, d_x, d_y, s));
+  } else if (t->dev.spmv_kernel == MF_SPMV_ROWGROUP) {
     const int nwv = (A.tilem + 3) / 4;
     const int blocks = ((nwv + 3) / 4 + 7) / 8 * 8;
     if (A.tilem > 0) {
@@ -136,7 +140,9 @@ extern "C" mf_status mf_stream_copy(const double *d_src, double *d_dst, int64_t 
 extern "C" mf_status mf_tile_set_spmv_kernel(mf_tiled *t, int kind) {
   if (!t) return fail(MF_ERR_ARG, "mf_tile_set_spmv_kernel: null handle");
   if (kind == MF_SPMV_AUTO) kind = default_spmv_kernel(t);
-  if (kind != MF_SPMV_STREAM && kind != MF_SPMV_ROWGROUP)
+  if (kind == MF_SPMV_STRIP && t->strips.nstrips == 0)
+    return fail(MF_ERR_ARG, "mf_tile_set_spmv_kernel: the handle has no row strips");
+  if (kind != MF_SPMV_STREAM && kind != MF_SPMV_ROWGROUP && kind != MF_SPMV_STRIP)
     return fail(MF_ERR_ARG, "mf_tile_set_spmv_kernel: unknown kernel");
   t->dev.spmv_kernel = kind;
   return MF_OK;

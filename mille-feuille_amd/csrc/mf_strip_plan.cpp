@@ -1,0 +1,149 @@
+// mf_strip_plan.cpp -- host side of the row strips (mf_strips.h): row order,
+// classes, widths and long-row pieces.
+#include <algorithm>
+#include <cmath>
+#include <numeric>
+
+#include "mf_internal.h"
+
+namespace mf {
+
+// Rows sorted by length inside windows of kStripWin strips (1024 rows): wide
+// enough that 64 rows of about equal length come together, narrow enough that
+// a strip's stores of y stay in a few cache lines.
+constexpr int kStripWin = 16;
+// Longest row of a sorted layout kept in its strip.
+constexpr int kLongRow = 64;
+
+void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info, StripPlan &P) {
+  const int rows = t->rowA, nstr = (16 * t->tilem + 63) / 64;
+  auto len = [&](int r) { return rowptr[r + 1] - rowptr[r]; };
+  // Unsorted strips where padding every row to the longest of its 64 costs
+  // at most a fifth; otherwise rows are sorted inside windows.
+  long long padded = 0;
+#pragma omp parallel for reduction(+ : padded)
+  for (int s = 0; s < nstr; ++s) {
+    int m = 0;
+    for (int r = 64 * s; r < std::min(rows, 64 * s + 64); ++r) m = std::max(m, len(r));
+    padded += 64LL * m;
+  }
+  const bool sorted = (double)padded > 1.2 * t->csrsize;
+  P.sorted = sorted;
+  P.nstrips = nstr;
+  std::vector<int> &rowmap = P.rowmap;
+  std::vector<LongRow> &lrow = P.lrow;
+  if (sorted) {
+    P.slot.resize(rows);
+    rowmap.assign((size_t)nstr * 64, -1);
+    const int wrows = 64 * kStripWin;
+#pragma omp parallel
+    {
+      std::vector<int> ord;
+#pragma omp for schedule(static)
+      for (int w = 0; w < (rows + wrows - 1) / wrows; ++w) {
+        const int r0 = w * wrows, r1 = std::min(rows, r0 + wrows);
+        ord.resize(r1 - r0);
+        std::iota(ord.begin(), ord.end(), r0);
+        // long rows count as empty: their entries are in pieces
+        auto key = [&](int r) { return len(r) > kLongRow ? 0 : len(r); };
+        std::stable_sort(ord.begin(), ord.end(), [&](int p, int q) { return key(p) > key(q); });
+        for (int i = 0; i < r1 - r0; ++i) {
+          P.slot[ord[i]] = r0 + i;
+          rowmap[r0 + i] = ord[i] | (len(ord[i]) > kLongRow ? kLongBit : 0);
+        }
+      }
+    }
+    // long rows, those of several pieces first
+    for (int many = 1; many >= 0; --many)
+      for (int r = 0; r < rows; ++r)
+        if (len(r) > kLongRow && (len(r) > kPieceEntries) == many) {
+          if (P.long_of.empty()) {
+            P.long_of.assign(rows, -1);
+            P.lane_long.assign((size_t)nstr * 64, -1);
+          }
+          P.long_of[r] = P.lane_long[P.slot[r]] = (int)lrow.size();
+          lrow.push_back(LongRow{r, P.slot[r], 0, 0});
+          P.nmulti += many;
+        }
+    // rows past the matrix (the last tile-row's padding) keep a lane each
+    for (int r = rows; r < 16 * t->tilem; ++r) rowmap[r] = r;
+  }
+  auto row_of = [&](int i) {  // matrix row of strip lane i, or -1
+    const int r = !sorted ? i : rowmap[i] < 0 ? rows : rowmap[i] & (kLongBit - 1);
+    return r < rows ? r : -1;
+  };
+  auto scale_of = [](int lo) { return std::ldexp(1.0f, std::max(-100, std::min(lo, 100))); };
+  auto narrow = [](int lo, int hi) { return hi == -127 || (lo > -100 && hi < 100 && hi - lo <= 7); };
+  auto pairs = [](int n) { return (n + 1) / 2; };
+  // classes and widths
+  P.desc.resize(nstr);
+  P.safe.resize(nstr);
+  int wide = 0;
+#pragma omp parallel for reduction(max : wide)
+  for (int s = 0; s < nstr; ++s) {
+    int lo = 127, hi = -127, m = 0, first = -1;
+    bool lead = true, packed = true, near = true, lng = false;
+    for (int i = 64 * s; i < 64 * s + 64; ++i) {
+      const int r = row_of(i);
+      if (r < 0) {
+        lead = false;
+        continue;
+      }
+      if (first < 0) first = r;
+      lead = lead && info[r].diag;
+      packed = packed && (info[r].plain & 1);
+      if (sorted && len(r) > kLongRow) {
+        lng = true;
+        continue;
+      }
+      near = near && (info[r].plain & 2);
+      lo = std::min<int>(lo, info[r].lo);
+      hi = std::max<int>(hi, info[r].hi);
+      m = std::max(m, len(r));
+    }
+    packed = packed && lead && narrow(lo, hi);
+    if (lead && m > 0) --m;
+    wide = std::max(wide, m);
+    StripDesc d;
+    d.off = 0;
+    d.npair = (uint16_t)pairs(m);
+    d.cls = packed ? kStripPacked : near ? kStripNear : kStripFull;
+    d.flags = (uint8_t)((lng ? kStripLong : 0) | (lead ? kStripLead : 0));
+    d.scale = packed ? scale_of(lo) : 1.0f;
+    d.base = sorted ? s / kStripWin * kStripWin * 64 : 64 * s;
+    P.desc[s] = d;
+    P.safe[s] = std::max(first, 0);
+  }
+  if (wide > 100000) return;  // (unsorted strips of rows this long: no layout)
+  for (size_t h = 0; h < lrow.size(); ++h) {
+    const RowInfo &q = info[lrow[h].row];
+    const bool lead = P.desc[lrow[h].lane >> 6].flags & kStripLead;
+    const int n = len(lrow[h].row) - (lead ? 1 : 0);
+    const bool packed = (q.plain & 1) && (lead || !q.diag) && narrow(q.lo, q.hi);
+    lrow[h].first = (int)P.piece_long.size();
+    lrow[h].n = (n + kPieceEntries - 1) / kPieceEntries;
+    for (int k = 0; k < lrow[h].n; ++k) {
+      StripDesc d;
+      d.off = 0;
+      d.npair = (uint16_t)pairs((std::min(n - k * kPieceEntries, kPieceEntries) + 63) / 64);
+      d.cls = packed ? kStripPacked : kStripFull;
+      d.flags = 0;
+      d.scale = packed ? scale_of(q.lo) : 1.0f;
+      d.base = lrow[h].row;
+      P.desc.push_back(d);
+      P.safe.push_back(lrow[h].row);
+      P.piece_long.push_back((int)h);
+    }
+  }
+  // offsets in each class's arrays
+  for (StripDesc &d : P.desc) {
+    uint64_t &n = d.cls == kStripPacked ? P.npacked : P.nfull;
+    d.off = (uint32_t)n;
+    n += d.npair;
+    P.any_full = P.any_full || (d.cls == kStripFull && d.npair > 0);
+    P.any_near = P.any_near || d.cls == kStripNear;
+  }
+  P.ok = P.npacked <= 0xffffffffull && P.nfull <= 0xffffffffull;
+}
+
+}  // namespace mf

@@ -1,0 +1,236 @@
+// mf_strips.h -- row strips: the device layout with one matrix row per lane,
+// and its product.
+//
+// A strip is 64 rows, one per lane of a wave.  Entry k of all 64 rows is
+// stored together, two entries at a time (lane l's entries 2k and 2k+1 at
+// 128 k + 2 l), so a wave reads its strip with coalesced 8- or 16-byte loads,
+// keeps every row sum in a register and needs neither LDS nor atomics; in a
+// banded matrix the lanes' gathers of x fall in consecutive addresses too.
+// Rows are padded to the longest of their strip.  Where consecutive rows
+// differ too much for that (see build_strips), the rows of each window of
+// kStripWin strips are sorted by length first, and rows longer than
+// kLongRow entries go to pieces: a piece has the layout of a strip whose 64
+// lanes all hold entries of one row.
+//
+// Three classes (where every row of a strip has a diagonal entry, the strip's
+// diagonals are stored apart, the lead: lead64, lead32):
+//   packed (kStripPacked): every entry but the lead in one 32-bit word, column
+//     field << 8 | (q + 128) with value q * scale, |q| <= 127 and scale a power
+//     of two common to the strip.  Used only where that holds every value
+//     exactly (graph Laplacians, constant-coefficient stencils), so the
+//     products are those of the FP64 values; 4 bytes an entry instead of 9.
+//   near (kStripNear): FP64 and FP32 values and 16-bit column fields.
+//   full (kStripFull): FP64 and FP32 values and 32-bit columns.
+// Padding never touches x (its product is replaced by 0), so an infinity or
+// NaN in x reaches exactly the rows that have an entry in its column.
+#pragma once
+
+#include <type_traits>
+
+#include "mf_device.h"
+
+namespace mf {
+
+struct StripView {
+  const StripDesc *desc;   // strips, then pieces
+  const uint32_t *words;   // packed entries
+  const double *vv;        // full entries: FP64 values, FP32 values, columns
+  const float *vf;
+  const int *vc;           // (-1: padding)
+  const uint16_t *vh;      // near columns (0: padding)
+  const double *lead64;    // diagonal of strip lane 64 s + lane
+  const float *lead32;
+  const int *rowmap;       // row of each strip lane (sorted layouts; -1: none), else null
+  const int *lane_long;    // long row of each strip lane (layouts with pieces), else null
+  const LongRow *lrow;     // nlong
+  const int *piece_long;   // long row of each piece
+  int nstrips, npieces, nlong, nmulti, nrows;
+};
+
+inline StripView strip_view_of(const mf_tiled *t) {
+  const StripLayout &s = t->strips;
+  return StripView{s.desc, s.words, s.vv, s.vf, s.vc, s.vh, s.lead64, s.lead32, s.rowmap,
+                   s.lane_long, s.lrow, s.piece_long, s.nstrips, s.npieces, s.nlong, s.nmulti,
+                   16 * t->tilem};
+}
+
+// Row of the lane's strip slot: its row, or -1; `lng` is set for a row whose
+// other entries are in pieces.
+__device__ __forceinline__ int strip_row(const StripView &S, int s, int lane, bool &lng) {
+  lng = false;
+  if (!S.rowmap) {
+    const int r = 64 * s + lane;
+    return r < S.nrows ? r : -1;
+  }
+  const int r = S.rowmap[64 * s + lane];
+  if (r < 0) return -1;
+  lng = (r & kLongBit) != 0;
+  return r & (kLongBit - 1);
+}
+
+// The lane's N word pairs at byte offset vo of the strip's words.
+template <int N>
+__device__ __forceinline__ void strip_load_words(const uint32_t *__restrict__ w, uint32_t vo, uint2 (&r)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) r[i] = ld_at<uint2>(w, vo + 512u * i);
+}
+
+// Adds the products of N loaded word pairs to acc.  xb points 2^23 entries
+// before the strip's base row (an address only: the packed column field is
+// biased by 2^23).
+template <int N, typename XT>
+__device__ __forceinline__ double strip_packed(const uint2 (&w)[N], const XT *xb, float sc, double acc) {
+  XT g[2 * N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    g[2 * i] = ld_at<XT>(xb, (w[i].x >> 8) * (uint32_t)sizeof(XT));
+    g[2 * i + 1] = ld_at<XT>(xb, (w[i].y >> 8) * (uint32_t)sizeof(XT));
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * N; ++i) {
+    const uint32_t u = (i & 1 ? w[i / 2].y : w[i / 2].x) & 255u;
+    // (u - 128) * scale, exact in FP32
+    const float a = __builtin_fmaf((float)u, sc, -128.0f * sc);
+    acc = __builtin_fma((double)a, u ? (double)g[i] : 0.0, acc);
+  }
+  return acc;
+}
+
+// The last pairs of a packed strip: four loaded ones and the np - k (< 4) after them.
+template <typename XT>
+__device__ __forceinline__ double strip_packed_rest(const uint32_t *__restrict__ w, uint32_t vo, int k, int np,
+                                                    const uint2 (&a)[4], const XT *xb, float sc, double acc) {
+  if (np - k >= 2) {
+    uint2 c[2];
+    strip_load_words(w, vo + 512u * k, c);
+    acc = strip_packed(a, xb, sc, acc);
+    acc = strip_packed(c, xb, sc, acc);
+    k += 2;
+  } else {
+    acc = strip_packed(a, xb, sc, acc);
+  }
+  if (np > k) {
+    uint2 c[1];
+    strip_load_words(w, vo + 512u * k, c);
+    acc = strip_packed(c, xb, sc, acc);
+  }
+  return acc;
+}
+
+// N value / column pairs of a full or near strip from the lane's entry e;
+// VT double or float.  Near columns: xb points 2^15 entries before the base.
+template <bool NEAR, int N, typename VT, typename XT>
+__device__ __forceinline__ double strip_full(const VT *__restrict__ v, const void *__restrict__ c, uint32_t e,
+                                             const XT *xb, double acc) {
+  VT a[2 * N];
+  uint32_t j[2 * N];
+  XT g[2 * N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    struct alignas(2 * sizeof(VT)) Pair { VT x, y; };
+    const Pair p = ld_at<Pair>(v, (e + 128u * i) * (uint32_t)sizeof(VT));
+    a[2 * i] = p.x;
+    a[2 * i + 1] = p.y;
+    if constexpr (NEAR) {
+      const uint32_t q = ld_at<uint32_t>(c, (e + 128u * i) * 2u);
+      j[2 * i] = q & 0xffffu;
+      j[2 * i + 1] = q >> 16;
+    } else {
+      const uint2 q = ld_at<uint2>(c, (e + 128u * i) * 4u);
+      j[2 * i] = q.x;
+      j[2 * i + 1] = q.y;
+    }
+  }
+  // (padding gathers an entry that exists: the base row's, or x[0])
+  auto pad = [](uint32_t q) { return NEAR ? q == 0u : (int)q < 0; };
+#pragma unroll
+  for (int i = 0; i < 2 * N; ++i)
+    g[i] = ld_at<XT>(xb, (pad(j[i]) ? (NEAR ? 1u << 15 : 0u) : j[i]) * (uint32_t)sizeof(XT));
+#pragma unroll
+  for (int i = 0; i < 2 * N; ++i) acc = __builtin_fma((double)a[i], pad(j[i]) ? 0.0 : (double)g[i], acc);
+  return acc;
+}
+
+template <bool NEAR, typename VT, typename XT>
+__device__ __forceinline__ double strip_full_sum(const VT *__restrict__ v, const void *__restrict__ c, int np,
+                                                 int lane, const XT *xb, double acc) {
+  const uint32_t e = 2u * lane;
+  int k = 0;
+  for (; k + 4 <= np; k += 4) acc = strip_full<NEAR, 4>(v, c, e + 128u * k, xb, acc);
+  const int rest = np - k;
+  if (rest == 3) return strip_full<NEAR, 3>(v, c, e + 128u * k, xb, acc);
+  if (rest == 2) return strip_full<NEAR, 2>(v, c, e + 128u * k, xb, acc);
+  if (rest == 1) return strip_full<NEAR, 1>(v, c, e + 128u * k, xb, acc);
+  return acc;
+}
+
+// Sum of the lane's entries of a strip or piece (without the lead), added to
+// acc.  XT double or float: the vector; V32: full and near strips
+// multiply the FP32 payload.  Strips of more than four pairs load the next four word pairs
+// before the gathers of the current ones.
+template <bool V32, typename XT>
+__device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc &d, const XT *__restrict__ x,
+                                            int lane, double acc) {
+  const int np = d.npair;
+  if (d.cls == kStripPacked) {
+    const uint32_t *w = S.words + (size_t)d.off * 128;
+    const XT *xb = x + ((ptrdiff_t)d.base - (1 << 23));
+    const uint32_t vo = 8u * lane;
+    if (np <= 4) {
+      if (np == 1) {
+        uint2 a[1];
+        strip_load_words(w, vo, a);
+        return strip_packed(a, xb, d.scale, acc);
+      }
+      if (np == 2) {
+        uint2 a[2];
+        strip_load_words(w, vo, a);
+        return strip_packed(a, xb, d.scale, acc);
+      }
+      if (np == 3) {
+        uint2 a[3];
+        strip_load_words(w, vo, a);
+        return strip_packed(a, xb, d.scale, acc);
+      }
+      if (np == 4) {
+        uint2 a[4];
+        strip_load_words(w, vo, a);
+        return strip_packed(a, xb, d.scale, acc);
+      }
+      return acc;
+    }
+    // (two buffers in turn: a copy of words in flight would wait for them)
+    uint2 a[4], b[4];
+    strip_load_words(w, vo, a);
+    int k = 4;
+    for (;;) {
+      if (np - k < 4) return strip_packed_rest(w, vo, k, np, a, xb, d.scale, acc);
+      strip_load_words(w, vo + 512u * k, b);
+      acc = strip_packed(a, xb, d.scale, acc);
+      k += 4;
+      if (np - k < 4) return strip_packed_rest(w, vo, k, np, b, xb, d.scale, acc);
+      strip_load_words(w, vo + 512u * k, a);
+      acc = strip_packed(b, xb, d.scale, acc);
+      k += 4;
+    }
+  }
+  const size_t o = (size_t)d.off * 128;
+  using VT = typename std::conditional<V32, float, double>::type;
+  const VT *v;
+  if constexpr (V32) v = S.vf + o; else v = S.vv + o;
+  if (d.cls == kStripNear)
+    return strip_full_sum<true>(v, S.vh + o, np, lane, x + ((ptrdiff_t)d.base - (1 << 15)), acc);
+  return strip_full_sum<false>(v, S.vc + o, np, lane, x, acc);
+}
+
+__device__ __forceinline__ StripDesc strip_desc(const StripView &S, int i) {
+  const int4 q = *reinterpret_cast<const int4 *>(S.desc + i);
+  int4 u;
+  u.x = __builtin_amdgcn_readfirstlane(q.x);
+  u.y = __builtin_amdgcn_readfirstlane(q.y);
+  u.z = __builtin_amdgcn_readfirstlane(q.z);
+  u.w = __builtin_amdgcn_readfirstlane(q.w);
+  return __builtin_bit_cast(StripDesc, u);
+}
+
+}  // namespace mf

@@ -1,0 +1,334 @@
+// mf_strips.hip -- builds the row strips of a handle on the GPU from its
+// uploaded tiles (a wave per row; 0.8 ms for 762k rows and 5.3M entries), and
+// the stand-alone product over them.
+#include <algorithm>
+#include <string>
+#include <vector>
+
+#include "mf_strips.h"
+
+namespace mf {
+
+namespace {
+
+// Lane's entries of row r in tile t: [b, e) of the tile's payload.
+__device__ __forceinline__ void tile_row_range(const TileView &A, int t, int r, int &b, int &e) {
+  b = A.rp16[(size_t)t * 16 + r];
+  e = r < 15 ? A.rp16[(size_t)t * 16 + r + 1] : A.tile_nz[t] + 1;
+}
+
+__device__ __forceinline__ int wave_min(int v) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) v = min(v, __shfl_xor(v, m));
+  return v;
+}
+
+// One wave per row, lanes over the tiles of its tile-row.
+__global__ __launch_bounds__(256) void k_row_info(TileView A, int rows, RowInfo *__restrict__ info) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  const int R = row >> 4, r = row & 15;
+  int lo = 127, hi = -127, diag = 0, plain = 1, far = 0;
+  for (int t = A.tile_ptr[R] + lane; t < A.tile_ptr[R + 1]; t += kWave) {
+    int b, e;
+    tile_row_range(A, t, r, b, e);
+    const int c0 = A.tile_col[t] << 4;
+    for (int k = A.tile_off[t] + b; k < A.tile_off[t] + e; ++k) {
+      const int c = c0 + (A.rc[k] & 15);
+      const double v = A.v64[k];
+      far = far || c - row > kNearCols || row - c > kNearCols;
+      plain = plain && A.v32[k] == (float)v && fabs(v) < 1e30 && c - row < (1 << 22) && row - c < (1 << 22);
+      if (c == row && !diag) {
+        diag = 1;
+        continue;
+      }
+      if (v == 0.0) continue;
+      const uint64_t u = __builtin_bit_cast(uint64_t, v);
+      const int ex = (int)((u >> 52) & 2047) - 1023;
+      const uint64_t m = (u & 0xfffffffffffffull) | 0x10000000000000ull;
+      lo = min(lo, ex < -100 ? -127 : ex - 52 + (int)__builtin_ctzll(m));
+      hi = max(hi, ex > 100 ? 127 : ex + 1);
+    }
+  }
+  lo = max(wave_min(lo), -127);
+  hi = -wave_min(-hi);
+  plain = (__ballot(!plain) == 0 ? 1 : 0) | (__ballot(far) == 0 ? 2 : 0);
+  diag = __ballot(diag) != 0;
+  if (lane == 0) info[row] = RowInfo{(int8_t)lo, (int8_t)hi, (uint8_t)diag, (uint8_t)plain};
+}
+
+struct FillArgs {
+  TileView A;
+  const StripDesc *desc;
+  const int *slot;      // strip lane of each row (64 s + lane), null: the row itself
+  const int *long_of;   // long row of each row or -1, null: none
+  const LongRow *lrow;
+  uint32_t *words;
+  double *vv;
+  float *vf;
+  int *vc;
+  uint16_t *vh;
+  double *lead64;
+  float *lead32;
+  int rows, nstrips;
+};
+
+// Entry p of strip lane `lane` (or of a piece's entry order) at descriptor d.
+__device__ __forceinline__ void put_entry(const FillArgs &a, const StripDesc &d, int lane, int p, int col, double v,
+                                          float f) {
+  const size_t i = (size_t)d.off * 128 + (size_t)(p >> 1) * 128 + 2 * lane + (p & 1);
+  if (d.cls == kStripPacked) {
+    const int q = (int)(v / (double)d.scale);  // exact: v = q * scale
+    a.words[i] = (uint32_t)(col - d.base + (1 << 23)) << 8 | (uint32_t)(q + 128);
+  } else {
+    a.vv[i] = v;
+    a.vf[i] = f;
+    if (d.cls == kStripNear)
+      a.vh[i] = (uint16_t)(col - d.base + (1 << 15));
+    else
+      a.vc[i] = col;
+  }
+}
+
+// One wave per row: its entries in tile order to the strip lane (or pieces)
+// of the row; padding was filled before.
+__global__ __launch_bounds__(256) void k_fill_strips(FillArgs a) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= a.rows) return;
+  const TileView &A = a.A;
+  const int R = row >> 4, r = row & 15;
+  const int slot = a.slot ? a.slot[row] : row;
+  const int h = a.long_of ? a.long_of[row] : -1;
+  const StripDesc sd = a.desc[slot >> 6];
+  const bool lead = sd.flags & kStripLead;  // the diagonal goes to the lead
+  const int piece0 = h >= 0 ? a.lrow[h].first : 0;
+  int pos = 0;  // off-diagonal (or all) entries before this batch of tiles
+  for (int t0 = A.tile_ptr[R]; t0 < A.tile_ptr[R + 1]; t0 += kWave) {
+    const int t = t0 + lane;
+    int b = 0, e = 0, dk = -1, c0 = 0, o = 0;
+    if (t < A.tile_ptr[R + 1]) {
+      tile_row_range(A, t, r, b, e);
+      c0 = A.tile_col[t] << 4;
+      o = A.tile_off[t];
+      if (lead && A.tile_col[t] == R)
+        for (int k = e - 1; k >= b; --k)
+          if ((A.rc[o + k] & 15) == r) dk = k;
+    }
+    const int n = e - b - (dk >= 0 ? 1 : 0);
+    int inc = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(inc, d);
+      if (lane >= d) inc += u;
+    }
+    int p = pos + inc - n;
+    pos += __builtin_amdgcn_readlane(inc, 63);
+    for (int k = b; k < e; ++k) {
+      const double v = A.v64[o + k];
+      const float f = A.v32[o + k];
+      if (k == dk) {
+        a.lead64[slot] = v;
+        a.lead32[slot] = f;
+        continue;
+      }
+      const int col = c0 + (A.rc[o + k] & 15);
+      if (h < 0) {
+        put_entry(a, sd, slot & 63, p, col, v, f);
+      } else {
+        // piece entries go round the lanes: entry q of a piece to lane q % 64
+        const int pc = p / kPieceEntries, q = p % kPieceEntries;
+        put_entry(a, a.desc[a.nstrips + piece0 + pc], q & 63, q >> 6, col, v, f);
+      }
+      ++p;
+    }
+  }
+}
+
+// Padding of a strip's packed entries: the word of "no entry" with a column
+// that exists.  One block per descriptor.
+__global__ __launch_bounds__(256) void k_pad_words(const StripDesc *__restrict__ desc, const int *__restrict__ safe,
+                                                   uint32_t *__restrict__ words) {
+  const StripDesc d = desc[blockIdx.x];
+  if (d.cls != kStripPacked) return;
+  const uint32_t w = (uint32_t)(safe[blockIdx.x] - d.base + (1 << 23)) << 8;
+  for (int i = threadIdx.x; i < 128 * d.npair; i += 256) words[(size_t)d.off * 128 + i] = w;
+}
+
+// y of a long row from the sum of its pieces.
+__device__ __forceinline__ void store_long(const StripView &S, const LongRow &lr, double sum,
+                                           const double *__restrict__ x, double *__restrict__ y) {
+  if (S.desc[lr.lane >> 6].flags & kStripLead) sum = __builtin_fma(S.lead64[lr.lane], x[lr.row], sum);
+  y[lr.row] = sum;
+}
+
+// y = A x over strips.  Blocks [0, pblocks): the long rows, a block for each
+// row of several pieces (its waves take the pieces in turn, and their sums
+// are added in piece order through LDS), then a wave for each row of one;
+// these are the longer jobs and start first, dealt round the XCDs.  The other
+// blocks: a strip per wave, each XCD a contiguous eighth of them.
+template <bool PIECES>
+__global__ __launch_bounds__(256, 8) void k_spmv_strip(StripView S, int pblocks, const double *__restrict__ x,
+                                                       double *__restrict__ y) {
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  int b = blockIdx.x;
+  if (PIECES && b < pblocks) {
+    if (b < S.nmulti) {
+      __shared__ double part[4];
+      const LongRow lr = S.lrow[b];
+      double sum = 0.0;
+      for (int k0 = 0; k0 < lr.n; k0 += 4) {
+        double v = 0.0;
+        if (k0 + wv < lr.n)
+          v = wave_sum(strip_sum<false>(S, strip_desc(S, S.nstrips + lr.first + k0 + wv), x, lane, 0.0));
+        __syncthreads();
+        if (lane == 0) part[wv] = v;
+        __syncthreads();
+        sum += ((part[0] + part[1]) + part[2]) + part[3];
+      }
+      if (threadIdx.x == 0) store_long(S, lr, sum, x, y);
+    } else {
+      const int h = S.nmulti + (b - S.nmulti) * 4 + wv;
+      if (h >= S.nlong) return;
+      const LongRow lr = S.lrow[h];
+      const double v = wave_sum(strip_sum<false>(S, strip_desc(S, S.nstrips + lr.first), x, lane, 0.0));
+      if (lane == 0) store_long(S, lr, v, x, y);
+    }
+    return;
+  }
+  if (PIECES) b -= pblocks;
+  const int per_xcd = (gridDim.x - (PIECES ? pblocks : 0)) >> 3;  // both counts are multiples of 8
+  const int s = ((b & 7) * per_xcd + (b >> 3)) * 4 + wv;
+  if (s >= S.nstrips) return;
+  const StripDesc d = strip_desc(S, s);
+  bool lng;
+  const int row = strip_row(S, s, lane, lng);
+  double acc = 0.0;
+  if ((d.flags & kStripLead) && row >= 0) acc = S.lead64[64 * s + lane] * x[row];
+  acc = strip_sum<false>(S, d, x, lane, acc);
+  if (row >= 0 && !lng) y[row] = acc;
+}
+
+template <typename T>
+mf_status upload(T *d, const std::vector<T> &h) {
+  if (!h.empty()) MF_HIP(hipMemcpy(d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
+  return MF_OK;
+}
+
+}  // namespace
+
+mf_status launch_spmv_strip(const mf_tiled *t, const double *d_x, double *d_y, hipStream_t s) {
+  const StripView S = strip_view_of(t);
+  const int sblocks = ((S.nstrips + 3) / 4 + 7) / 8 * 8;
+  const int pblocks = (S.nmulti + (S.nlong - S.nmulti + 3) / 4 + 7) / 8 * 8;
+  if (S.nlong > 0)
+    k_spmv_strip<true><<<pblocks + sblocks, 256, 0, s>>>(S, pblocks, d_x, d_y);
+  else
+    k_spmv_strip<false><<<sblocks, 256, 0, s>>>(S, 0, d_x, d_y);
+  MF_HIP(hipGetLastError());
+  return MF_OK;
+}
+
+void free_strips(mf_tiled *t) {
+  StripLayout &s = t->strips;
+  if (s.slab) (void)hipFree(s.slab);
+  s = StripLayout();
+}
+
+mf_status build_strips(mf_tiled *t, const int *rowptr) {
+  StripLayout &L = t->strips;
+  const int rows = t->rowA;
+  if (rows == 0 || t->tilenum == 0) return MF_OK;
+  const TileView A = view_of(t);
+  std::vector<RowInfo> info(rows);
+  {
+    RowInfo *d = nullptr;
+    MF_HIP(hipMalloc(&d, sizeof(RowInfo) * rows));
+    k_row_info<<<(rows + 3) / 4, 256>>>(A, rows, d);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpy(info.data(), d, sizeof(RowInfo) * rows, hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    if (e != hipSuccess) return fail(MF_ERR_HIP, std::string("build_strips: ") + hipGetErrorString(e));
+  }
+  StripPlan P;
+  plan_strips(t, rowptr, info, P);
+  if (!P.ok) return MF_OK;
+  const int nstr = P.nstrips;
+  const uint64_t np = P.npacked, nf = P.nfull;
+  L.sorted = P.sorted;
+  L.npieces = (int)P.piece_long.size();
+  L.nlong = (int)P.lrow.size();
+  L.nmulti = P.nmulti;
+  L.hdesc = P.desc;
+  int *d_safe = nullptr, *d_slot = nullptr, *d_long = nullptr;
+  Slab slab, tmp;
+  slab.add(&L.desc, P.desc.size());
+  slab.add(&L.words, 128 * np);
+  slab.add(&L.vv, 128 * nf);
+  slab.add(&L.vf, 128 * nf);
+  if (P.any_full) slab.add(&L.vc, 128 * nf);
+  if (P.any_near) slab.add(&L.vh, 128 * nf);
+  slab.add(&L.lead64, 64 * (size_t)nstr);
+  slab.add(&L.lead32, 64 * (size_t)nstr);
+  if (P.sorted) slab.add(&L.rowmap, P.rowmap.size());
+  if (L.nlong > 0) {
+    slab.add(&L.lane_long, P.lane_long.size());
+    slab.add(&L.lrow, P.lrow.size());
+    slab.add(&L.piece_long, P.piece_long.size());
+  }
+  tmp.add(&d_safe, P.safe.size());
+  if (P.sorted) tmp.add(&d_slot, P.slot.size());
+  if (L.nlong > 0) tmp.add(&d_long, P.long_of.size());
+  MF_TRY(slab.alloc(&L.slab));
+  MF_HIP(hipMemset(L.lead64, 0, sizeof(double) * 64 * (size_t)nstr));
+  MF_HIP(hipMemset(L.lead32, 0, sizeof(float) * 64 * (size_t)nstr));
+  if (nf > 0) {
+    MF_HIP(hipMemset(L.vv, 0, sizeof(double) * 128 * nf));
+    MF_HIP(hipMemset(L.vf, 0, sizeof(float) * 128 * nf));
+    if (L.vc) MF_HIP(hipMemset(L.vc, 0xff, sizeof(int) * 128 * nf));
+    if (L.vh) MF_HIP(hipMemset(L.vh, 0, sizeof(uint16_t) * 128 * nf));
+  }
+  // temporaries of the fill
+  void *scratch = nullptr;
+  MF_TRY(tmp.alloc(&scratch));
+  mf_status st = upload(L.desc, P.desc);
+  if (st == MF_OK) st = upload(d_safe, P.safe);
+  if (st == MF_OK && P.sorted) st = upload(L.rowmap, P.rowmap);
+  if (st == MF_OK && P.sorted) st = upload(d_slot, P.slot);
+  if (st == MF_OK && L.nlong > 0) {
+    st = upload(L.lane_long, P.lane_long);
+    if (st == MF_OK) st = upload(L.lrow, P.lrow);
+    if (st == MF_OK) st = upload(L.piece_long, P.piece_long);
+    if (st == MF_OK) st = upload(d_long, P.long_of);
+  }
+  if (st == MF_OK) {
+    k_pad_words<<<(unsigned)P.desc.size(), 256>>>(L.desc, d_safe, L.words);
+    FillArgs a{A, L.desc, d_slot, d_long, L.lrow, L.words, L.vv, L.vf, L.vc, L.vh,
+               L.lead64, L.lead32, rows, nstr};
+    k_fill_strips<<<(rows + 3) / 4, 256>>>(a);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e != hipSuccess) st = fail(MF_ERR_HIP, std::string("build_strips: ") + hipGetErrorString(e));
+  }
+  (void)hipFree(scratch);
+  if (st == MF_OK) L.nstrips = nstr;
+  return st;
+}
+
+}  // namespace mf
+
+using namespace mf;
+
+extern "C" mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pieces, int *sorted,
+                                        int64_t *packed_slots, int64_t *full_slots) {
+  if (!t) return fail(MF_ERR_ARG, "mf_tile_strip_info: null handle");
+  const StripLayout &L = t->strips;
+  int64_t n[2] = {0, 0};
+  if (L.nstrips > 0)
+    for (const StripDesc &d : L.hdesc) n[d.cls == kStripPacked ? 0 : 1] += 128 * (int64_t)d.npair;
+  if (strips) *strips = L.nstrips;
+  if (pieces) *pieces = L.npieces;
+  if (sorted) *sorted = L.sorted;
+  if (packed_slots) *packed_slots = n[0];
+  if (full_slots) *full_slots = n[1];
+  return MF_OK;
+}

@@ -39,53 +39,119 @@ namespace mf {
 constexpr int kPad = 64;
 constexpr int kSpmvWaveNnz = 1024;
 
-__global__ void k_pack_payloads(int T, const int *__restrict__ off, const double *__restrict__ v64,
-                                float *__restrict__ v32, uint16_t *__restrict__ v16,
-                                int8_t *__restrict__ v8, float *__restrict__ s16,
-                                float *__restrict__ s8, double *__restrict__ qerr,
-                                double *__restrict__ amax) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= T) return;
-  const int a = off[t], b = off[t + 1];
+// Host arrays of the tiles as uploaded for the packing.
+struct PackSrc {
+  const double *val;      // csrsize values, tile by tile
+  const float *low;       // the caller's FP32 copy, or null: (float) value
+  const uint8_t *col;     // column nibble of each value
+  const uint8_t *ptr;     // row starts: 16 per tile, `hlast` per tile of the last tile-row
+  const int *off;         // tilenum + 1 value offsets
+  int tlast, hlast;       // first tile and rows of the last tile-row
+};
+
+struct PackDst {
+  const int *tile_off;
+  uint8_t *tile_nz, *rc, *rp16;
+  double *v64;
+  float *v32;
+  uint16_t *v16;
+  int8_t *v8;
+  float *s16, *s8;
+  double *qerr, *amax;
+};
+
+__device__ __forceinline__ double max16(double v) {
+#pragma unroll
+  for (int m = 8; m >= 1; m >>= 1) v = fmax(v, __shfl_xor(v, m));
+  return v;
+}
+
+// Tile-row of every tile and the diagonal tile of every tile-row: 16 lanes
+// per tile-row.
+__global__ __launch_bounds__(256) void k_tile_rows(int tm, const int *__restrict__ tile_ptr,
+                                                   const int *__restrict__ tile_col, int *__restrict__ tile_row,
+                                                   int *__restrict__ diag) {
+  const int r = blockIdx.x * 16 + (threadIdx.x >> 4);
+  if (r >= tm) return;
+  for (int t = tile_ptr[r] + (threadIdx.x & 15); t < tile_ptr[r + 1]; t += 16) {
+    tile_row[t] = r;
+    if (tile_col[t] == r) diag[r] = t;
+  }
+}
+
+// Payload layout of one tile per 16 lanes, lane r packing row r: entries
+// padded per tile to a multiple of 4 (zero values that repeat the tile's last
+// (row,col) byte), so every 4-entry chunk of the streamed SpMV lies in one
+// tile; the FP32 / FP16 / INT8 copies, their scales and errors; the 16 row
+// starts (rows past the last row of a short final tile-row start at the
+// tile's nnz, which is then <= 15*16) and nnz - 1.  A thread per tile took
+// 0.20 ms for the 525k tiles of a 90 x 91 x 93 Laplacian, and its inputs were
+// packed row by row on the host (20 ms).
+__global__ __launch_bounds__(256) void k_pack_tiles(int T, PackSrc s, PackDst d) {
+  const int t = blockIdx.x * 16 + (threadIdx.x >> 4), r = threadIdx.x & 15;
+  if (t >= T) return;  // (alike in the 16 lanes that share a reduction)
+  const int o = s.off[t], nz = s.off[t + 1] - o, po = d.tile_off[t], pz = d.tile_off[t + 1] - po;
+  const int h = t >= s.tlast ? s.hlast : 16;
+  const uint8_t *rp = s.ptr + (t >= s.tlast ? (size_t)s.tlast * 16 + (size_t)(t - s.tlast) * s.hlast : (size_t)t * 16);
+  const int b = r < h ? rp[r] : nz, e = r < h - 1 ? rp[r + 1] : nz;
   double m = 0.0;
-  for (int k = a; k < b; ++k) m = fmax(m, fabs(v64[k]));
-  amax[t] = m;
+  for (int k = b; k < e; ++k) m = fmax(m, fabs(s.val[o + k]));
+  m = max16(m);
   // FP16: power-of-two scale 2^e with e = floor(log2 max|a|), so the scaled
   // magnitudes lie in [.., 2); scaling by a power of two is exact in FP32, so
   // for in-range tiles the stored value equals (half)(float)a.
-  int e = m > 0.0 ? ilogb(m) : 0;
-  e = e < -100 ? -100 : (e > 100 ? 100 : e);
-  const float sc16 = ldexpf(1.0f, e);
-  const float inv16 = ldexpf(1.0f, -e);
+  int x = m > 0.0 ? ilogb(m) : 0;
+  x = x < -100 ? -100 : (x > 100 ? 100 : x);
+  const float sc16 = ldexpf(1.0f, x);
+  const float inv16 = ldexpf(1.0f, -x);
   // INT8: smallest power-of-two scale with max|a|/scale <= 127 (exact
   // division; tiles of multiples of the scale, such as the -1 couplings of a
   // Laplacian, are stored exactly), round to nearest even.
   float sc8 = 1.0f;
   if (m > 0.0) {
-    int e8 = ilogb(m / 127.0);
-    if (ldexp(127.0, e8) < m) ++e8;
-    e8 = e8 < -120 ? -120 : (e8 > 120 ? 120 : e8);
-    sc8 = ldexpf(1.0f, e8);
+    int x8 = ilogb(m / 127.0);
+    if (ldexp(127.0, x8) < m) ++x8;
+    x8 = x8 < -120 ? -120 : (x8 > 120 ? 120 : x8);
+    sc8 = ldexpf(1.0f, x8);
   }
-  s16[t] = sc16;
-  s8[t] = sc8;
   double e32 = 0.0, e16 = 0.0, e8 = 0.0;
-  for (int k = a; k < b; ++k) {
-    const double v = v64[k];
+  for (int k = b; k < e; ++k) {
+    const double v = s.val[o + k];
+    const int c = s.col[o + k], i = po + k;
+    d.rc[i] = (uint8_t)((r << 4) | c);
+    d.v64[i] = v;
     const float f = (float)v;
-    v32[k] = f;
+    d.v32[i] = s.low ? s.low[o + k] : f;
     e32 = fmax(e32, fabs(v - (double)f));
-    const _Float16 h = (_Float16)(f * inv16);
-    v16[k] = __builtin_bit_cast(uint16_t, h);
-    e16 = fmax(e16, fabs(v - (double)((float)h * sc16)));
+    const _Float16 g = (_Float16)(f * inv16);
+    d.v16[i] = __builtin_bit_cast(uint16_t, g);
+    e16 = fmax(e16, fabs(v - (double)((float)g * sc16)));
     double q = rint(v / (double)sc8);
     q = q > 127.0 ? 127.0 : (q < -127.0 ? -127.0 : q);
-    v8[k] = (int8_t)q;
+    d.v8[i] = (int8_t)q;
     e8 = fmax(e8, fabs(v - q * (double)sc8));
+    if (k == nz - 1)
+      for (int z = nz; z < pz; ++z) {
+        d.rc[po + z] = (uint8_t)((r << 4) | c);
+        d.v64[po + z] = 0.0;
+        d.v32[po + z] = 0.0f;
+        d.v16[po + z] = 0;
+        d.v8[po + z] = 0;
+      }
   }
-  qerr[t] = e32;
-  qerr[T + t] = e16;
-  qerr[2 * T + t] = e8;
+  e32 = max16(e32);
+  e16 = max16(e16);
+  e8 = max16(e8);
+  d.rp16[(size_t)t * 16 + r] = (uint8_t)b;
+  if (r == 0) {
+    d.tile_nz[t] = (uint8_t)(nz - 1);
+    d.s16[t] = sc16;
+    d.s8[t] = sc8;
+    d.amax[t] = m;
+    d.qerr[t] = e32;
+    d.qerr[T + t] = e16;
+    d.qerr[2 * T + t] = e8;
+  }
 }
 
 template <typename T>
@@ -102,7 +168,7 @@ static mf_status dalloc(T **p, size_t n) {
 
 mf_status upload_spmv_schedule(mf_tiled *t, int wave_nnz);
 
-mf_status upload_tiles(mf_tiled *t, int device) {
+mf_status upload_tiles(mf_tiled *t, int device, const int *rowptr) {
   DeviceLayout &d = t->dev;
   MF_HIP(hipSetDevice(device));
   d.device = device;
@@ -110,13 +176,7 @@ mf_status upload_tiles(mf_tiled *t, int device) {
   d.npad = kTile * std::max(t->tilem, t->tilen);
   if (d.npad == 0) d.npad = kTile;
 
-  // Payload layout: each tile's entries start at a multiple of 4 (padded per
-  // tile to a multiple of 4 with zero values that repeat the tile's last
-  // (row,col) byte), so every 4-entry chunk of the streamed SpMV lies in one
-  // tile.  Per entry: (row << 4) | col inside the tile, from the tile's row
-  // starts.  Per tile: the 16 row starts (rows past the last row of a short
-  // final tile-row start at the tile's nnz, which is then <= 15*16) and
-  // nnz - 1.
+  // payload offsets: each tile's entries padded to a multiple of 4
   std::vector<int> &poff = t->pay_off;
   poff.assign(T + 1, 0);
   for (int tt = 0; tt < T; ++tt) {
@@ -125,82 +185,77 @@ mf_status upload_tiles(mf_tiled *t, int device) {
   }
   const int ZP = poff[T];
   d.npay = ZP;
-  std::vector<int> tile_row(T);
-  std::vector<uint8_t> rc((size_t)ZP + kPad, 0);
-  std::vector<uint8_t> tnz(T > 0 ? T : 1, 0);
-  std::vector<double> v64((size_t)ZP + kPad, 0.0);
-  std::vector<float> v32((size_t)ZP + kPad, 0.0f);
-  std::vector<uint8_t> rp16((size_t)T * kTile + kPad, 0);
-  std::vector<int> diag(TM, -1);
   int max_tiles = 0;
-  for (int bi = 0; bi < TM; ++bi) {
-    const int h = bi == TM - 1 ? t->rowA - (TM - 1) * kTile : kTile;
-    max_tiles = std::max(max_tiles, t->tile_ptr[bi + 1] - t->tile_ptr[bi]);
-    for (int tt = t->tile_ptr[bi]; tt < t->tile_ptr[bi + 1]; ++tt) {
-      tile_row[tt] = bi;
-      if (t->tile_columnidx[tt] == bi) diag[bi] = tt;
-      const int off = t->csr_offset[tt], nzt = t->csr_offset[tt + 1] - off;
-      const int po = poff[tt];
-      tnz[tt] = (uint8_t)(nzt - 1);
-      const unsigned char *rp = &t->Blockcsr_Ptr[t->csrptr_offset[tt]];
-      for (int r = 0; r < kTile; ++r) rp16[(size_t)tt * kTile + r] = (uint8_t)(r < h ? rp[r] : nzt);
-      for (int r = 0; r < h; ++r) {
-        const int e = r == h - 1 ? nzt : rp[r + 1];
-        for (int k = rp[r]; k < e; ++k)
-          rc[po + k] = (uint8_t)((r << 4) | t->Tile_csr_Col[off + k]);
-      }
-      for (int k = 0; k < nzt; ++k) {
-        v64[po + k] = t->Blockcsr_Val[off + k];
-        v32[po + k] = t->Blockcsr_Val_Low[off + k];
-      }
-      for (int k = nzt; k < poff[tt + 1] - po; ++k) rc[po + k] = rc[po + nzt - 1];
-    }
-  }
+  for (int bi = 0; bi < TM; ++bi) max_tiles = std::max(max_tiles, t->tile_ptr[bi + 1] - t->tile_ptr[bi]);
   d.max_tiles_per_row = max_tiles;
-  d.spmv_kernel = default_spmv_kernel(t);
-  MF_TRY(dalloc(&d.tile_ptr, TM + 1));
-  MF_TRY(dalloc(&d.tile_col, T));
-  MF_TRY(dalloc(&d.tile_off, T + 1));
-  MF_TRY(dalloc(&d.tile_row, T));
-  MF_TRY(dalloc(&d.tile_nz, T));
-  MF_TRY(dalloc(&d.rc, (size_t)ZP + kPad));
-  MF_TRY(dalloc(&d.rp16, (size_t)T * kTile + kPad));
-  MF_TRY(dalloc(&d.v64, (size_t)ZP + kPad));
-  MF_TRY(dalloc(&d.v32, (size_t)ZP + kPad));
-  MF_TRY(dalloc(&d.v16, (size_t)ZP + kPad));
-  MF_TRY(dalloc(&d.v8, (size_t)ZP + kPad));
-  MF_TRY(dalloc(&d.s16, T));
-  MF_TRY(dalloc(&d.s8, T));
-  MF_TRY(dalloc(&d.qerr, 3 * (size_t)T));
-  MF_TRY(dalloc(&d.amax, T));
-  MF_TRY(dalloc(&d.prec, T));
-  MF_TRY(dalloc(&d.prec_user, T));
-  MF_TRY(dalloc(&d.diag_tile, TM));
+  Slab slab;
+  slab.add(&d.tile_ptr, TM + 1);
+  slab.add(&d.tile_col, T);
+  slab.add(&d.tile_off, T + 1);
+  slab.add(&d.tile_row, T);
+  slab.add(&d.tile_nz, T);
+  slab.add(&d.rc, (size_t)ZP + kPad);
+  slab.add(&d.rp16, (size_t)T * kTile + kPad);
+  slab.add(&d.v64, (size_t)ZP + kPad);
+  slab.add(&d.v32, (size_t)ZP + kPad);
+  slab.add(&d.v16, (size_t)ZP + kPad);
+  slab.add(&d.v8, (size_t)ZP + kPad);
+  slab.add(&d.s16, T);
+  slab.add(&d.s8, T);
+  slab.add(&d.qerr, 3 * (size_t)T);
+  slab.add(&d.amax, T);
+  slab.add(&d.prec, T);
+  slab.add(&d.prec_user, T);
+  slab.add(&d.diag_tile, TM);
+  MF_TRY(slab.alloc(&d.slab));
   MF_HIP(hipMemcpy(d.tile_ptr, t->tile_ptr.data(), sizeof(int) * (TM + 1), hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(d.tile_col, t->tile_columnidx.data(), sizeof(int) * T, hipMemcpyHostToDevice));
   MF_HIP(hipMemcpy(d.tile_off, poff.data(), sizeof(int) * (T + 1), hipMemcpyHostToDevice));
-  if (T > 0) MF_HIP(hipMemcpy(d.tile_nz, tnz.data(), T, hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(d.tile_row, tile_row.data(), sizeof(int) * T, hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(d.rc, rc.data(), (size_t)ZP + kPad, hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(d.rp16, rp16.data(), rp16.size(), hipMemcpyHostToDevice));
-  MF_HIP(hipMemset(d.v16, 0, sizeof(uint16_t) * ((size_t)ZP + kPad)));
-  MF_HIP(hipMemset(d.v8, 0, (size_t)ZP + kPad));
-  MF_HIP(hipMemcpy(d.v64, v64.data(), sizeof(double) * ((size_t)ZP + kPad), hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(d.diag_tile, diag.data(), sizeof(int) * TM, hipMemcpyHostToDevice));
+  // the slots past the last tile that a 16-byte load may touch
+  MF_HIP(hipMemset(d.rc + ZP, 0, kPad));
+  MF_HIP(hipMemset(d.v64 + ZP, 0, sizeof(double) * kPad));
+  MF_HIP(hipMemset(d.v32 + ZP, 0, sizeof(float) * kPad));
+  MF_HIP(hipMemset(d.v16 + ZP, 0, sizeof(uint16_t) * kPad));
+  MF_HIP(hipMemset(d.v8 + ZP, 0, kPad));
+  if (TM > 0) MF_HIP(hipMemset(d.diag_tile, 0xff, sizeof(int) * TM));
   // per-wave work of the stand-alone SpMV, about kSpmvWaveNnz entries per
   // wave (retuned by mf_tile_set_schedule)
   MF_TRY(upload_spmv_schedule(t, kSpmvWaveNnz));
-  MF_HIP(hipMemset(d.prec, MF_PREC_FP64, T));
-  MF_HIP(hipMemset(d.prec_user, MF_PREC_FP64, T));
   if (T > 0) {
-    k_pack_payloads<<<(T + 255) / 256, 256>>>(T, d.tile_off, d.v64, d.v32, d.v16, d.v8, d.s16,
-                                              d.s8, d.qerr, d.amax);
-    MF_HIP(hipGetLastError());
+    MF_HIP(hipMemset(d.prec, MF_PREC_FP64, T));
+    MF_HIP(hipMemset(d.prec_user, MF_PREC_FP64, T));
+    MF_HIP(hipMemcpy(d.tile_col, t->tile_columnidx.data(), sizeof(int) * T, hipMemcpyHostToDevice));
+    // the reference arrays, for the packing only
+    double *val = nullptr;
+    float *low = nullptr;
+    uint8_t *col = nullptr, *ptr = nullptr;
+    int *off = nullptr;
+    void *tmp = nullptr;
+    Slab src;
+    src.add(&val, t->csrsize);
+    if (t->low_given) src.add(&low, t->csrsize);
+    src.add(&col, t->csrsize);
+    src.add(&ptr, t->csrptrlen);
+    src.add(&off, T + 1);
+    MF_TRY(src.alloc(&tmp));
+    auto up = [](void *q, const void *h, size_t bytes) { return hipMemcpy(q, h, bytes, hipMemcpyHostToDevice); };
+    hipError_t e = up(val, t->Blockcsr_Val.data(), sizeof(double) * t->csrsize);
+    if (e == hipSuccess && low) e = up(low, t->Blockcsr_Val_Low.data(), sizeof(float) * t->csrsize);
+    if (e == hipSuccess) e = up(col, t->Tile_csr_Col.data(), t->csrsize);
+    if (e == hipSuccess) e = up(ptr, t->Blockcsr_Ptr.data(), t->csrptrlen);
+    if (e == hipSuccess) e = up(off, t->csr_offset.data(), sizeof(int) * (T + 1));
+    if (e == hipSuccess) {
+      k_tile_rows<<<(TM + 15) / 16, 256>>>(TM, d.tile_ptr, d.tile_col, d.tile_row, d.diag_tile);
+      const PackSrc ps{val, low, col, ptr, off, t->tile_ptr[TM - 1], t->rowA - (TM - 1) * kTile};
+      const PackDst pd{d.tile_off, d.tile_nz, d.rc, d.rp16, d.v64, d.v32, d.v16, d.v8, d.s16, d.s8, d.qerr, d.amax};
+      k_pack_tiles<<<(T + 15) / 16, 256>>>(T, ps, pd);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    (void)hipFree(tmp);
+    if (e != hipSuccess) return fail(MF_ERR_HIP, std::string("tile upload: ") + hipGetErrorString(e));
   }
-  // The FP32 payload keeps the caller's FP32 copy when one was given
-  // (the reference passes Val_Low, src/csr2block.h:248).
-  MF_HIP(hipMemcpy(d.v32, v32.data(), sizeof(float) * ((size_t)ZP + kPad), hipMemcpyHostToDevice));
-  MF_HIP(hipDeviceSynchronize());
+  MF_TRY(build_strips(t, rowptr));
+  d.spmv_kernel = default_spmv_kernel(t);
   return MF_OK;
 }
 
@@ -211,11 +266,24 @@ bool regular_tilerows(const mf_tiled *t) {
   return t->dev.max_tiles_per_row <= 4.0 * mean + 8.0;
 }
 
-int default_spmv_kernel(const mf_tiled *) {
-  // The streamed kernel handles any sparsity and was the faster of the two
-  // on the 3D 7-point 128^3 Laplacian on MI355X (mf_tune_spmv also times
-  // the row-group kernel on matrices with regular tile-rows).
-  return MF_SPMV_STREAM;
+int default_spmv_kernel(const mf_tiled *t) {
+  // Both kernels run at the rate of their bytes (strips: an entry's word or
+  // value and column, a lead per row; tiles: value, byte and metadata), so the
+  // fewer bytes win, with a margin for what strips save besides.  Measured on
+  // MI355X, strips / streamed tiles, operands in the caches and not: 128^3
+  // 7-point Laplacian (packed, 67 against 151 MB) 17.5 / 30.2 and 36.7 / 68.9
+  // us; the same pattern with random values (near, 143 MB) 24.9 / 30.1 and
+  // 57.9 / 68.8; 64-entry bands of random values (near, 65 against 58 MB)
+  // 12.3 / 13.2 and 26.3 / 28.6; 150k-row kNN graph, random values (17
+  // against 19 MB) 5.7 / 6.2 and 16.4 / 13.9; 200k-row power-law graph (packed,
+  // pieces; 16 against 135 MB) 25.8 / 149 and 41 / 215.
+  const StripLayout &L = t->strips;
+  if (L.nstrips == 0) return MF_SPMV_STREAM;
+  double strip = 8.0 * 64.0 * L.nstrips;
+  for (const StripDesc &d : L.hdesc)
+    strip += 128.0 * d.npair * (d.cls == kStripPacked ? 4.0 : d.cls == kStripNear ? 10.0 : 12.0);
+  const double tiles = 9.0 * t->dev.npay + 13.0 * t->tilenum;
+  return strip <= 1.2 * tiles ? MF_SPMV_STRIP : MF_SPMV_STREAM;
 }
 
 // Stand-alone SpMV schedule of about wave_nnz payload slots per wave, heavy
@@ -257,15 +325,13 @@ mf_status upload_spmv_schedule(mf_tiled *t, int wave_nnz) {
 void free_device(mf_tiled *t) {
   DeviceLayout &d = t->dev;
   if (d.device >= 0) (void)hipSetDevice(d.device);
-  void *ptrs[] = {d.tile_ptr, d.tile_col, d.tile_off, d.tile_row, d.rc, d.rp16, d.spmv_desc, d.tile_nz,
-                  d.spmv_part, d.spmv_cnt, d.spmv_hn, d.spmv_hbase,
-                  d.v64,      d.v32,      d.v16,      d.v8,       d.s16,    d.s8,
-                  d.qerr,     d.amax,     d.prec,     d.prec_user, d.diag_tile, d.mlp, d.feat16,
+  void *ptrs[] = {d.slab, d.spmv_desc, d.spmv_part, d.spmv_cnt, d.spmv_hn, d.spmv_hbase, d.mlp, d.feat16,
                   t->sched.wave_tr, t->sched.wave_res, t->sched.wave_win, t->sched.win_desc, t->sched.heavy_part,
                   t->sched.heavy_cnt, t->sched.heavy_n, t->sched.heavy_base, t->sched.heavy_tr,
                   t->sched.wave_heavy, t->work};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
+  free_strips(t);
   d = DeviceLayout();
   t->sched = Schedule();
   t->work = nullptr;
@@ -289,7 +355,7 @@ extern "C" mf_status mf_tile_create(int rowA, int colA, const int *rowptr, const
   }
   mf_tiled *t = new mf_tiled();
   mf_status st = build_tiles_host(t, rowA, colA, rowptr, colidx, val, val_low);
-  if (st == MF_OK && device != -1) st = upload_tiles(t, device);
+  if (st == MF_OK && device != -1) st = upload_tiles(t, device, rowptr);
   if (device == -1) t->dev.npad = kTile * std::max(std::max(t->tilem, t->tilen), 1);
   if (st != MF_OK) {
     std::string msg = mf_last_error();
@@ -360,5 +426,7 @@ extern "C" mf_status mf_tile_set_schedule(mf_tiled *t, int spmv_wave_nnz) {
   MF_HIP(hipSetDevice(t->dev.device));
   MF_HIP(hipDeviceSynchronize());
   MF_TRY(upload_spmv_schedule(t, spmv_wave_nnz));
+  // the schedule is the streamed kernel's
+  if (t->dev.spmv_kernel == MF_SPMV_STRIP) t->dev.spmv_kernel = MF_SPMV_STREAM;
   return MF_OK;
 }

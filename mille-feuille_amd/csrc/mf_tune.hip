@@ -4,7 +4,7 @@
 // SpMV: the streamed kernel's entries per wave set the number and length of
 // the per-wave windows (more waves hide more latency, longer waves pay their
 // setup less often); the row-group kernel is a candidate where tile-rows are
-// regular.  Batched CG: the waves per (system, right-hand side) item trade
+// regular, the strip kernel (FP64) where the handle has strips.  Batched CG: the waves per (system, right-hand side) item trade
 // per-item parallelism against the number of items in flight.
 #include <algorithm>
 #include <vector>
@@ -81,6 +81,7 @@ extern "C" mf_status mf_tune_spmv(mf_tiled *t, int mode, mf_tune_report *rep) {
   const int old_nnz = t->dev.spmv_wave_nnz, old_kernel = t->dev.spmv_kernel;
   std::vector<int> cand = {384, 512, 768, 1024, 1536, 2048};
   if (regular_tilerows(t)) cand.push_back(0);
+  if (mode == kAll64 && t->strips.nstrips > 0) cand.push_back(-1);
   *rep = mf_tune_report{};
   rep->ncand = (int)cand.size();
   float best = 0.0f;
@@ -90,13 +91,13 @@ extern "C" mf_status mf_tune_spmv(mf_tiled *t, int mode, mf_tune_report *rep) {
       MF_TRY(mf_tile_set_schedule(t, cand[i]));
       t->dev.spmv_kernel = MF_SPMV_STREAM;
     } else {
-      t->dev.spmv_kernel = MF_SPMV_ROWGROUP;
+      t->dev.spmv_kernel = cand[i] < 0 ? MF_SPMV_STRIP : MF_SPMV_ROWGROUP;
     }
     float us = 0.0f;
     const mf_status st = time_median([&] { return mf_spmv(t, x, x32, y, mode, nullptr); }, 5, 25, &us);
     if (st != MF_OK) {
-      t->dev.spmv_kernel = old_kernel;
       (void)mf_tile_set_schedule(t, old_nnz);
+      t->dev.spmv_kernel = old_kernel;
       return st;
     }
     rep->cand[i] = cand[i];
@@ -109,10 +110,11 @@ extern "C" mf_status mf_tune_spmv(mf_tiled *t, int mode, mf_tune_report *rep) {
   rep->best = cand[bi];
   if (cand[bi] > 0) {
     MF_TRY(mf_tile_set_schedule(t, cand[bi]));
-    t->dev.spmv_kernel = MF_SPMV_STREAM;
+    // (mode 1 of a handle on strips runs the streamed kernel already)
+    t->dev.spmv_kernel = mode == kPerTile && old_kernel == MF_SPMV_STRIP ? MF_SPMV_STRIP : MF_SPMV_STREAM;
   } else {
     MF_TRY(mf_tile_set_schedule(t, old_nnz));
-    t->dev.spmv_kernel = MF_SPMV_ROWGROUP;
+    t->dev.spmv_kernel = cand[bi] < 0 ? MF_SPMV_STRIP : MF_SPMV_ROWGROUP;
   }
   return MF_OK;
 }

@@ -75,7 +75,7 @@ class TiledMatrix:
         vals = [C.c_int() for _ in range(6)]
         check("mf_tile_info", lib.mf_tile_info(h, *[C.byref(v) for v in vals]))
         self.tilem, self.tilen, self.tilenum, self.csrsize, self.csrptrlen, self.npad = [v.value for v in vals]
-        self._spmv_kernel = _lib.SPMV_STREAM
+        self._spmv_kernel = _lib.SPMV_AUTO
 
     def free(self):
         if getattr(self, "h", None):
@@ -168,6 +168,8 @@ class TiledMatrix:
         check("mf_tile_set_schedule", lib.mf_tile_set_schedule(self.h, int(spmv_wave_nnz)))
         if int(spmv_wave_nnz) > 0:
             self._wave_nnz = int(spmv_wave_nnz)
+            if self._spmv_kernel not in (_lib.SPMV_STREAM, _lib.SPMV_ROWGROUP):
+                self._spmv_kernel = _lib.SPMV_STREAM  # as the library does
 
     def tune_spmv(self, mode=0):
         """Autotunes the stand-alone SpMV (mf_tune_spmv) for `mode` at the
@@ -176,18 +178,25 @@ class TiledMatrix:
         rep = _lib.MfTuneReport()
         check("mf_tune_spmv", lib.mf_tune_spmv(self.h, int(mode), C.byref(rep)))
         d = rep.as_dict()
-        self._spmv_kernel = _lib.SPMV_ROWGROUP if d["best"] == 0 else _lib.SPMV_STREAM
+        if d["best"] <= 0:
+            self._spmv_kernel = _lib.SPMV_ROWGROUP if d["best"] == 0 else _lib.SPMV_STRIP
+        elif int(mode) == 0 or self._spmv_kernel == _lib.SPMV_ROWGROUP:
+            self._spmv_kernel = _lib.SPMV_STREAM
         if d["best"] > 0:
             self._wave_nnz = int(d["best"])
         return d
 
     def spmv_kernel_name(self):
         """Device kernel that mf_spmv launches for this handle (mode 0): the
-        row-group kernel, or the streamed one, instantiated with piece
-        bookkeeping when a tile-row holds more than 4*max(wave_nnz, 4096)
-        padded payload slots (the library's heavy tile-row rule)."""
+        row-group kernel, the strip kernel (with pieces when the layout has
+        long rows), or the streamed one, instantiated with piece bookkeeping
+        when a tile-row holds more than 4*max(wave_nnz, 4096) padded payload
+        slots (the library's heavy tile-row rule)."""
         if self._spmv_kernel == _lib.SPMV_ROWGROUP:
             return "mf::k_spmv_rg<0>"
+        d = self.strips()
+        if d["strips"] and self._spmv_kernel != _lib.SPMV_STREAM:
+            return f"mf::k_spmv_strip<{'true' if d['pieces'] else 'false'}>"
         a = self.arrays()
         slots = (np.diff(a["csr_offset"]).astype(np.int64) + 3) // 4 * 4
         pre = np.concatenate([[0], np.cumsum(slots)])
@@ -195,12 +204,21 @@ class TiledMatrix:
         heavy = bool((row_slots > 4 * max(getattr(self, "_wave_nnz", 1024), 4096)).any())
         return f"mf::k_spmv<0, {'true' if heavy else 'false'}>"
 
+    def strips(self):
+        """Sizes of the handle's row-strip layout: strips (0: none), pieces of
+        long rows, whether rows are sorted, and the entry slots
+        stored packed (one 32-bit word each) and in full."""
+        v = [C.c_int(), C.c_int(), C.c_int(), C.c_int64(), C.c_int64()]
+        check("mf_tile_strip_info", lib.mf_tile_strip_info(self.h, *[C.byref(q) for q in v]))
+        return dict(zip(("strips", "pieces", "sorted", "packed_slots", "full_slots"), [q.value for q in v]))
+
     def set_spmv_kernel(self, kind):
-        """'auto', 'stream' or 'rowgroup' (or the MF_SPMV_* value)."""
-        k = {"auto": _lib.SPMV_AUTO, "stream": _lib.SPMV_STREAM, "rowgroup": _lib.SPMV_ROWGROUP}
+        """'auto', 'stream', 'rowgroup' or 'strip' (or the MF_SPMV_* value)."""
+        k = {"auto": _lib.SPMV_AUTO, "stream": _lib.SPMV_STREAM, "rowgroup": _lib.SPMV_ROWGROUP,
+             "strip": _lib.SPMV_STRIP}
         kind = k.get(kind, kind)
         check("mf_tile_set_spmv_kernel", lib.mf_tile_set_spmv_kernel(self.h, kind))
-        self._spmv_kernel = _lib.SPMV_STREAM if kind == _lib.SPMV_AUTO else kind
+        self._spmv_kernel = kind
 
     def get_precision(self):
         out = np.zeros(max(self.tilenum, 1), np.uint8)

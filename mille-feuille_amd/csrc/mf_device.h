@@ -1501,12 +1501,39 @@ __device__ __forceinline__ bool wave_infer(const TileView &A, const InferCtx &ic
   return wave_infer_tiles(A, ic, A.tile_ptr[tr0], A.tile_ptr[tr1], lane);
 }
 
-// Deterministic sum over the 64 lanes of a wave (fixed xor tree); every lane
-// gets the result.
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+// v of the lane that the DPP control names, 0 where there is none or the row
+// is masked off.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_take(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+__device__ __forceinline__ double read_lane(double v, int l) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, l), hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), l);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// Lane 15 of each row of 16 lanes gets the row's sum (row_shr 1, 2, 4, 8).
+__device__ __forceinline__ double row_sum15(double v) {
+  v += dpp_take<0x111, 0xf>(v);
+  v += dpp_take<0x112, 0xf>(v);
+  v += dpp_take<0x114, 0xf>(v);
+  v += dpp_take<0x118, 0xf>(v);
   return v;
+}
+
+// Deterministic sum over the 64 lanes of a wave, the same in every lane: rows
+// of 16 lanes, then row_bcast 15 and 31 (data-parallel moves; the same tree
+// over LDS-crossbar shuffles took about 0.3 us a value).
+__device__ __forceinline__ double wave_sum(double v) {
+  v = row_sum15(v);
+  v += dpp_take<0x142, 0xa>(v);
+  v += dpp_take<0x143, 0xc>(v);
+  return read_lane(v, 63);
 }
 
 // A wave-uniform double moved to scalar registers, so that loop state which
@@ -1518,17 +1545,22 @@ __device__ __forceinline__ double uniform_double(double v) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// Deterministic sum over the block: wave sums, then waves in index order.
-// `lds` must hold blockDim.x/64 doubles.  Every thread gets the result.
+// Sum of the waves' values lds[0 .. nw), nw <= 16, in every lane.
+__device__ __forceinline__ double sum_waves(const double *lds, int nw) {
+  const int l = threadIdx.x & 15;
+  return read_lane(row_sum15(l < nw ? lds[l] : 0.0), 15);
+}
+
+// Deterministic sum over the block (at most 16 waves): wave sums, then a row
+// of lanes over the waves.  `lds` must hold blockDim.x/64 doubles.  Every
+// thread gets the result.
 __device__ __forceinline__ double block_sum(double v, double *lds) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   v = wave_sum(v);
   __syncthreads();
   if (lane == 0) lds[w] = v;
   __syncthreads();
-  double s = 0.0;
-  for (int i = 0; i < nw; ++i) s += lds[i];
-  return uniform_double(s);  // every lane summed the same values in the same order
+  return sum_waves(lds, nw);
 }
 
 // Grid synchronisation for a co-resident grid.
@@ -1537,73 +1569,91 @@ __device__ __forceinline__ double block_sum(double v, double *lds) {
 // blocks).  Publication: every wave first drains its own outstanding memory
 // operations (s_waitcnt vmcnt(0)), the block meets at s_barrier, and thread 0
 // alone issues the agent-scope release (one L2 write-back per block) and
-// stores the epoch in the block's own arrival word.  Block 0 watches all
-// arrival words (one lane per block), then publishes the epoch in `flag`;
-// every other block's thread 0 polls that one word and issues the single
-// agent-scope acquire (L1/L2 invalidate) for its block before the block
-// barrier releases the other waves.  Measured on MI355X with one 1024-thread
-// block per CU: about 5 us per sync, against 30-120 us when every wave
-// fences and 4-7 us more when all blocks hit one atomic counter.
+// stores the epoch in the block's own arrival word.  Every block's first wave
+// then watches all arrival words (one 256-byte load per 64 blocks) and issues
+// the single agent-scope acquire (L1/L2 invalidate) for its block before the
+// block barrier releases the other waves: one trip through memory.  (Block 0
+// watching the words and publishing a flag that the others poll took 4.2-4.8
+// us a sync on the full grid of an MI355X, two trips.)
 //
 // Every wait is bounded: after kSpinLimit polls a waiter raises `abort` and
 // returns, so a block that is not resident (or any lost arrival) ends the
 // kernel with an error the host reports, never a hang.
-constexpr int kMaxBlocks = 4096;
+constexpr int kMaxBlocks = 512;
+
+// From kCopyBlocks blocks on, what a block posts goes to 8 copies, and block b
+// watches copy b % 8 (its XCD's): all blocks watching one copy keep the few
+// memory channels that hold it busy, and the posts wait behind the polls.
+// Measured on MI355X, 256 blocks of the 64^3 CG (from a block's arrival to its
+// release): one copy 5.0 us a sum and 4.1 a barrier, 8 copies 3.7 and 2.4.
+constexpr int kCopies = 8;
+constexpr int kCopyBlocks = 64;
+
+__device__ __forceinline__ int sync_copies() { return (int)gridDim.x >= kCopyBlocks ? kCopies : 1; }
+__device__ __forceinline__ int sync_copy() { return (int)gridDim.x >= kCopyBlocks ? (int)(blockIdx.x & 7) : 0; }
 
 struct GridSync {
-  unsigned flag;
-  unsigned pad0[63];
   unsigned abort;
-  unsigned pad1[63];
-  unsigned arrive[kMaxBlocks];
+  unsigned pad[127];  // the polled words start on a line of their own
+  unsigned arrive[kCopies][kMaxBlocks];
 };
 
 constexpr unsigned kSpinLimit = 1u << 22;
 
-__device__ __forceinline__ bool wait_word(unsigned *w, GridSync *gs, unsigned epoch) {
-  unsigned n = 0;
-  while (__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
-    if (++n > kSpinLimit) {
-      __hip_atomic_store(&gs->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return false;
-    }
-    if ((n & 1023u) == 0 &&
-        __hip_atomic_load(&gs->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      return false;
-    __builtin_amdgcn_s_sleep(1);
+// One more poll of a bounded wait; false when the wait is over (limit, or
+// another waiter's abort).
+__device__ __forceinline__ bool spin_on(unsigned &n, GridSync *gs) {
+  if (++n > kSpinLimit) {
+    __hip_atomic_store(&gs->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
   }
+  if ((n & 1023u) == 0 && __hip_atomic_load(&gs->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    return false;
+  __builtin_amdgcn_s_sleep(1);
   return true;
+}
+
+// A wave waits until words [0, n) have all reached the epoch.
+__device__ __forceinline__ void wait_words(const unsigned *w, int n, GridSync *gs, unsigned epoch) {
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < n; base += 256) {
+    unsigned spins = 0;
+    for (;;) {
+      bool ok = true;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = base + 64 * u + lane;
+        const unsigned v = i < n ? __hip_atomic_load(w + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : epoch;
+        ok = ok && v >= epoch;
+      }
+      if (__ballot(!ok) == 0) break;
+      if (!spin_on(spins, gs)) return;
+    }
+  }
 }
 
 __device__ __forceinline__ void drain_own_memory_ops() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// Arrival + master wait + release of the flag.  On return the whole grid has
-// passed the sync point and this block has acquired.  `master_work` runs in
-// block 0 after every arrival has been seen and before the flag is
-// published (used by grid_sum to add the partials).
-template <typename F>
-__device__ __forceinline__ void grid_arrive_wait(GridSync *gs, unsigned &epoch, F master_work) {
+// Arrival of the block at a sync point, and the wait for all others.  Work
+// that touches no memory another block reads or writes may go between.
+// RELEASE = false: every store since the last sync point that another block
+// reads was an agent-scope one, already at the coherent level once drained.
+template <bool RELEASE = true>
+__device__ __forceinline__ void grid_arrive(GridSync *gs, unsigned &epoch) {
   drain_own_memory_ops();
   __syncthreads();
   ++epoch;
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __hip_atomic_store(&gs->arrive[blockIdx.x], epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((int)threadIdx.x < sync_copies()) {
+    if (RELEASE) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __hip_atomic_store(&gs->arrive[threadIdx.x][blockIdx.x], epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (blockIdx.x == 0) {
-    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x)
-      if (!wait_word(&gs->arrive[b], gs, epoch)) break;
-    if (threadIdx.x < (int)gridDim.x) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __syncthreads();
-    master_work();
-    drain_own_memory_ops();
-    __syncthreads();
-    if (threadIdx.x == 0)
-      __hip_atomic_store(&gs->flag, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-  } else if (threadIdx.x == 0) {
-    wait_word(&gs->flag, gs, epoch);
+}
+
+__device__ __forceinline__ void grid_wait(GridSync *gs, unsigned epoch) {
+  if (threadIdx.x < 64) {
+    wait_words(gs->arrive[sync_copy()], gridDim.x, gs, epoch);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
@@ -1612,12 +1662,11 @@ __device__ __forceinline__ void grid_arrive_wait(GridSync *gs, unsigned &epoch, 
 // Plain grid barrier.
 __device__ __forceinline__ void grid_sync(GridSync *gs, unsigned &epoch, int *lds_i) {
   (void)lds_i;
-  grid_arrive_wait(gs, epoch, [] {});
+  grid_arrive(gs, epoch);
+  grid_wait(gs, epoch);
 }
 
-// Sum over the block of NV values per thread: fixed-order wave trees, then
-// the waves' sums in wave order.  `lds` must hold NV * blockDim.x/64
-// doubles.  Every thread gets the NV totals.
+// block_sum of NV values.  `lds` must hold NV * blockDim.x/64 doubles.
 template <int NV>
 __device__ __forceinline__ void block_sum_n(double (&v)[NV], double *lds) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -1630,38 +1679,13 @@ __device__ __forceinline__ void block_sum_n(double (&v)[NV], double *lds) {
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    double s = 0.0;
-    for (int k = 0; k < nw; ++k) s += lds[i * nw + k];
-    v[i] = uniform_double(s);  // every lane summed the same values in the same order
-  }
+  for (int i = 0; i < NV; ++i) v[i] = sum_waves(lds + i * nw, nw);
 }
 
 // Barrier of the block's waves for LDS traffic only: it waits for the
 // wave's own LDS operations, not for its outstanding global stores (which a
 // full __syncthreads would drain).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// block_sum_n with LDS-only barriers (callers whose global stores need no
-// ordering against the sum).
-template <int NV>
-__device__ __forceinline__ void block_sum_lds(double (&v)[NV], double *lds) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) v[i] = wave_sum(v[i]);
-  lds_barrier();
-  if (lane == 0) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) lds[i * nw + w] = v[i];
-  }
-  lds_barrier();
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    double s = 0.0;
-    for (int k = 0; k < nw; ++k) s += lds[i * nw + k];
-    v[i] = uniform_double(s);
-  }
-}
 
 // Grid-wide deterministic sum of NV values per thread, also a full barrier.
 // Each block writes its NV block sums to partials[slot][block][i] and
@@ -1686,7 +1710,8 @@ __device__ __forceinline__ void grid_sum(double (&v)[NV], double *partials, Grid
 #pragma unroll
     for (int i = 0; i < NV; ++i) buf[blockIdx.x * NV + i] = v[i];
   }
-  grid_arrive_wait(gs, epoch, [] {});
+  grid_arrive(gs, epoch);
+  grid_wait(gs, epoch);
   double s[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) s[i] = 0.0;
@@ -1704,21 +1729,25 @@ __device__ __forceinline__ void grid_sum(double (&v)[NV], double *partials, Grid
 }
 
 // ---------------------------------------------------------------------------
-// Value-only grid sum with epoch-tagged mailboxes.
+// Value-only grid sum with epoch-tagged words.
 //
-// Every 64-bit mailbox word carries the sync point's epoch in its high half
-// and 32 bits of a value in its low half (64-bit agent-scope atomic stores
-// and loads), so a reader that sees the epoch in every word of a mailbox
-// holds the whole value, with no memory fence, no drain of other stores and
-// no second round trip.  Each block posts its NV block sums in its mailbox;
-// block 0 reads every mailbox and adds them in block order with a fixed
-// tree, and posts the totals in the result mailbox, which every other
-// block's thread 0 polls.  This orders no other memory: it is used where the
-// next phase reads only the calling wave's own rows (the rows its SpMV
-// epilogue wrote), and a full barrier (grid_sync, grid_sum) precedes every
-// phase that reads other waves' data.  Waits are bounded as in wait_word.
+// Every 64-bit word carries the sync point's epoch in its high half and 32
+// bits of a value in its low half (64-bit agent-scope atomic stores and
+// loads), so a reader that sees the epoch in every word of a value holds the
+// whole value, with no memory fence, no drain of other stores and no second
+// round trip.  Each block posts its NV block sums; every block's first wave
+// reads all blocks' words and adds them in a fixed order, so every block gets
+// the same totals after one trip through memory.  The words of one kind lie
+// together (word k of block b at k * blocks + b of a set) and successive epochs take
+// turns in two sets, so a block that has gone on to the next sum never
+// overwrites what a slower one still reads.  This orders no other memory: it
+// is used where the next phase reads only the calling wave's own rows (the
+// rows its SpMV epilogue wrote), and a full barrier (grid_sync, grid_sum)
+// precedes every phase that reads other waves' data.  Waits are bounded.
+// Measured on MI355X: 1.9 us on 4 blocks, 3.7 us on 256 (block 0 adding all
+// sums and posting the totals, with serial sums over the waves: 5.1 and 6.3).
 // ---------------------------------------------------------------------------
-constexpr int kMboxWords = 2 * kMaxGridSum;  // one 64-byte line per block
+constexpr int kMboxWords = kCopies * 8;  // per block and copy: two sets of two values
 
 template <int NV>
 __device__ __forceinline__ void mbox_post(unsigned long long *mb, unsigned epoch, const double (&v)[NV]) {
@@ -1744,13 +1773,7 @@ __device__ __forceinline__ bool mbox_take(const unsigned long long *mb, unsigned
       ok = ok && (unsigned)(w[k] >> 32) == epoch;
     }
     if (ok) break;
-    if (++n > kSpinLimit) {
-      __hip_atomic_store(&gs->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return false;
-    }
-    if ((n & 1023u) == 0 && __hip_atomic_load(&gs->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      return false;
-    __builtin_amdgcn_s_sleep(1);
+    if (!spin_on(n, gs)) return false;
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i)
@@ -1758,45 +1781,75 @@ __device__ __forceinline__ bool mbox_take(const unsigned long long *mb, unsigned
   return true;
 }
 
-// mbox: (gridDim.x + 1) * kMboxWords words, zero before the launch.
+// mbox: gridDim.x * kMboxWords words, zero before the launch.  lds: NV *
+// 16 doubles.  Blocks of at most 16 waves.
 template <int NV>
 __device__ __forceinline__ void grid_sum_values(double (&v)[NV], unsigned long long *mbox, GridSync *gs,
                                                 unsigned &epoch, double *lds) {
-  static_assert(NV <= kMaxGridSum, "grid_sum_values width");
-  __shared__ double bcast[kMaxGridSum];
-  const int G = gridDim.x;
-  block_sum_lds<NV>(v, lds);
+  static_assert(NV <= 2, "grid_sum_values width");
+  __shared__ double bcast[2];
+  const int G = gridDim.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) v[i] = wave_sum(v[i]);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) lds[16 * i + w] = v[i];
+  }
   ++epoch;
-  if (threadIdx.x == 0) mbox_post<NV>(mbox + (size_t)blockIdx.x * kMboxWords, epoch, v);
-  unsigned long long *res = mbox + (size_t)G * kMboxWords;
-  if (blockIdx.x == 0) {
+  lds_barrier();
+  if (w == 0) {
+    auto set_of = [&](int c) { return mbox + (size_t)(2 * c + (int)(epoch & 1u)) * 4 * G; };
+    const unsigned long long *set = set_of(sync_copy());
+    double t[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      t[i] = sum_waves(lds + 16 * i, nw);
+    if (lane < 2 * NV * sync_copies()) {
+      // lane 2 NV c + k posts half k & 1 of value k / 2 to copy c
+      const int c = lane / (2 * NV), k = lane % (2 * NV);
+      const uint64_t b = __builtin_bit_cast(uint64_t, NV > 1 && k >= 2 ? t[NV - 1] : t[0]);
+      __hip_atomic_store(set_of(c) + (size_t)k * G + blockIdx.x,
+                         (unsigned long long)epoch << 32 | (k & 1 ? b >> 32 : b & 0xffffffffull), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
     double s[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) s[i] = 0.0;
-    for (int b = threadIdx.x; b < G; b += blockDim.x) {
-      double t[NV];
-      if (!mbox_take<NV>(mbox + (size_t)b * kMboxWords, epoch, gs, t)) break;
+    for (int base = 0; base < G; base += 256) {
+      unsigned spins = 0;
+      unsigned long long q[4][2 * NV];
+      for (;;) {
+        bool ok = true;
 #pragma unroll
-      for (int i = 0; i < NV; ++i) s[i] += t[i];
+        for (int u = 0; u < 4; ++u) {
+          const int b = base + 64 * u + lane;
+#pragma unroll
+          for (int k = 0; k < 2 * NV; ++k)
+            q[u][k] = b < G ? __hip_atomic_load(set + (size_t)k * G + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                            : (unsigned long long)epoch << 32;
+#pragma unroll
+          for (int k = 0; k < 2 * NV; ++k) ok = ok && (unsigned)(q[u][k] >> 32) == epoch;
+        }
+        if (__ballot(!ok) == 0 || !spin_on(spins, gs)) break;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          s[i] += __builtin_bit_cast(double, (q[u][2 * i + 1] & 0xffffffffull) << 32 | (q[u][2 * i] & 0xffffffffull));
     }
-    block_sum_lds<NV>(s, lds);
-    if (threadIdx.x == 0) mbox_post<NV>(res, epoch, s);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] = s[i];
-  } else {
-    if (threadIdx.x == 0) {
-      double t[NV];
+    for (int i = 0; i < NV; ++i) s[i] = wave_sum(s[i]);
+    if (lane == 0) {
 #pragma unroll
-      for (int i = 0; i < NV; ++i) t[i] = 0.0;
-      mbox_take<NV>(res, epoch, gs, t);
-#pragma unroll
-      for (int i = 0; i < NV; ++i) bcast[i] = t[i];
+      for (int i = 0; i < NV; ++i) bcast[i] = s[i];
     }
-    lds_barrier();
-#pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] = uniform_double(bcast[i]);
   }
-  lds_barrier();  // bcast and lds are free again
+  // (the next sum's first barrier separates its write of bcast from these
+  // reads, and this one its writes of lds from the first wave's reads)
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) v[i] = uniform_double(bcast[i]);
 }
 
 }  // namespace mf

@@ -145,6 +145,7 @@ struct StripLayout {
   int nlong = 0;     // rows with pieces, those longer than a piece first
   int nmulti = 0;    // rows longer than a piece
   int sorted = 0;    // rows sorted by length inside windows of strips
+  bool lean = false; // a product over strips reads fewer bytes than over tiles (lean_strips)
   StripDesc *desc = nullptr;
   uint32_t *words = nullptr;
   double *vv = nullptr;
@@ -186,6 +187,17 @@ struct Schedule {
   int *wave_heavy = nullptr;      // device, nwaves+1: heavy tile-rows each wave owns
 };
 
+// Schedule of the strip solvers for one wave count: equal contiguous runs of
+// strips, and the pieces of long rows dealt to the waves with the least work.
+struct StripSchedule {
+  int nwaves = 0;
+  std::vector<int> wave_tr;      // tile-rows of each wave's strips, nwaves + 1
+  std::vector<int> wave_piece;   // bounds of each wave's pieces, nwaves + 1
+  std::vector<int> piece_order;  // npieces
+  int *d_wave_tr = nullptr, *d_wave_piece = nullptr, *d_piece_order = nullptr;
+  void *slab = nullptr;
+};
+
 }  // namespace mf
 
 struct mf_tiled {
@@ -203,6 +215,7 @@ struct mf_tiled {
   mf::DeviceLayout dev;
   mf::StripLayout strips;
   mf::Schedule sched;
+  mf::StripSchedule strip_sched;
   int sched_waves_for = 0;  // wave count the cached schedule was built for
   // device scratch owned by the handle (solver workspace), grown on demand
   void *work = nullptr;
@@ -221,6 +234,8 @@ mf_status upload_tiles(mf_tiled *t, int device, const int *rowptr);
 mf_status build_strips(mf_tiled *t, const int *rowptr);
 void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info, StripPlan &p);
 void free_strips(mf_tiled *t);
+bool lean_strips(const mf_tiled *t);
+void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s);
 void free_device(mf_tiled *t);
 // nnz-balanced contiguous tile-row partition for `nwaves` waves.
 std::vector<int> balance_tilerows(const mf_tiled *t, int nwaves);

@@ -264,14 +264,23 @@ __global__ void k_seg_norm2(const double *__restrict__ v, int n, int nseg, float
   seg2d[c] = s;
 }
 
-// Deterministic single-block sum.
+// Deterministic single-block sum: an exchange tree in each wave, then the
+// waves in order.  The FP16 features are rounded from this sum, so its order
+// of additions stays what it was (block_sum adds in another).
 __global__ __launch_bounds__(1024) void k_sum_one_block(const double *__restrict__ v, int n,
                                                         double *__restrict__ out) {
   __shared__ double lds[16];
   double s = 0.0;
   for (int i = threadIdx.x; i < n; i += 1024) s += v[i];
-  s = block_sum(s, lds);
-  if (threadIdx.x == 0) *out = s;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double sum = 0.0;
+    for (int w = 0; w < 16; ++w) sum += lds[w];
+    *out = sum;
+  }
 }
 
 __global__ void k_features(int T, const uint16_t *__restrict__ feat16,

@@ -29,27 +29,14 @@
 #include <vector>
 #include <type_traits>
 
-#include "mf_device.h"
+#include "mf_strip_solve.h"
 
 namespace mf {
 
 // Packed MLP of a handle (mf_learned.hip), or null when none is installed.
 const MlpDevice *policy_mlp(const mf_tiled *t);
 
-constexpr int kBlock = 1024;  // 16 waves, one block per CU
-constexpr int kWavesPerBlock = kBlock / 64;
 constexpr int kUpd = 4;  // 64-row groups per step of the vector loops (loads first)
-
-enum StatSlot {
-  kStIters = 0,
-  kStRefresh,
-  kStFallback,
-  kStRecursive,
-  kStTrue,
-  kStBB,
-  kStStatus,
-  kStCount = 16
-};
 
 // Wave index of the calling wave in the solver's tile-row order.  Blocks are
 // dispatched round-robin over the 8 XCDs (block b on XCD b % 8); with a grid
@@ -1106,7 +1093,7 @@ constexpr size_t kVecSkew = 4096 + 256;
 mf_status get_workspace(mf_tiled *t, int G, Workspace &w) {
   const size_t n = t->dev.npad, segs = t->tilen > t->tilem ? t->tilen : t->tilem;
   size_t need = 6 * align256(n * 8) + 6 * align256(n * 4) + 12 * kVecSkew + 2 * align256(segs) + align256(segs * 4) +
-                align256(2 * kMaxGridSum * (size_t)G * 8) + align256(((size_t)G + 1) * kMboxWords * 8) +
+                align256(2 * kMaxGridSum * (size_t)G * 8) + align256((size_t)G * kMboxWords * 8) +
                 align256(sizeof(GridSync)) + align256(kStCount * 8) +
                 align256(5 * 8);
   if (t->work_bytes < need) {
@@ -1135,7 +1122,7 @@ mf_status get_workspace(mf_tiled *t, int G, Workspace &w) {
   w.seg_s = (uint8_t *)take(segs);
   w.seg2 = (float *)take(segs * 4);
   w.partials = (double *)take(2 * kMaxGridSum * (size_t)G * 8);
-  w.mbox = (unsigned long long *)take(((size_t)G + 1) * kMboxWords * 8);
+  w.mbox = (unsigned long long *)take((size_t)G * kMboxWords * 8);
   w.gs = (GridSync *)take(sizeof(GridSync));
   w.stats = (double *)take(kStCount * 8);
   w.hist = (unsigned long long *)take(5 * 8);
@@ -1395,7 +1382,7 @@ mf_status fill_u32(void *p, size_t bytes, uint32_t v, hipStream_t st) {
 // Carves the workspace and the schedule of a solve out of the scratch array;
 // fails when they do not fit.  Host schedule arrays are copied in.
 mf_status scratch_layout(const mf_tiled *t, int G, const HostSchedule &hs, unsigned char *base,
-                         Workspace &w, Schedule &sc, hipStream_t st) {
+                         Workspace &w, Schedule &sc, hipStream_t st, unsigned char **spare, size_t *spare_bytes) {
   const size_t n = t->dev.npad, segs = t->tilen > t->tilem ? t->tilen : t->tilem;
   const int nwaves = (int)hs.b.size() - 1, nh = (int)hs.hn.size();
   size_t off = 0;
@@ -1403,7 +1390,6 @@ mf_status scratch_layout(const mf_tiled *t, int G, const HostSchedule &hs, unsig
   const size_t o_vec = take(6 * align256(n * 8) + 4 * align256(n * 4));
   const size_t o_segp = take(segs), o_segs = take(segs), o_seg2 = take(segs * 4);
   const size_t o_part = take(2 * kMaxGridSum * (size_t)G * 8);
-  const size_t o_mbox = take(((size_t)G + 1) * kMboxWords * 8);
   const size_t o_gs = take(sizeof(GridSync)), o_stats = take(kStCount * 8), o_hist = take(5 * 8);
   const size_t o_tr = take(sizeof(int) * (nwaves + 1)), o_res = take(sizeof(int) * nwaves);
   const size_t o_win = take(sizeof(int) * (nwaves + 1)), o_desc = take(sizeof(WaveDesc) * hs.wd.size());
@@ -1411,10 +1397,20 @@ mf_status scratch_layout(const mf_tiled *t, int G, const HostSchedule &hs, unsig
   const size_t o_hcnt = take(sizeof(unsigned) * std::max(nh, 1)), o_hn = take(sizeof(int) * std::max(nh, 1));
   const size_t o_hbase = take(sizeof(int) * std::max(nh, 1));
   const size_t o_htr = take(sizeof(int) * std::max(nh, 1)), o_wh = take(sizeof(int) * (nwaves + 1));
+  take(((size_t)G + 1) * 64);  // (part of the limit that callers rely on)
   if (off > kScratchBytes)
     return fail(MF_ERR_ARG, "mf_cg_solve_noalloc: the system needs " + std::to_string(off) +
                                 " bytes of workspace, more than the " + std::to_string(kScratchBytes) +
                                 " bytes of the allocation-free scratch (about 150,000 rows)");
+  // The mailboxes of the value sums: behind the rest, or (large systems) in
+  // the place of a vector that only BiCGSTAB uses.
+  const size_t mbox_bytes = (size_t)G * kMboxWords * 8;
+  const size_t o_mbox = off + mbox_bytes <= kScratchBytes ? off : o_vec + 5 * align256(n * 8);
+  if (o_mbox != off && mbox_bytes > n * 8)
+    return fail(MF_ERR_ARG, "mf_cg_solve_noalloc: no room for the grid sums' mailboxes");
+  if (o_mbox == off) take(mbox_bytes);
+  *spare = base + off;
+  *spare_bytes = off < kScratchBytes ? kScratchBytes - off : 0;
   unsigned char *v = base + o_vec;
   w.r = (double *)v; v += align256(n * 8);
   w.p = (double *)v; v += align256(n * 8);
@@ -1461,9 +1457,236 @@ mf_status scratch_layout(const mf_tiled *t, int G, const HostSchedule &hs, unsig
   // the scratch keeps the last call's contents: clear what starts at zero
   MF_TRY(fill_u32(base + o_vec, o_segp - o_vec, 0u, st));  // vectors (zero padding)
   MF_TRY(fill_u32(base + o_segp, o_part - o_segp, 0u, st));  // segment levels (FP64 = 0), norms
-  MF_TRY(fill_u32(base + o_mbox, o_tr - o_mbox, 0u, st));  // mailboxes, barrier, stats, histogram
+  MF_TRY(fill_u32(base + o_mbox, mbox_bytes, 0u, st));
+  MF_TRY(fill_u32(base + o_gs, o_tr - o_gs, 0u, st));  // barrier, stats, histogram
   MF_TRY(fill_u32(base + o_hcnt, align256(sizeof(unsigned) * std::max(nh, 1)), 0u, st));
   return MF_OK;
+}
+
+// The strip solver's schedule of the handle for a wave count (cached).
+static mf_status ensure_strip_schedule(mf_tiled *t, int nwaves) {
+  StripSchedule &s = t->strip_sched;
+  if (s.slab && s.nwaves == nwaves) return MF_OK;
+  if (s.slab) MF_HIP(hipFree(s.slab));
+  s = StripSchedule();
+  plan_strip_schedule(t, nwaves, s);
+  Slab slab;
+  slab.add(&s.d_wave_tr, nwaves + 1);
+  slab.add(&s.d_wave_piece, nwaves + 1);
+  slab.add(&s.d_piece_order, s.piece_order.size());
+  MF_TRY(slab.alloc(&s.slab));
+  MF_HIP(hipMemcpy(s.d_wave_tr, s.wave_tr.data(), sizeof(int) * (nwaves + 1), hipMemcpyHostToDevice));
+  MF_HIP(hipMemcpy(s.d_wave_piece, s.wave_piece.data(), sizeof(int) * (nwaves + 1), hipMemcpyHostToDevice));
+  if (!s.piece_order.empty())
+    MF_HIP(hipMemcpy(s.d_piece_order, s.piece_order.data(), sizeof(int) * s.piece_order.size(),
+                     hipMemcpyHostToDevice));
+  return MF_OK;
+}
+
+// Blocks of a persistent solve without an override: a small system gets about
+// 1024 rows per block (at least 4 blocks; whole multiples of 8 from 8 on, for
+// the XCD-contiguous block order), so the grid-wide sums and syncs span fewer
+// blocks (one strip per wave).  From about 256k rows on, the full grid.
+static int want_blocks(const mf_tiled *t, const mf_solve_opts &opt) {
+  if (opt.blocks > 0) return opt.blocks;
+  const int rows = t->tilem * 16;
+  const int want = std::max(4, (rows + 1023) / 1024);
+  return want >= 8 ? (want + 7) / 8 * 8 : want;
+}
+
+static hipError_t launch_grid(const void *kern, int G, void **args, hipStream_t st) {
+  // The grid never exceeds what the occupancy query says is resident at once.
+  // A cooperative launch also guarantees it; when the runtime refuses one
+  // (e.g. another process holds the device's cooperative queue) the same grid
+  // is launched normally: the barrier needs only atomics, and its bounded
+  // spin turns a block that is not resident into a reported abort.
+  hipError_t le = hipLaunchCooperativeKernel(kern, dim3(G), dim3(kBlock), args, 0, st);
+  if (le == hipErrorIllegalState || le == hipErrorNotSupported) {
+    (void)hipGetLastError();
+    le = hipLaunchKernel(kern, dim3(G), dim3(kBlock), args, 0, st);
+  }
+  return le;
+}
+
+// Grid of a strip solve, or 0 where the tile solver runs: the memory form and
+// per-tile or per-segment levels (FIXED, RULE) need tiles; a handle whose
+// strips read more bytes than its tiles keeps them; rows sorted across
+// tile-rows cannot be inferred per wave (LEARNED); and a wave holds the
+// vectors of at most kMaxWaveStrips strips (2.1M rows on 256 CUs: three FP64
+// vectors of 8 strips are 48 of a lane's 128 registers).  Both sides are
+// measured at k_cg_strip.
+static mf_status strip_grid(const mf_tiled *t, const mf_solve_opts &opt, bool bicg, int *G) {
+  *G = 0;
+  const StripLayout &L = t->strips;
+  const int pol = opt.policy;
+  if (bicg || !L.lean || opt.form == MF_FORM_MEMORY || 2 * L.npieces > t->rowA) return MF_OK;
+  if (pol != MF_POLICY_FP64 && pol != MF_POLICY_ERRBOUND && !(pol == MF_POLICY_LEARNED && !L.sorted)) return MF_OK;
+  int g = 0;
+  MF_TRY(grid_for(strip_cg_kernel(kMaxWaveStrips, pol != MF_POLICY_FP64), want_blocks(t, opt), &g, kBlock, true));
+  const int per = (L.nstrips + g * kWavesPerBlock - 1) / (g * kWavesPerBlock);
+  if (per <= kMaxWaveStrips) *G = g;
+  return MF_OK;
+}
+
+static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solve_opts opt, mf_report *rep,
+                            int G, bool noalloc) {
+  hipStream_t st = (hipStream_t)opt.stream;
+  const StripLayout &L = t->strips;
+  const int nwaves = G * kWavesPerBlock, per = (L.nstrips + nwaves - 1) / nwaves;
+  const size_t n = t->dev.npad, rows = 16 * (size_t)t->tilem;
+  const size_t segs = std::max(t->tilen, t->tilem);
+  Workspace w;
+  StripSchedule nsched;
+  const StripSchedule *sc = &t->strip_sched;
+  unsigned char *spare = nullptr;
+  size_t spare_bytes = 0;
+  if (noalloc) {
+    // the tile solver's layout, so that the same systems fit
+    HostSchedule hs;
+    build_schedule(t, nwaves, hs);
+    Schedule unused;
+    unsigned char *base = nullptr;
+    MF_TRY(scratch_address(t->dev.device, &base));
+    MF_TRY(scratch_layout(t, G, hs, base, w, unused, st, &spare, &spare_bytes));
+    plan_strip_schedule(t, nwaves, nsched);
+    sc = &nsched;
+  } else {
+    MF_TRY(ensure_strip_schedule(t, nwaves));
+    MF_TRY(get_workspace(t, G, w));
+  }
+  // Piece sums and the allocation-free schedule: behind the scratch layout
+  // where they fit, else in the place of vectors that only the tile solvers
+  // use (q .. s: 24 bytes a row, of at least 100,000 rows then).
+  const size_t mail_bytes = sizeof(unsigned long long) * 2 * (size_t)L.npieces;
+  const size_t need = align256(mail_bytes) + 2 * align256(sizeof(int) * (nwaves + 1)) +
+                      align256(sizeof(int) * (size_t)std::max(L.npieces, 1));
+  unsigned char *c = (unsigned char *)w.q;
+  if (noalloc && need <= spare_bytes) c = spare;
+  else if ((noalloc ? need : mail_bytes) > 24 * n)
+    return fail(MF_ERR_ARG, "solve: no room for the long rows' piece sums");
+  auto take = [&](size_t bytes) { unsigned char *p = c; c += align256(bytes); return p; };
+  unsigned long long *pmail = (unsigned long long *)take(mail_bytes);
+  if (noalloc) {
+    nsched.d_wave_tr = (int *)take(sizeof(int) * (nwaves + 1));
+    nsched.d_wave_piece = (int *)take(sizeof(int) * (nwaves + 1));
+    nsched.d_piece_order = (int *)take(sizeof(int) * std::max<size_t>(nsched.piece_order.size(), 1));
+    MF_HIP(hipMemcpyAsync(nsched.d_wave_tr, nsched.wave_tr.data(), sizeof(int) * (nwaves + 1), hipMemcpyHostToDevice, st));
+    MF_HIP(hipMemcpyAsync(nsched.d_wave_piece, nsched.wave_piece.data(), sizeof(int) * (nwaves + 1), hipMemcpyHostToDevice, st));
+    if (!nsched.piece_order.empty())
+      MF_HIP(hipMemcpyAsync(nsched.d_piece_order, nsched.piece_order.data(), sizeof(int) * nsched.piece_order.size(), hipMemcpyHostToDevice, st));
+  }
+  if (opt.policy == MF_POLICY_ERRBOUND && t->tilenum > 0) {
+    MF_TRY(apply_errbound_levels(t, st));
+    MF_TRY(wave_uniform_levels(t, sc->d_wave_tr, nwaves, st));
+  }
+  // Entries of the gathered vectors past the rows (columns beyond them).
+  if (n > rows) {
+    MF_TRY(fill_u32(w.r + rows, (n - rows) * 8, 0u, st));
+    MF_TRY(fill_u32(w.p + rows, (n - rows) * 8, 0u, st));
+    MF_TRY(fill_u32(w.r32 + rows, (n - rows) * 4, 0u, st));
+  }
+  StripSolveArgs a;
+  a.S = strip_view_of(t);
+  a.A = view_of(t);
+  a.b = d_b;
+  a.x = d_x;
+  a.r = w.r;
+  a.p = w.p;
+  a.r32 = w.r32;
+  a.wave_piece = sc->d_wave_piece;
+  a.piece_order = sc->d_piece_order;
+  a.pmail = pmail;
+  a.partials = w.partials;
+  a.mbox = w.mbox;
+  a.gs = w.gs;
+  a.stats = w.stats;
+  a.hist = w.hist;
+  a.tol2 = opt.tol * opt.tol;
+  a.ratio2 = opt.refresh_ratio * opt.refresh_ratio;
+  a.maxiter = opt.maxiter;
+  a.fixed_iters = opt.fixed_iters;
+  a.check_interval = opt.check_interval;
+  a.max_refresh = opt.max_refresh;
+  a.refresh_every = opt.refresh_every;
+  a.mlp = opt.policy == MF_POLICY_LEARNED ? policy_mlp(t) : nullptr;
+  a.feat16 = t->dev.feat16;
+  a.seg2 = w.seg2;
+  a.prec_rw = t->dev.prec;
+  a.nseg = (int)segs;
+  if (a.mlp) MF_TRY(fill_u32(w.seg2, segs * 4, 0u, st));
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (!noalloc) {
+    MF_HIP(hipEventCreate(&e0));
+    MF_HIP(hipEventCreate(&e1));
+    MF_HIP(hipEventRecord(e0, st));
+  }
+  // barrier words, statistics and histogram are contiguous
+  char *z0 = (char *)w.gs, *z1 = (char *)(w.hist + 5);
+  mf_report r;
+  std::memset(&r, 0, sizeof(r));
+  double stats[kStCount];
+  mf_status ret = MF_OK;
+  bool mixed = opt.policy != MF_POLICY_FP64;
+  for (;;) {
+    if (ret == MF_OK) ret = fill_u32(z0, (size_t)(z1 - z0), 0u, st);
+    if (ret == MF_OK) ret = fill_u32(w.mbox, (size_t)G * kMboxWords * 8, 0u, st);
+    if (ret == MF_OK && mail_bytes) ret = fill_u32(pmail, mail_bytes, 0u, st);
+    void *args[] = {&a};
+    hipError_t e = ret == MF_OK ? launch_grid(strip_cg_kernel(per, mixed), G, args, st) : hipSuccess;
+    if (e != hipSuccess) ret = fail(MF_ERR_COOP, std::string("hipLaunchCooperativeKernel: ") + hipGetErrorString(e));
+    struct Back {
+      GridSync gs;
+      double stats[kStCount];
+      unsigned long long hist[5];
+    } back;
+    static_assert(sizeof(GridSync) % 256 == 0 && sizeof(double) * kStCount <= 256, "report layout");
+    if (ret == MF_OK) {
+      // (one copy: the three lie behind each other, 256-byte aligned)
+      std::vector<char> buf((size_t)(z1 - (char *)w.gs));
+      e = hipMemcpyAsync(buf.data(), w.gs, buf.size(), hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e != hipSuccess) ret = fail(MF_ERR_HIP, std::string("solve: ") + hipGetErrorString(e));
+      std::memcpy(&back.gs, buf.data(), sizeof(GridSync));
+      std::memcpy(back.stats, buf.data() + ((char *)w.stats - (char *)w.gs), sizeof(back.stats));
+      std::memcpy(back.hist, buf.data() + ((char *)w.hist - (char *)w.gs), sizeof(back.hist));
+      if (ret == MF_OK && back.gs.abort)
+        ret = fail(MF_ERR_COOP, "solve: grid barrier timed out (grid not co-resident?)");
+    }
+    if (ret != MF_OK) break;
+    std::memcpy(stats, back.stats, sizeof(stats));
+    r.iterations += (int)stats[kStIters];
+    r.refreshes += (int)stats[kStRefresh];
+    for (int i = 0; i < 5; ++i) r.prec_hist[i] += (long long)back.hist[i];
+    if (!mixed && r.fell_back) r.prec_hist[0] += (long long)stats[kStIters] * t->tilenum;
+    if (!mixed || stats[kStFallback] == 0.0) break;
+    // FP64 from the x that the mixed solve reached
+    mixed = false;
+    r.fell_back = 1;
+    a.maxiter = opt.maxiter - r.iterations;
+    if (opt.fixed_iters > 0) a.fixed_iters = opt.fixed_iters - r.iterations;
+  }
+  if (e0) {
+    float ms = 0.0f;
+    if (ret == MF_OK && hipEventRecord(e1, st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
+        hipEventElapsedTime(&ms, e0, e1) == hipSuccess)
+      r.time_ms = ms;
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+  }
+  if (ret != MF_OK) return ret;
+  const double bb = stats[kStBB];
+  r.rel_residual = bb > 0 ? std::sqrt(stats[kStTrue] / bb) : std::sqrt(stats[kStTrue]);
+  r.rel_residual_recursive = bb > 0 ? std::sqrt(stats[kStRecursive] / bb) : 0.0;
+  r.grid_blocks = G;
+  r.form_used = MF_FORM_RESIDENT;
+  r.policy_used = opt.policy;
+  ret = (int)stats[kStStatus];
+  if (ret == MF_OK && opt.fixed_iters <= 0 && !(r.rel_residual <= opt.tol)) ret = MF_NOT_CONVERGED;
+  r.status = ret;
+  if (rep) *rep = r;
+  if (ret == MF_ERR_BREAKDOWN) set_error("solve: breakdown (zero or non-finite denominator)");
+  if (ret == MF_NOT_CONVERGED) set_error("solve: tolerance not reached");
+  return ret;
 }
 
 mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_solve_opts *o,
@@ -1486,13 +1709,18 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   MF_HIP(hipSetDevice(t->dev.device));
   hipStream_t st = (hipStream_t)opt.stream;
   const int mode = spmv_mode_for(opt.policy);
+  if (opt.form < MF_FORM_AUTO || opt.form > MF_FORM_RESIDENT) return fail(MF_ERR_ARG, "solve: unknown form");
+  {
+    int Gs = 0;
+    MF_TRY(strip_grid(t, opt, bicg, &Gs));
+    if (Gs > 0) return run_strips(t, d_b, d_x, opt, rep, Gs, noalloc);
+  }
 
   const void *kern;
-  int G = 0, block = kBlock;
+  int G = 0;
   mf_status sst = MF_OK;
   bool resident_windows = false;
   HostSchedule nsched;  // allocation-free solves: the schedule built on the host
-  if (opt.form < MF_FORM_AUTO || opt.form > MF_FORM_RESIDENT) return fail(MF_ERR_ARG, "solve: unknown form");
   {
     // The grid is at most the occupancy of the streamed kernel (one block of
     // 16 waves per CU for both forms).  Unless the memory form is asked for,
@@ -1505,18 +1733,7 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
                                : (mode == kAll64 ? (const void *)k_cg<kAll64, false>
                                   : mode == kPerSeg ? (const void *)k_cg<kPerSeg, false>
                                                     : (const void *)k_cg<kPerTile, false>);
-    // Without an override, a small system gets about 1024 rows per block (at
-    // least 4 blocks; whole multiples of 8 from 8 on, for the XCD-contiguous
-    // block order), so the grid-wide sums and syncs span fewer blocks: on
-    // MI355X an FP64 CG iteration of a 4096-row system takes 10.1 us on 4
-    // blocks against 13.5 us on the full grid, and of a 32768-row one 11.1 us
-    // on 32 blocks against 14.4 us.  From about 256k rows on, the full grid.
-    int want = opt.blocks;
-    if (want <= 0) {
-      const int rows = t->tilem * 16;
-      want = std::max(4, (rows + 1023) / 1024);
-      if (want >= 8) want = (want + 7) / 8 * 8;
-    }
+    const int want = want_blocks(t, opt);
     sst = grid_for(kstream, want, &G);
     if (sst != MF_OK) return sst;
     if (noalloc) {
@@ -1549,13 +1766,15 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   if (noalloc) {
     unsigned char *base = nullptr;
     MF_TRY(scratch_address(t->dev.device, &base));
-    MF_TRY(scratch_layout(t, G, nsched, base, w, scr_sched, st));
+    unsigned char *spare = nullptr;
+    size_t spare_bytes = 0;
+    MF_TRY(scratch_layout(t, G, nsched, base, w, scr_sched, st, &spare, &spare_bytes));
     sch = &scr_sched;
   } else {
     sst = get_workspace(t, G, w);
     if (sst != MF_OK) return sst;
     MF_HIP(hipMemsetAsync(w.gs, 0, sizeof(GridSync), st));
-    MF_HIP(hipMemsetAsync(w.mbox, 0, ((size_t)G + 1) * kMboxWords * 8, st));
+    MF_HIP(hipMemsetAsync(w.mbox, 0, (size_t)G * kMboxWords * 8, st));
     if (t->sched.nheavy > 0)
       MF_HIP(hipMemsetAsync(t->sched.heavy_cnt, 0, sizeof(unsigned) * t->sched.nheavy, st));
     MF_HIP(hipMemsetAsync(w.hist, 0, 5 * 8, st));
@@ -1629,16 +1848,7 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
     MF_HIP(hipEventRecord(e0, st));
   }
   void *args[] = {&a};
-  // The grid never exceeds what the occupancy query says is resident at once.
-  // A cooperative launch also guarantees it; when the runtime refuses one
-  // (e.g. another process holds the device's cooperative queue) the same grid
-  // is launched normally: the barrier needs only atomics, and its bounded
-  // spin turns a block that is not resident into a reported abort.
-  hipError_t le = hipLaunchCooperativeKernel(kern, dim3(G), dim3(block), args, 0, st);
-  if (le == hipErrorIllegalState || le == hipErrorNotSupported) {
-    (void)hipGetLastError();
-    le = hipLaunchKernel(kern, dim3(G), dim3(block), args, 0, st);
-  }
+  const hipError_t le = launch_grid(kern, G, args, st);
   if (le != hipSuccess) {
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);

@@ -3,6 +3,8 @@
 #include <algorithm>
 #include <cmath>
 #include <numeric>
+#include <queue>
+#include <vector>
 
 #include "mf_internal.h"
 
@@ -144,6 +146,36 @@ void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo
     P.any_near = P.any_near || d.cls == kStripNear;
   }
   P.ok = P.npacked <= 0xffffffffull && P.nfull <= 0xffffffffull;
+}
+
+void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s) {
+  const StripLayout &L = t->strips;
+  s.nwaves = nwaves;
+  s.wave_tr.resize(nwaves + 1);
+  s.wave_piece.assign(nwaves + 1, 0);
+  s.piece_order.clear();
+  auto bound = [&](int w) { return (int)((long long)L.nstrips * w / nwaves); };
+  for (int w = 0; w <= nwaves; ++w) s.wave_tr[w] = std::min(4 * bound(w), t->tilem);
+  if (L.npieces == 0) return;
+  // a strip costs its pairs and about six pairs' worth of own rows and waits
+  using Load = std::pair<int, int>;
+  std::priority_queue<Load, std::vector<Load>, std::greater<Load>> pq;
+  for (int w = 0; w < nwaves; ++w) {
+    int c = 0;
+    for (int i = bound(w); i < bound(w + 1); ++i) c += 6 + L.hdesc[i].npair;
+    pq.push({c, w});
+  }
+  std::vector<std::vector<int>> mine(nwaves);
+  for (int q = 0; q < L.npieces; ++q) {
+    const Load top = pq.top();
+    pq.pop();
+    mine[top.second].push_back(q);
+    pq.push({top.first + 4 + L.hdesc[L.nstrips + q].npair, top.second});
+  }
+  for (int w = 0; w < nwaves; ++w) {
+    s.piece_order.insert(s.piece_order.end(), mine[w].begin(), mine[w].end());
+    s.wave_piece[w + 1] = (int)s.piece_order.size();
+  }
 }
 
 }  // namespace mf

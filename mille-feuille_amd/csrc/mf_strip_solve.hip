@@ -1,0 +1,416 @@
+// mf_strip_solve.hip -- persistent CG over row strips, its vectors on chip.
+//
+// One cooperative launch runs the whole solve, as in mf_solve.hip, on the row
+// strips of the handle (mf_strips.h): a wave owns up to kMaxWaveStrips strips,
+// 64 rows each, one row per lane.  Only the vector that the product gathers
+// (r) is in memory.  The search direction p, s = A p and the iterate x of the
+// wave's rows stay in the lanes' registers for the whole solve, and w = A r
+// and the own entries of r pass from the product to the update through the
+// wave's part of the LDS, so an iteration reads the matrix and r and writes r
+// (FP64: 16 bytes a row besides the matrix, instead of 80).  x goes to memory
+// when the residual is recomputed, and at the end.
+//
+// Arithmetic: sums and scalars FP64.  Under a mixed policy r, p and s are
+// rounded to FP32 where the tile solver stores them in FP32, and the strips
+// multiply the FP32 payload (in FP64 arithmetic; packed strips hold it
+// exactly).  A wave whose learned levels include FP64 runs its strips at FP64.
+#include <cmath>
+#include <type_traits>
+
+#include "mf_strip_solve.h"
+
+namespace mf {
+
+namespace {
+
+__device__ __forceinline__ int solver_wave() {
+  const int G = gridDim.x;
+  const int lb = (G & 7) ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3);
+  return __builtin_amdgcn_readfirstlane(lb * kWavesPerBlock + (int)(threadIdx.x >> 6));
+}
+
+// Store that writes through the XCD's L2 (see mf_solve.hip).
+template <typename T>
+__device__ __forceinline__ void wt(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ double sum16(double v) {
+#pragma unroll
+  for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+  return v;
+}
+
+// The wave's strips [s0, s0 + n).
+struct StripWave {
+  int s0, n, lane;
+};
+
+// Sum of the pieces of lane's long row, posted by the waves that hold them
+// (values tagged with the product's ordinal, as in grid_sum_values; waits are
+// bounded).
+__device__ __forceinline__ double take_pieces(const StripSolveArgs &a, int h, unsigned tag) {
+  const LongRow lr = a.S.lrow[h];
+  double sum = 0.0;
+  for (int j = 0; j < lr.n; ++j) {
+    double v[1] = {0.0};
+    if (!mbox_take<1>(a.pmail + 2 * (size_t)(lr.first + j), tag, a.gs, v)) break;
+    sum += v[0];
+  }
+  return sum;
+}
+
+// Products of the wave's pieces (posted for the rows' owners), then of its
+// strips: w and the rows' own entries of x to wl and rl (lane's slot of strip
+// k at 64 k), and the sums of own^2 and w * own.  Pieces never wait, and an
+// owner waits only after its own pieces, so every wait ends.
+template <typename XT>
+__device__ __forceinline__ void strip_product(const StripSolveArgs &a, const StripWave &w, const XT *__restrict__ x,
+                                              unsigned tag, bool v32, double *wl, double *rl, double (&g)[2]) {
+  const StripView &S = a.S;
+  g[0] = g[1] = 0.0;
+  if (S.npieces > 0) {
+    const int wid = solver_wave();
+    const int q1 = __builtin_amdgcn_readfirstlane(a.wave_piece[wid + 1]);
+    for (int q = __builtin_amdgcn_readfirstlane(a.wave_piece[wid]); q < q1; ++q) {
+      const int pc = __builtin_amdgcn_readfirstlane(a.piece_order[q]);
+      const double v[1] = {wave_sum(strip_sum(S, strip_desc(S, S.nstrips + pc), x, w.lane, 0.0, v32))};
+      if (w.lane == 0) mbox_post<1>(a.pmail + 2 * (size_t)pc, tag, v);
+    }
+  }
+#pragma unroll 1
+  for (int k = 0; k < w.n; ++k) {
+    const int s = w.s0 + k;
+    const StripDesc d = strip_desc(S, s);
+    bool lng;
+    const int row = strip_row(S, s, w.lane, lng);
+    const double own = row >= 0 ? (double)x[row] : 0.0;
+    double acc = 0.0;
+    if ((d.flags & kStripLead) && row >= 0)
+      acc = (v32 ? (double)S.lead32[64 * s + w.lane] : S.lead64[64 * s + w.lane]) * own;
+    acc = strip_sum(S, d, x, w.lane, acc, v32);
+    if ((d.flags & kStripLong) && lng) acc += take_pieces(a, S.lane_long[64 * s + w.lane], tag);
+    wl[64 * k + w.lane] = acc;
+    rl[64 * k + w.lane] = own;
+    g[0] += own * own;
+    g[1] += acc * own;
+  }
+}
+
+// Tiles [t0, t1) counted per level (wave-uniform).
+__device__ __forceinline__ void count_levels(const uint8_t *prec, int t0, int t1, int lane, unsigned (&n)[5]) {
+#pragma unroll
+  for (int l = 0; l < 5; ++l) n[l] = 0;
+  for (int t = t0; t < t1; t += kWave) {
+    const int u = t + lane;
+    const int p = u < t1 ? prec[u] : 255;
+#pragma unroll
+    for (int l = 0; l < 5; ++l) n[l] += (unsigned)__builtin_popcountll(__ballot(p == l));
+  }
+}
+
+__device__ __forceinline__ void add_hist(unsigned long long c, unsigned long long *h, int lane) {
+  if (lane == 0 && c) atomicAdd(h, c);
+}
+
+}  // namespace
+
+// Learned levels of tiles [t0, t1) from the installed network.  Out of line:
+// it runs once per check interval, and inlined its 36 operand registers were
+// spilled around every product.
+__device__ __noinline__ void infer_levels(const int *tile_col, InferCtx c, int t0, int t1, int lane) {
+  TileView A;
+  A.tile_col = tile_col;
+  wave_infer_tiles(A, c, t0, t1, lane);
+}
+
+// Chronopoulos-Gear CG: w = A r with gamma = r.r and delta = w.r, one fused
+// grid sum, then p = r + beta p, s = w + beta s, x += alpha p, r -= alpha s and
+// a grid sync (the exits, refreshes and fallback of k_cg; a mixed solve that
+// needs FP64 ends, and the host starts an FP64 one from its x).
+//
+// Measured on MI355X, us per iteration, FP64 / error bound (streamed tiles with
+// the vectors in memory before): 7-point 128^3 31.2 / 32.0 (54.0 / 45.0), of
+// which the product 16.9, the update's stores 6.5 and the two synchronisations
+// 7.6; 117 x 89 x 86 16.2 / 17.4 (30.0 / 29.4); 64^3 10.6 / 11.8 (16.7 / 18.7), of
+// which synchronisation 6; 5-point 64^2 5.5 / 6.9 (10.8 / 13.3); 200k-row power
+// law 30.7 / 29.9 (97 / 107).  The 128^3 product moves 84 MB (5.0 TB/s).
+//
+// Each round of the
+// loop is one product: of x for a residual (kRes), of r for an iteration
+// (kIter) or of p for s after a refresh (kDir).
+template <int KS, bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
+  using VT = typename std::conditional<MIXED, float, double>::type;
+  enum Round { kRes, kIter, kDir };
+  __shared__ double lds[kMaxGridSum * kWavesPerBlock];
+  __shared__ double lw[kWavesPerBlock][KS * 64];  // A times the vector, of the wave's rows
+  __shared__ double lr[kWavesPerBlock][KS * 64];  // the vector's own entries
+  const int wid = solver_wave();
+  double *wl = lw[threadIdx.x >> 6], *rl = lr[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
+  StripWave W;
+  W.lane = lane;
+  {
+    const int nw = gridDim.x * kWavesPerBlock;
+    W.s0 = (int)((long long)a.S.nstrips * wid / nw);
+    W.n = (int)((long long)a.S.nstrips * (wid + 1) / nw) - W.s0;
+  }
+  // tiles whose levels the wave counts (and infers: learned solves run on
+  // unsorted strips, whose tile-rows are the wave's own)
+  int t0 = 0, t1 = 0;
+  if (MIXED) {
+    if (a.S.rowmap) {
+      const int nw = gridDim.x * kWavesPerBlock;
+      t0 = (int)((long long)a.A.tilenum * wid / nw);
+      t1 = (int)((long long)a.A.tilenum * (wid + 1) / nw);
+    } else {
+      t0 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * W.s0, a.A.tilem)]);
+      t1 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * (W.s0 + W.n), a.A.tilem)]);
+    }
+  }
+  auto row_of = [&](int k) {
+    // (the lane is hidden from the optimizer here, which would otherwise keep
+    // every strip's row and row-map address in registers for the whole solve)
+    int l = lane;
+    asm("" : "+v"(l));
+    bool lng;
+    return strip_row(a.S, W.s0 + k, l, lng);
+  };
+  unsigned epoch = 0, tag = 0;
+  int slot = 0, lds_i = 0;
+  VT p[KS], s[KS];
+  double x[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    p[k] = s[k] = VT(0);
+    x[k] = 0.0;
+    if (k < W.n) {
+      const int row = row_of(k);
+      if (row >= 0) x[k] = a.x[row];
+    }
+  }
+  const bool learned = MIXED && a.mlp != nullptr;
+  double rr = 0.0, bb = 0.0, stop2 = 0.0, rr_ref = 0.0, gamma_old = 1.0, alpha_old = 1.0;
+  int it = 0, it_ref = 0, refresh = -1, status = 0;
+  bool first = true;      // the next step starts a new direction
+  bool fell = false;      // mixed: stopped for the FP64 solver to go on
+  bool infer = learned;   // new levels in the next product
+  bool full64 = false;    // FP64 payload under FP32 vectors (learned FP64 levels)
+  bool end = false;       // this residual is the last one, for the report
+  unsigned nlev[5] = {0, 0, 0, 0, 0};  // the wave's tiles per level
+  unsigned long long hist[5] = {0, 0, 0, 0, 0};
+  if (MIXED && !learned) count_levels(a.A.prec, t0, t1, lane, nlev);
+
+  Round round = kRes;
+  for (;;) {
+    double gd[2];
+    ++tag;
+    if (MIXED && round == kIter) {
+      if (infer) {
+        InferCtx c;
+        c.w = a.mlp;
+        c.feat16 = a.feat16;
+        c.seg2 = a.seg2;
+        c.prec_out = a.prec_rw;
+        c.seg_scale = rr > 0.0 ? (float)(sqrt((double)a.nseg) / sqrt(rr)) : 0.0f;
+        c.progress = (float)(log10(fmax(bb > 0.0 ? sqrt(rr / bb) : 1.0, 1e-16)) / 16.0);
+        infer_levels(a.A.tile_col, c, t0, t1, lane);
+        count_levels(a.prec_rw, t0, t1, lane, nlev);
+        full64 = nlev[0] > 0;
+        infer = false;
+      }
+      strip_product(a, W, (const float *)a.r32, tag, !full64, wl, rl, gd);
+    } else {
+      const double *v = round == kRes ? a.x : round == kIter ? a.r : a.p;
+      strip_product(a, W, v, tag, false, wl, rl, gd);
+    }
+    if (round == kRes) {
+      // r = b - A x of the wave's rows (stored unless it is the last)
+      double tr[2] = {0.0, 0.0};
+      for (int k = 0; k < W.n; ++k) {
+        const int row = row_of(k);
+        if (row >= 0) {
+          const double bv = a.b[row];
+          double rv = bv - wl[64 * k + lane];
+          if (MIXED && !end) {
+            const float rf = (float)rv;
+            a.r32[row] = rf;
+            rv = rf;
+          } else if (!end) {
+            a.r[row] = rv;
+          }
+          tr[0] += rv * rv;
+          tr[1] += bv * bv;
+          if (learned && refresh < 0) {
+            // segment norms of r0 for the first inference
+            const double d2 = sum16(rv * rv);
+            if ((lane & 15) == 0) a.seg2[row >> 4] = (float)d2;
+          }
+        }
+      }
+      grid_sum<2>(tr, a.partials, a.gs, epoch, slot, lds, &lds_i);
+      if (end) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          a.stats[kStIters] = it;
+          a.stats[kStRefresh] = refresh;
+          a.stats[kStFallback] = fell;
+          a.stats[kStRecursive] = rr;
+          a.stats[kStTrue] = tr[0];
+          a.stats[kStBB] = bb;
+          a.stats[kStStatus] = status;
+        }
+        break;
+      }
+      ++refresh;
+      if (refresh == 0) {  // the initial residual
+        bb = tr[1];
+        stop2 = uniform_double(a.tol2 * bb);
+        rr = rr_ref = tr[0];
+        if (bb == 0.0 || (a.fixed_iters <= 0 && rr <= stop2)) {
+          end = true;
+        } else {
+          round = kIter;
+        }
+        continue;
+      }
+      it_ref = it;
+      // A recursive residual far below the true one leaves beta meaningless,
+      // and so does one that met the tolerance while the true one did not:
+      // restart the search direction from the recomputed residual.
+      if (tr[0] > 4.0 * rr || (rr <= stop2 && tr[0] > stop2)) first = true;
+      rr = tr[0];
+      if (tr[0] <= stop2) {
+        end = true;
+        continue;
+      }
+      if (it >= a.maxiter) {
+        status = MF_NOT_CONVERGED;
+        end = true;
+        continue;
+      }
+      if (MIXED && (tr[0] > 0.25 * rr_ref || refresh > a.max_refresh)) {
+        // stagnation: x is the start of an FP64 solve
+        fell = end = true;
+        continue;
+      }
+      rr_ref = rr;
+      if (first) {
+        round = kIter;
+        grid_sync(a.gs, epoch, &lds_i);
+      } else {
+        // s = A p in FP64 so that s and the new r stay consistent
+        round = kDir;
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+          if (k < W.n) {
+            const int row = row_of(k);
+            if (row >= 0) wt(a.p + row, (double)p[k]);
+          }
+        grid_sync(a.gs, epoch, &lds_i);
+      }
+      continue;
+    }
+    if (round == kDir) {
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < W.n) s[k] = (VT)wl[64 * k + lane];
+      round = kIter;
+      // (a wave that went on would post the next product's piece sums over
+      // these)
+      grid_sync(a.gs, epoch, &lds_i);
+      continue;
+    }
+    if (MIXED) {
+#pragma unroll
+      for (int l = 0; l < 5; ++l) hist[l] += nlev[l];
+    }
+    grid_sum_values<2>(gd, a.mbox, a.gs, epoch, lds);
+    const double gamma = gd[0], delta = gd[1];
+    rr = gamma;
+    bool pending = false;  // recompute the FP64 residual before the step
+    if (a.fixed_iters <= 0) {
+      pending = gamma <= stop2 || (MIXED &&
+                                   (gamma <= a.ratio2 * rr_ref || it - it_ref >= a.refresh_every));
+      if (!pending && it >= a.maxiter) {
+        status = MF_NOT_CONVERGED;
+        end = true;
+      }
+    }
+    double beta = 0.0, alpha = gamma / delta;
+    if (!first) {
+      beta = gamma / gamma_old;
+      alpha = gamma / (delta - beta * gamma / alpha_old);
+    }
+    if (!pending && !end && (!isfinite(alpha) || alpha == 0.0 || (MIXED && !(alpha > 0.0)))) {
+      // (a low-precision operator that lost definiteness: FP64 goes on)
+      if (MIXED) fell = true;
+      else status = MF_ERR_BREAKDOWN;
+      end = true;
+    }
+    const bool step = !pending && !end;
+    // p = r + beta p, x += alpha p: needed by no other wave, so done while the
+    // arrivals of the other blocks are awaited
+    auto update_px = [&] {
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < W.n) {
+          p[k] = (VT)(rl[64 * k + lane] + beta * (double)p[k]);
+          x[k] += alpha * (double)p[k];
+        }
+    };
+    if (step) {
+      first = false;
+      alpha = uniform_double(alpha);
+      beta = uniform_double(beta);
+      gamma_old = gamma;
+      alpha_old = alpha;
+      ++it;
+      const bool lupd = learned && (it % a.check_interval) == 0;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        if (k < W.n) {
+          const int row = row_of(k);
+          // (mixed: w, p, s and r rounded to FP32 as the tile solver stores them)
+          s[k] = (VT)((double)(VT)wl[64 * k + lane] + beta * (double)s[k]);
+          const VT rn = (VT)(rl[64 * k + lane] - alpha * (double)s[k]);
+          if (row >= 0) wt((MIXED ? (VT *)a.r32 : (VT *)a.r) + row, rn);
+          if (MIXED && lupd) {
+            const double d = sum16(row >= 0 ? (double)rn * (double)rn : 0.0);
+            if ((lane & 15) == 0 && row >= 0) wt(a.seg2 + (row >> 4), (float)d);
+          }
+        }
+      }
+      infer = lupd;
+      end = a.fixed_iters > 0 && it >= a.fixed_iters;
+    }
+    if (pending || end) {
+      // x to memory, for the residual
+      if (step) update_px();
+      round = kRes;
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < W.n) {
+          const int row = row_of(k);
+          if (row >= 0) wt(a.x + row, x[k]);
+        }
+    }
+    grid_arrive<false>(a.gs, epoch);
+    if (step && !end) update_px();
+    grid_wait(a.gs, epoch);
+  }
+  if (MIXED) {
+#pragma unroll
+    for (int l = 0; l < 5; ++l) add_hist(hist[l], a.hist + l, lane);
+  }
+}
+
+
+const void *strip_cg_kernel(int strips, bool mixed) {
+  if (strips <= 1) return mixed ? (const void *)k_cg_strip<1, true> : (const void *)k_cg_strip<1, false>;
+  if (strips <= 2) return mixed ? (const void *)k_cg_strip<2, true> : (const void *)k_cg_strip<2, false>;
+  if (strips <= 4) return mixed ? (const void *)k_cg_strip<4, true> : (const void *)k_cg_strip<4, false>;
+  return mixed ? (const void *)k_cg_strip<8, true> : (const void *)k_cg_strip<8, false>;
+}
+
+}  // namespace mf

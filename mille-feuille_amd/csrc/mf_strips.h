@@ -165,12 +165,12 @@ __device__ __forceinline__ double strip_full_sum(const VT *__restrict__ v, const
 }
 
 // Sum of the lane's entries of a strip or piece (without the lead), added to
-// acc.  XT double or float: the vector; V32: full and near strips
-// multiply the FP32 payload.  Strips of more than four pairs load the next four word pairs
-// before the gathers of the current ones.
-template <bool V32, typename XT>
+// acc.  XT double or float: the vector; v32 (float vectors only): full and
+// near strips multiply the FP32 payload.  Strips of more than four pairs load
+// the next four word pairs before the gathers of the current ones.
+template <typename XT>
 __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc &d, const XT *__restrict__ x,
-                                            int lane, double acc) {
+                                            int lane, double acc, bool v32 = false) {
   const int np = d.npair;
   if (d.cls == kStripPacked) {
     const uint32_t *w = S.words + (size_t)d.off * 128;
@@ -215,12 +215,13 @@ __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc 
     }
   }
   const size_t o = (size_t)d.off * 128;
-  using VT = typename std::conditional<V32, float, double>::type;
-  const VT *v;
-  if constexpr (V32) v = S.vf + o; else v = S.vv + o;
-  if (d.cls == kStripNear)
-    return strip_full_sum<true>(v, S.vh + o, np, lane, x + ((ptrdiff_t)d.base - (1 << 15)), acc);
-  return strip_full_sum<false>(v, S.vc + o, np, lane, x, acc);
+  const XT *xn = x + ((ptrdiff_t)d.base - (1 << 15));
+  if (std::is_same<XT, float>::value && v32) {
+    if (d.cls == kStripNear) return strip_full_sum<true>(S.vf + o, S.vh + o, np, lane, xn, acc);
+    return strip_full_sum<false>(S.vf + o, S.vc + o, np, lane, x, acc);
+  }
+  if (d.cls == kStripNear) return strip_full_sum<true>(S.vv + o, S.vh + o, np, lane, xn, acc);
+  return strip_full_sum<false>(S.vv + o, S.vc + o, np, lane, x, acc);
 }
 
 __device__ __forceinline__ StripDesc strip_desc(const StripView &S, int i) {

@@ -255,6 +255,7 @@ mf_status upload_tiles(mf_tiled *t, int device, const int *rowptr) {
     if (e != hipSuccess) return fail(MF_ERR_HIP, std::string("tile upload: ") + hipGetErrorString(e));
   }
   MF_TRY(build_strips(t, rowptr));
+  t->strips.lean = lean_strips(t);
   d.spmv_kernel = default_spmv_kernel(t);
   return MF_OK;
 }
@@ -266,7 +267,7 @@ bool regular_tilerows(const mf_tiled *t) {
   return t->dev.max_tiles_per_row <= 4.0 * mean + 8.0;
 }
 
-int default_spmv_kernel(const mf_tiled *t) {
+bool lean_strips(const mf_tiled *t) {
   // Both kernels run at the rate of their bytes (strips: an entry's word or
   // value and column, a lead per row; tiles: value, byte and metadata), so the
   // fewer bytes win, with a margin for what strips save besides.  Measured on
@@ -278,13 +279,15 @@ int default_spmv_kernel(const mf_tiled *t) {
   // against 19 MB) 5.7 / 6.2 and 16.4 / 13.9; 200k-row power-law graph (packed,
   // pieces; 16 against 135 MB) 25.8 / 149 and 41 / 215.
   const StripLayout &L = t->strips;
-  if (L.nstrips == 0) return MF_SPMV_STREAM;
+  if (L.nstrips == 0) return false;
   double strip = 8.0 * 64.0 * L.nstrips;
   for (const StripDesc &d : L.hdesc)
     strip += 128.0 * d.npair * (d.cls == kStripPacked ? 4.0 : d.cls == kStripNear ? 10.0 : 12.0);
   const double tiles = 9.0 * t->dev.npay + 13.0 * t->tilenum;
-  return strip <= 1.2 * tiles ? MF_SPMV_STRIP : MF_SPMV_STREAM;
+  return strip <= 1.2 * tiles;
 }
+
+int default_spmv_kernel(const mf_tiled *t) { return t->strips.lean ? MF_SPMV_STRIP : MF_SPMV_STREAM; }
 
 // Stand-alone SpMV schedule of about wave_nnz payload slots per wave, heavy
 // tile-rows cut into one-window pieces, uploaded in place of the previous one.
@@ -328,12 +331,13 @@ void free_device(mf_tiled *t) {
   void *ptrs[] = {d.slab, d.spmv_desc, d.spmv_part, d.spmv_cnt, d.spmv_hn, d.spmv_hbase, d.mlp, d.feat16,
                   t->sched.wave_tr, t->sched.wave_res, t->sched.wave_win, t->sched.win_desc, t->sched.heavy_part,
                   t->sched.heavy_cnt, t->sched.heavy_n, t->sched.heavy_base, t->sched.heavy_tr,
-                  t->sched.wave_heavy, t->work};
+                  t->sched.wave_heavy, t->strip_sched.slab, t->work};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   free_strips(t);
   d = DeviceLayout();
   t->sched = Schedule();
+  t->strip_sched = StripSchedule();
   t->work = nullptr;
   t->work_bytes = 0;
 }

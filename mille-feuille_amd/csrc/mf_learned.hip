@@ -364,6 +364,8 @@ mf_status build_static_features(mf_tiled *t) {
     MF_HIP(hipMemcpy(qerr.data(), t->dev.qerr, sizeof(double) * 3 * (size_t)T, hipMemcpyDeviceToHost));
   std::vector<double> tsum(T, 0.0), amax(T, 0.0), amin(T, 0.0);
   std::vector<double> rowsum(TM, 0.0), dom(TM, INFINITY);
+  // row starts past the last tile's (a short last tile-row) count as 0
+  auto start = [&](int i) { return i < t->csrptrlen ? (int)t->Blockcsr_Ptr[i] : 0; };
   for (int R = 0; R < TM; ++R) {
     double diag[16] = {0}, off[16] = {0};
     bool has[16] = {false};
@@ -373,8 +375,8 @@ mf_status build_static_features(mf_tiled *t) {
       const int p0 = t->csrptr_offset[ti];
       double mx = 0.0, mn = INFINITY, s = 0.0;
       for (int r = 0; r < 16; ++r) {
-        const int a = z0 + t->Blockcsr_Ptr[p0 + r];
-        const int b = r < 15 ? z0 + t->Blockcsr_Ptr[p0 + r + 1] : z1;
+        const int a = z0 + start(p0 + r);
+        const int b = r < 15 ? z0 + start(p0 + r + 1) : z1;
         for (int k = a; k < b && k < z1; ++k) {
           const double v = std::fabs(t->Blockcsr_Val[k]);
           s += v;

@@ -1519,17 +1519,17 @@ static mf_status strip_grid(const mf_tiled *t, const mf_solve_opts &opt, bool bi
   *G = 0;
   const StripLayout &L = t->strips;
   const int pol = opt.policy;
-  if (bicg || !L.lean || opt.form == MF_FORM_MEMORY || 2 * L.npieces > t->rowA) return MF_OK;
+  if (!L.lean || opt.form == MF_FORM_MEMORY || 2 * L.npieces > t->rowA) return MF_OK;
   if (pol != MF_POLICY_FP64 && pol != MF_POLICY_ERRBOUND && !(pol == MF_POLICY_LEARNED && !L.sorted)) return MF_OK;
   int g = 0;
-  MF_TRY(grid_for(strip_cg_kernel(kMaxWaveStrips, pol != MF_POLICY_FP64), want_blocks(t, opt), &g, kBlock, true));
+  MF_TRY(grid_for(strip_solve_kernel(kMaxWaveStrips, bicg, pol != MF_POLICY_FP64), want_blocks(t, opt), &g, kBlock, true));
   const int per = (L.nstrips + g * kWavesPerBlock - 1) / (g * kWavesPerBlock);
   if (per <= kMaxWaveStrips) *G = g;
   return MF_OK;
 }
 
 static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solve_opts opt, mf_report *rep,
-                            int G, bool noalloc) {
+                            int G, bool bicg, bool noalloc) {
   hipStream_t st = (hipStream_t)opt.stream;
   const StripLayout &L = t->strips;
   const int nwaves = G * kWavesPerBlock, per = (L.nstrips + nwaves - 1) / nwaves;
@@ -1584,6 +1584,7 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
     MF_TRY(fill_u32(w.r + rows, (n - rows) * 8, 0u, st));
     MF_TRY(fill_u32(w.p + rows, (n - rows) * 8, 0u, st));
     MF_TRY(fill_u32(w.r32 + rows, (n - rows) * 4, 0u, st));
+    MF_TRY(fill_u32(w.p32 + rows, (n - rows) * 4, 0u, st));
   }
   StripSolveArgs a;
   a.S = strip_view_of(t);
@@ -1593,6 +1594,7 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
   a.r = w.r;
   a.p = w.p;
   a.r32 = w.r32;
+  a.p32 = w.p32;
   a.wave_piece = sc->d_wave_piece;
   a.piece_order = sc->d_piece_order;
   a.pmail = pmail;
@@ -1632,7 +1634,7 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
     if (ret == MF_OK) ret = fill_u32(w.mbox, (size_t)G * kMboxWords * 8, 0u, st);
     if (ret == MF_OK && mail_bytes) ret = fill_u32(pmail, mail_bytes, 0u, st);
     void *args[] = {&a};
-    hipError_t e = ret == MF_OK ? launch_grid(strip_cg_kernel(per, mixed), G, args, st) : hipSuccess;
+    hipError_t e = ret == MF_OK ? launch_grid(strip_solve_kernel(per, bicg, mixed), G, args, st) : hipSuccess;
     if (e != hipSuccess) ret = fail(MF_ERR_COOP, std::string("hipLaunchCooperativeKernel: ") + hipGetErrorString(e));
     struct Back {
       GridSync gs;
@@ -1657,12 +1659,16 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
     r.iterations += (int)stats[kStIters];
     r.refreshes += (int)stats[kStRefresh];
     for (int i = 0; i < 5; ++i) r.prec_hist[i] += (long long)back.hist[i];
-    if (!mixed && r.fell_back) r.prec_hist[0] += (long long)stats[kStIters] * t->tilenum;
+    if (!mixed && r.fell_back) r.prec_hist[0] += (long long)stats[kStIters] * t->tilenum * (bicg ? 2 : 1);
     if (!mixed || stats[kStFallback] == 0.0) break;
     // FP64 from the x that the mixed solve reached
     mixed = false;
     r.fell_back = 1;
     a.maxiter = opt.maxiter - r.iterations;
+    if (a.maxiter <= 0) {
+      stats[kStStatus] = MF_NOT_CONVERGED;
+      break;
+    }
     if (opt.fixed_iters > 0) a.fixed_iters = opt.fixed_iters - r.iterations;
   }
   if (e0) {
@@ -1713,7 +1719,7 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   {
     int Gs = 0;
     MF_TRY(strip_grid(t, opt, bicg, &Gs));
-    if (Gs > 0) return run_strips(t, d_b, d_x, opt, rep, Gs, noalloc);
+    if (Gs > 0) return run_strips(t, d_b, d_x, opt, rep, Gs, bicg, noalloc);
   }
 
   const void *kern;

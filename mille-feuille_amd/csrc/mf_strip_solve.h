@@ -26,8 +26,8 @@ struct StripSolveArgs {
   TileView A;                // tile levels (learned policy, histogram)
   const double *b;
   double *x;
-  double *r, *p;             // gathered vectors, FP64 ...
-  float *r32;                // ... and FP32 (mixed)
+  double *r, *p;             // vectors in memory, FP64 (r: BiCGSTAB's s) ...
+  float *r32, *p32;          // ... and FP32 (mixed)
   const int *wave_piece;     // per wave, bounds of its pieces in piece_order
   const int *piece_order;
   unsigned long long *pmail; // two tagged words per piece
@@ -45,7 +45,8 @@ struct StripSolveArgs {
   int nseg;
 };
 
-// Kernel of the strip CG for `strips` strips per wave (1 .. kMaxWaveStrips).
-const void *strip_cg_kernel(int strips, bool mixed);
+// Kernel of the strip CG or BiCGSTAB for `strips` strips per wave (1 ..
+// kMaxWaveStrips).
+const void *strip_solve_kernel(int strips, bool bicg, bool mixed);
 
 }  // namespace mf

@@ -1,9 +1,10 @@
-// mf_strip_solve.hip -- persistent CG over row strips, its vectors on chip.
+// mf_strip_solve.hip -- persistent CG and BiCGSTAB over row strips, their
+// vectors on chip.
 //
 // One cooperative launch runs the whole solve, as in mf_solve.hip, on the row
 // strips of the handle (mf_strips.h): a wave owns up to kMaxWaveStrips strips,
-// 64 rows each, one row per lane.  Only the vector that the product gathers
-// (r) is in memory.  The search direction p, s = A p and the iterate x of the
+// 64 rows each, one row per lane.  Only the vectors that a product gathers
+// (CG: r) are in memory.  The search direction p, s = A p and the iterate x of the
 // wave's rows stay in the lanes' registers for the whole solve, and w = A r
 // and the own entries of r pass from the product to the update through the
 // wave's part of the LDS, so an iteration reads the matrix and r and writes r
@@ -61,14 +62,15 @@ __device__ __forceinline__ double take_pieces(const StripSolveArgs &a, int h, un
 }
 
 // Products of the wave's pieces (posted for the rows' owners), then of its
-// strips: w and the rows' own entries of x to wl and rl (lane's slot of strip
-// k at 64 k), and the sums of own^2 and w * own.  Pieces never wait, and an
-// owner waits only after its own pieces, so every wait ends.
+// strips: w and (own_out) the rows' own entries of x to wl and rl (lane's slot of
+// strip k at 64 k), and the sums of own^2, w * own and w^2.  Pieces never
+// wait, and an owner waits only after its own pieces, so every wait ends.
 template <typename XT>
 __device__ __forceinline__ void strip_product(const StripSolveArgs &a, const StripWave &w, const XT *__restrict__ x,
-                                              unsigned tag, bool v32, double *wl, double *rl, double (&g)[2]) {
+                                              unsigned tag, bool v32, bool own_out, double *wl, double *rl,
+                                              double (&g)[3]) {
   const StripView &S = a.S;
-  g[0] = g[1] = 0.0;
+  g[0] = g[1] = g[2] = 0.0;
   if (S.npieces > 0) {
     const int wid = solver_wave();
     const int q1 = __builtin_amdgcn_readfirstlane(a.wave_piece[wid + 1]);
@@ -91,9 +93,10 @@ __device__ __forceinline__ void strip_product(const StripSolveArgs &a, const Str
     acc = strip_sum(S, d, x, w.lane, acc, v32);
     if ((d.flags & kStripLong) && lng) acc += take_pieces(a, S.lane_long[64 * s + w.lane], tag);
     wl[64 * k + w.lane] = acc;
-    rl[64 * k + w.lane] = own;
+    if (own_out) rl[64 * k + w.lane] = own;
     g[0] += own * own;
     g[1] += acc * own;
+    g[2] += acc * acc;
   }
 }
 
@@ -109,11 +112,52 @@ __device__ __forceinline__ void count_levels(const uint8_t *prec, int t0, int t1
   }
 }
 
+// The wave's strips, and the tiles whose levels it counts (and infers: learned
+// solves run on unsorted strips, whose tile-rows are the wave's own).
+template <bool MIXED>
+__device__ __forceinline__ void wave_share(const StripSolveArgs &a, int wid, int lane, StripWave &W, int &t0, int &t1) {
+  const int nw = gridDim.x * kWavesPerBlock;
+  W.lane = lane;
+  W.s0 = (int)((long long)a.S.nstrips * wid / nw);
+  W.n = (int)((long long)a.S.nstrips * (wid + 1) / nw) - W.s0;
+  t0 = t1 = 0;
+  if (!MIXED) return;
+  if (a.S.rowmap) {
+    t0 = (int)((long long)a.A.tilenum * wid / nw);
+    t1 = (int)((long long)a.A.tilenum * (wid + 1) / nw);
+  } else {
+    t0 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * W.s0, a.A.tilem)]);
+    t1 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * (W.s0 + W.n), a.A.tilem)]);
+  }
+}
+
+// Row of the lane in strip s0 + k.  The lane is hidden from the optimizer,
+// which would otherwise keep every strip's row and row-map address in
+// registers for the whole solve.
+__device__ __forceinline__ int wave_row(const StripSolveArgs &a, const StripWave &W, int k) {
+  int l = W.lane;
+  asm("" : "+v"(l));
+  bool lng;
+  return strip_row(a.S, W.s0 + k, l, lng);
+}
+
 __device__ __forceinline__ void add_hist(unsigned long long c, unsigned long long *h, int lane) {
   if (lane == 0 && c) atomicAdd(h, c);
 }
 
 }  // namespace
+
+// Inference context for a multiplied vector of squared norm v2.
+__device__ __forceinline__ InferCtx infer_ctx(const StripSolveArgs &a, double v2, double rr, double bb) {
+  InferCtx c;
+  c.w = a.mlp;
+  c.feat16 = a.feat16;
+  c.seg2 = a.seg2;
+  c.prec_out = a.prec_rw;
+  c.seg_scale = v2 > 0.0 ? (float)(sqrt((double)a.nseg) / sqrt(v2)) : 0.0f;
+  c.progress = (float)(log10(fmax(bb > 0.0 ? sqrt(rr / bb) : 1.0, 1e-16)) / 16.0);
+  return c;
+}
 
 // Learned levels of tiles [t0, t1) from the installed network.  Out of line:
 // it runs once per check interval, and inlined its 36 operand registers were
@@ -130,11 +174,11 @@ __device__ __noinline__ void infer_levels(const int *tile_col, InferCtx c, int t
 // needs FP64 ends, and the host starts an FP64 one from its x).
 //
 // Measured on MI355X, us per iteration, FP64 / error bound (streamed tiles with
-// the vectors in memory before): 7-point 128^3 31.2 / 32.0 (54.0 / 45.0), of
-// which the product 16.9, the update's stores 6.5 and the two synchronisations
-// 7.6; 117 x 89 x 86 16.2 / 17.4 (30.0 / 29.4); 64^3 10.6 / 11.8 (16.7 / 18.7), of
-// which synchronisation 6; 5-point 64^2 5.5 / 6.9 (10.8 / 13.3); 200k-row power
-// law 30.7 / 29.9 (97 / 107).  The 128^3 product moves 84 MB (5.0 TB/s).
+// the vectors in memory before): 7-point 128^3 28.9 / 29.9 (54.0 / 45.0), of
+// which the product 15, the update's stores 6.5 and the two synchronisations
+// 7.6; 117 x 89 x 86 15.3 / 16.6 (30.0 / 29.4); 64^3 10.3 / 11.6 (16.7 / 18.7), of
+// which synchronisation 6; 5-point 64^2 5.6 / 6.9 (10.8 / 13.3); 200k-row power
+// law 30.6 / 30.1 (97 / 107).  The 128^3 product moves 84 MB.
 //
 // Each round of the
 // loop is one product: of x for a residual (kRes), of r for an iteration
@@ -150,33 +194,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
   double *wl = lw[threadIdx.x >> 6], *rl = lr[threadIdx.x >> 6];
   const int lane = threadIdx.x & 63;
   StripWave W;
-  W.lane = lane;
-  {
-    const int nw = gridDim.x * kWavesPerBlock;
-    W.s0 = (int)((long long)a.S.nstrips * wid / nw);
-    W.n = (int)((long long)a.S.nstrips * (wid + 1) / nw) - W.s0;
-  }
-  // tiles whose levels the wave counts (and infers: learned solves run on
-  // unsorted strips, whose tile-rows are the wave's own)
-  int t0 = 0, t1 = 0;
-  if (MIXED) {
-    if (a.S.rowmap) {
-      const int nw = gridDim.x * kWavesPerBlock;
-      t0 = (int)((long long)a.A.tilenum * wid / nw);
-      t1 = (int)((long long)a.A.tilenum * (wid + 1) / nw);
-    } else {
-      t0 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * W.s0, a.A.tilem)]);
-      t1 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * (W.s0 + W.n), a.A.tilem)]);
-    }
-  }
-  auto row_of = [&](int k) {
-    // (the lane is hidden from the optimizer here, which would otherwise keep
-    // every strip's row and row-map address in registers for the whole solve)
-    int l = lane;
-    asm("" : "+v"(l));
-    bool lng;
-    return strip_row(a.S, W.s0 + k, l, lng);
-  };
+  int t0, t1;
+  wave_share<MIXED>(a, wid, lane, W, t0, t1);
+  auto row_of = [&](int k) { return wave_row(a, W, k); };
   unsigned epoch = 0, tag = 0;
   int slot = 0, lds_i = 0;
   VT p[KS], s[KS];
@@ -204,26 +224,19 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
 
   Round round = kRes;
   for (;;) {
-    double gd[2];
+    double gd3[3];
     ++tag;
     if (MIXED && round == kIter) {
       if (infer) {
-        InferCtx c;
-        c.w = a.mlp;
-        c.feat16 = a.feat16;
-        c.seg2 = a.seg2;
-        c.prec_out = a.prec_rw;
-        c.seg_scale = rr > 0.0 ? (float)(sqrt((double)a.nseg) / sqrt(rr)) : 0.0f;
-        c.progress = (float)(log10(fmax(bb > 0.0 ? sqrt(rr / bb) : 1.0, 1e-16)) / 16.0);
-        infer_levels(a.A.tile_col, c, t0, t1, lane);
+        infer_levels(a.A.tile_col, infer_ctx(a, rr, rr, bb), t0, t1, lane);
         count_levels(a.prec_rw, t0, t1, lane, nlev);
         full64 = nlev[0] > 0;
         infer = false;
       }
-      strip_product(a, W, (const float *)a.r32, tag, !full64, wl, rl, gd);
+      strip_product(a, W, (const float *)a.r32, tag, !full64, true, wl, rl, gd3);
     } else {
       const double *v = round == kRes ? a.x : round == kIter ? a.r : a.p;
-      strip_product(a, W, v, tag, false, wl, rl, gd);
+      strip_product(a, W, v, tag, false, true, wl, rl, gd3);
     }
     if (round == kRes) {
       // r = b - A x of the wave's rows (stored unless it is the last)
@@ -325,6 +338,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
 #pragma unroll
       for (int l = 0; l < 5; ++l) hist[l] += nlev[l];
     }
+    double gd[2] = {gd3[0], gd3[1]};
     grid_sum_values<2>(gd, a.mbox, a.gs, epoch, lds);
     const double gamma = gd[0], delta = gd[1];
     rr = gamma;
@@ -406,11 +420,293 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
 }
 
 
-const void *strip_cg_kernel(int strips, bool mixed) {
-  if (strips <= 1) return mixed ? (const void *)k_cg_strip<1, true> : (const void *)k_cg_strip<1, false>;
-  if (strips <= 2) return mixed ? (const void *)k_cg_strip<2, true> : (const void *)k_cg_strip<2, false>;
-  if (strips <= 4) return mixed ? (const void *)k_cg_strip<4, true> : (const void *)k_cg_strip<4, false>;
-  return mixed ? (const void *)k_cg_strip<8, true> : (const void *)k_cg_strip<8, false>;
+// BiCGSTAB (van der Vorst) over row strips, with the scalars, exits, restarts
+// and refreshes of k_bicgstab.  Gathered, and so in memory: p and s.  Of the
+// wave's rows, x, r^, v and r (s between the two products) are in registers,
+// p's own entries in rl from its product on, and t = A s in wl.  Each round is
+// one product: of x (kRes), p or s.  A mixed solve that breaks down or
+// stagnates ends, and the host starts an FP64 one from its x.
+//
+// Measured on MI355X, convection-diffusion 100^3, us per iteration: FP64 37.2,
+// error bound 39.3 (tiles with the vectors in memory: 67.8 and 59.7): two
+// products of about 8 us, three sums and two barriers of 15 us together.
+constexpr int kStripRestarts = 8;
+
+template <int KS, bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_bicgstab_strip(StripSolveArgs a) {
+  using VT = typename std::conditional<MIXED, float, double>::type;
+  enum Round { kRes, kP, kS };
+  __shared__ double lds[kMaxGridSum * kWavesPerBlock];
+  __shared__ double lw[kWavesPerBlock][KS * 64];
+  __shared__ double lr[kWavesPerBlock][KS * 64];
+  const int wid = solver_wave();
+  double *wl = lw[threadIdx.x >> 6], *rl = lr[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
+  StripWave W;
+  int t0, t1;
+  wave_share<MIXED>(a, wid, lane, W, t0, t1);
+  auto row_of = [&](int k) { return wave_row(a, W, k); };
+  VT *const gp = MIXED ? (VT *)a.p32 : (VT *)a.p, *const gs_ = MIXED ? (VT *)a.r32 : (VT *)a.r;
+  unsigned epoch = 0, tag = 0;
+  int slot = 0, lds_i = 0;
+  VT rs[KS], rh[KS], v[KS];
+  double x[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    rs[k] = rh[k] = v[k] = VT(0);
+    x[k] = 0.0;
+    if (k < W.n) {
+      const int row = row_of(k);
+      if (row >= 0) x[k] = a.x[row];
+    }
+  }
+  const bool learned = MIXED && a.mlp != nullptr;
+  double rho = 0.0, rr = 0.0, rho_new = 0.0, rr_new = 0.0, bb = 0.0, stop2 = 0.0, rr_ref = 0.0, pp_last = 0.0;
+  double alpha = 0.0, omega = 0.0;
+  int it = 0, it_ref = 0, refresh = -1, restarts = 0, status = 0;
+  bool fresh = true;     // this residual starts r, r^ and p anew
+  bool infer = learned, full64 = false, fell = false, end = false;
+  unsigned nlev[5] = {0, 0, 0, 0, 0};
+  unsigned long long hist[5] = {0, 0, 0, 0, 0};
+  if (MIXED && !learned) count_levels(a.A.prec, t0, t1, lane, nlev);
+  // x to memory and a grid barrier, before a residual
+  auto sync_x = [&] {
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      if (k < W.n) {
+        const int row = row_of(k);
+        if (row >= 0) wt(a.x + row, x[k]);
+      }
+    grid_arrive<false>(a.gs, epoch);
+    grid_wait(a.gs, epoch);
+  };
+
+  Round round = kRes;
+  for (;;) {
+    double gd[3];
+    ++tag;
+    if (MIXED && round != kRes) {
+      if (round == kP && infer) {
+        infer_levels(a.A.tile_col, infer_ctx(a, pp_last, rr, bb), t0, t1, lane);
+        count_levels(a.prec_rw, t0, t1, lane, nlev);
+        full64 = nlev[0] > 0;
+        infer = false;
+      }
+      strip_product(a, W, (const float *)(round == kP ? gp : gs_), tag, !full64, round == kP, wl, rl, gd);
+    } else {
+      const double *u = round == kRes ? a.x : (const double *)(round == kP ? gp : gs_);
+      strip_product(a, W, u, tag, false, round == kP, wl, rl, gd);
+    }
+    bool step = false;  // go on to p = r + beta (p - omega v)
+    bool restart = false;
+    if (round == kRes) {
+      double tr[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < W.n) {
+          const int row = row_of(k);
+          if (row >= 0) {
+            const double bv = a.b[row];
+            double rv = bv - wl[64 * k + lane];
+            if (!end) {
+              rs[k] = (VT)rv;
+              rv = (double)rs[k];
+              if (fresh) {
+                rh[k] = rs[k];
+                wt(gp + row, rs[k]);
+              }
+            }
+            tr[0] += rv * rv;
+            tr[1] += rv * (double)rh[k];
+            tr[2] += bv * bv;
+            if (MIXED && learned && refresh < 0) {
+              // segment norms of p = r0 for the first inference
+              const double d2 = sum16(rv * rv);
+              if ((lane & 15) == 0) wt(a.seg2 + (row >> 4), (float)d2);
+            }
+          }
+        }
+      grid_sum<3>(tr, a.partials, a.gs, epoch, slot, lds, &lds_i);
+      if (end) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          a.stats[kStIters] = it;
+          a.stats[kStRefresh] = refresh;
+          a.stats[kStFallback] = fell;
+          a.stats[kStRecursive] = rr;
+          a.stats[kStTrue] = tr[0];
+          a.stats[kStBB] = bb;
+          a.stats[kStStatus] = status;
+        }
+        break;
+      }
+      ++refresh;
+      it_ref = it;
+      if (fresh) {
+        if (refresh == 0) {
+          bb = tr[2];
+          stop2 = uniform_double(a.tol2 * bb);
+          pp_last = tr[0];
+        }
+        rr = rho = rr_ref = tr[0];
+        fresh = false;
+        if (bb == 0.0 || ((a.fixed_iters <= 0 || refresh > 0) && rr <= stop2)) {
+          end = true;
+          continue;
+        }
+        ++it;
+        round = kP;
+        continue;
+      }
+      if (tr[0] <= stop2) {
+        rr = tr[0];
+        end = true;
+        continue;
+      }
+      if (MIXED && it < a.maxiter && (tr[0] > 0.25 * rr_ref || refresh > a.max_refresh)) {
+        rr = tr[0];
+        fell = end = true;
+        continue;
+      }
+      // A recursive residual far below the true one makes beta meaningless.
+      restart = tr[0] > 4.0 * rr_new;
+      rr_new = rr_ref = tr[0];
+      rho_new = tr[1];
+      step = true;
+    } else if (round == kP) {
+      // v = A p, alpha = rho / (v . r^), s = r - alpha v
+      double vr[1] = {0.0};
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < W.n) {
+          const double vv = wl[64 * k + lane];
+          vr[0] += vv * (double)rh[k];
+          v[k] = (VT)vv;
+        }
+      if (MIXED) {
+#pragma unroll
+        for (int l = 0; l < 5; ++l) hist[l] += 2 * nlev[l];
+      }
+      grid_sum_values<1>(vr, a.mbox, a.gs, epoch, lds);
+      if (!(vr[0] != 0.0) || !isfinite(vr[0])) {
+        if (MIXED) fell = end = true;
+        restart = true;
+      } else {
+        alpha = uniform_double(rho / vr[0]);
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+          if (k < W.n) {
+            const int row = row_of(k);
+            rs[k] = (VT)((double)rs[k] - alpha * (double)v[k]);
+            if (row >= 0) wt(gs_ + row, rs[k]);
+          }
+        grid_arrive<false>(a.gs, epoch);
+        grid_wait(a.gs, epoch);
+        round = kS;
+        continue;
+      }
+    } else {
+      // t = A s, omega = t.s / t.t, x += alpha p + omega s, r = s - omega t
+      double tw[2] = {gd[1], gd[2]};
+      grid_sum_values<2>(tw, a.mbox, a.gs, epoch, lds);
+      omega = uniform_double(tw[1] != 0.0 && isfinite(tw[1]) ? tw[0] / tw[1] : 0.0);
+      double nw[2] = {0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < W.n) {
+          const double sv = (double)rs[k];
+          x[k] += alpha * rl[64 * k + lane] + omega * sv;
+          rs[k] = (VT)(sv - omega * wl[64 * k + lane]);
+          nw[0] += (double)rs[k] * (double)rh[k];
+          nw[1] += (double)rs[k] * (double)rs[k];
+        }
+      grid_sum_values<2>(nw, a.mbox, a.gs, epoch, lds);
+      rho_new = nw[0];
+      rr_new = nw[1];
+      if (a.fixed_iters > 0) {
+        if (it >= a.fixed_iters) {
+          rr = rr_new;
+          end = true;
+        } else {
+          step = true;
+        }
+      } else if (rr_new <= stop2 || omega == 0.0 || !isfinite(rr_new) ||
+                 (MIXED && (rr_new <= a.ratio2 * rr_ref || it - it_ref >= a.refresh_every))) {
+        // the FP64 residual first (p, v and the scalars of this step are kept)
+        round = kRes;
+        sync_x();
+        continue;
+      } else {
+        step = true;
+      }
+    }
+    if (step && !restart && a.fixed_iters <= 0) {
+      if (it >= a.maxiter) {
+        rr = rr_new;
+        status = MF_NOT_CONVERGED;
+        end = true;
+      } else if (omega == 0.0 || rho == 0.0 || rho_new == 0.0 || !isfinite(rho_new)) {
+        restart = true;
+      }
+    } else if (step && restart && it >= a.maxiter) {
+      rr = rr_new;
+      status = MF_NOT_CONVERGED;
+      end = true;
+    }
+    if (restart && !end && ++restarts > kStripRestarts) {
+      status = MF_ERR_BREAKDOWN;
+      end = true;
+    }
+    if (restart || end) {
+      round = kRes;
+      fresh = true;
+      sync_x();
+      continue;
+    }
+    const double beta = uniform_double((rho_new / rho) * (alpha / omega));
+    rho = rho_new;
+    rr = rr_new;
+    const bool lupd = learned && (it % a.check_interval) == 0;
+    double pp[1] = {0.0};
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      if (k < W.n) {
+        const int row = row_of(k);
+        const VT pv = (VT)((double)rs[k] + beta * (rl[64 * k + lane] - omega * (double)v[k]));
+        if (row >= 0) wt(gp + row, pv);
+        if (MIXED && lupd) {
+          const double d = row >= 0 ? (double)pv * (double)pv : 0.0, d2 = sum16(d);
+          pp[0] += d;
+          if ((lane & 15) == 0 && row >= 0) wt(a.seg2 + (row >> 4), (float)d2);
+        }
+      }
+    if (lupd) {
+      grid_sum<1>(pp, a.partials, a.gs, epoch, slot, lds, &lds_i);
+      pp_last = pp[0];
+      infer = true;
+    } else {
+      grid_arrive<false>(a.gs, epoch);
+      grid_wait(a.gs, epoch);
+    }
+    ++it;
+    round = kP;
+  }
+  if (MIXED) {
+#pragma unroll
+    for (int l = 0; l < 5; ++l) add_hist(hist[l], a.hist + l, lane);
+  }
+}
+
+template <int KS>
+static const void *strip_kernel(bool bicg, bool mixed) {
+  if (bicg) return mixed ? (const void *)k_bicgstab_strip<KS, true> : (const void *)k_bicgstab_strip<KS, false>;
+  return mixed ? (const void *)k_cg_strip<KS, true> : (const void *)k_cg_strip<KS, false>;
+}
+
+const void *strip_solve_kernel(int strips, bool bicg, bool mixed) {
+  if (strips <= 1) return strip_kernel<1>(bicg, mixed);
+  if (strips <= 2) return strip_kernel<2>(bicg, mixed);
+  if (strips <= 4) return strip_kernel<4>(bicg, mixed);
+  return strip_kernel<8>(bicg, mixed);
 }
 
 }  // namespace mf

@@ -224,13 +224,14 @@ __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc 
   return strip_full_sum<false>(S.vv + o, S.vc + o, np, lane, x, acc);
 }
 
+// Descriptor i (wave-uniform), by a scalar load: descriptors do not change
+// while kernels run, which the constant address space tells the compiler.
 __device__ __forceinline__ StripDesc strip_desc(const StripView &S, int i) {
-  const int4 q = *reinterpret_cast<const int4 *>(S.desc + i);
-  int4 u;
-  u.x = __builtin_amdgcn_readfirstlane(q.x);
-  u.y = __builtin_amdgcn_readfirstlane(q.y);
-  u.z = __builtin_amdgcn_readfirstlane(q.z);
-  u.w = __builtin_amdgcn_readfirstlane(q.w);
+  typedef const __attribute__((address_space(4))) uint32_t *ConstPtr;
+  const ConstPtr q = (ConstPtr)(uintptr_t)(S.desc + i);
+  struct Raw { uint32_t w[4]; } u;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) u.w[k] = q[k];
   return __builtin_bit_cast(StripDesc, u);
 }
 

@@ -1,5 +1,6 @@
 // mf_batch.hip -- many independent systems, each with several right-hand
-// sides, solved by CG in one persistent launch captured in a hipGraph.
+// sides, solved by CG in one persistent launch captured in a hipGraph: the
+// host side, and the kernel over tiles.
 //
 // A work item is one (system, right-hand side) pair.  The systems are split
 // over 8 queues, one per XCD (blocks are dispatched round-robin, block b on
@@ -9,17 +10,18 @@
 // item of its XCD's queue, solves it with its waves and takes another; when
 // that queue is empty it takes items from the other queues in turn.  So the
 // blocks solving one system's right-hand sides run at the same time on one
-// XCD and read the system's tiles through that XCD's L2.
+// XCD and read the system's matrix through that XCD's L2.  There is no grid
+// barrier, so blocks need not be co-resident and the launch is an ordinary
+// one.
 //
-// Inside a block the solve is the single-system memory-form CG: the 8 waves
-// own nnz-balanced tile-row ranges of the system, the SpMV is the streamed
-// wave SpMV, dot products are deterministic block sums and every phase ends
-// at a block barrier; there is no grid barrier, so blocks need not be
-// co-resident and the launch is an ordinary one.  Precision follows the
-// handle's current tile levels (FP64, or the FIXED / ERRBOUND levels set
-// before the launch) with FP64 scalars, FP64 x, FP32 work vectors under mixed
-// levels, periodic FP64 true-residual recomputation and FP64 fallback on
-// stagnation.
+// FP64 and error-bound batches of handles with row strips run k_batch_strip
+// (mf_batch_strip.hip).  k_batch_cg, for the caller's own per-tile levels and
+// for handles without strips: an item's 8 waves own nnz-balanced tile-row
+// ranges of the system, the SpMV is the streamed wave SpMV, dot products are
+// deterministic block sums and every phase ends at a block barrier.
+// Precision follows the handle's current tile levels with FP64 scalars, FP64
+// x, FP32 work vectors under mixed levels, periodic FP64 true-residual
+// recomputation and FP64 fallback on stagnation.
 //
 // Timing: each item records the realtime clock (100 MHz) at start and end;
 // a system's time is its last end minus its first start.
@@ -29,44 +31,15 @@
 #include <numeric>
 #include <vector>
 
-#include "mf_device.h"
+#include "mf_batch.h"
 
 namespace mf {
 
-// Waves per (system, right-hand side) item: 4, 8 (default) or 16, picked by
-// opts->batch_waves or by mf_tune_batch.
+// Tiles run best at 8 waves an item, strips at 16: the item's vectors then fit
+// on chip up to 16,384 rows (errbound, 48 kNN systems of 1,000 to 16,000 rows x
+// 8 right-hand sides: 4 waves 42.7 ms, 8 waves 24.5, 16 waves 12.0).
 constexpr int kBatchWavesDefault = 8;
-
-struct BatchSys {
-  TileView A;
-  const int *wave_tr;  // waves per item + 1 tile-row bounds
-  const double *b;     // npad * nrhs, right-hand side j at j * npad
-  double *x;           // npad * nrhs
-  int npad;
-  int mixed;           // 1: per-tile levels (A.prec), 0: every tile FP64
-};
-
-struct BatchArgs {
-  const BatchSys *sys;
-  const int2 *items;  // (system, right-hand side), queue by queue
-  const int *qoff;    // kQueues + 1: items of queue q at [qoff[q], qoff[q+1])
-  int nitems;
-  int *head;          // kQueues work-queue heads
-  double *work;       // per block: r, p, q (npad_max doubles each), p32
-  long long stride;   // doubles per block
-  int *iters;
-  double *relres;
-  unsigned long long *tstamp;  // per item: start, end
-  double tol2;
-  int maxiter;
-  double ratio2;
-  int max_refresh;
-  int refresh_every;
-};
-
-constexpr int kQueues = 8;  // one per XCD
-
-__device__ __forceinline__ unsigned long long realtime() { return __builtin_amdgcn_s_memrealtime(); }
+constexpr int kStripWavesDefault = 16;
 
 __global__ void k_batch_reset(int *head, int nitems, int *iters, double *relres) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -89,21 +62,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch_cg(BatchArgs a) {
   PrecCount cnt;
   int q = blockIdx.x % kQueues, tried = 0;  // this XCD's queue first
   for (;;) {
-    if (threadIdx.x == 0) {
-      // next item of queue q; an empty queue passes to the next one, and
-      // after all kQueues are empty the block ends (every head only grows)
-      int it = -1;
-      while (tried < kQueues) {
-        const int k = atomicAdd(&a.head[q], 1);
-        if (a.qoff[q] + k < a.qoff[q + 1]) {
-          it = a.qoff[q] + k;
-          break;
-        }
-        q = (q + 1) % kQueues;
-        ++tried;
-      }
-      item_s = it;
-    }
+    if (threadIdx.x == 0) item_s = next_item(a, q, tried);
     __syncthreads();
     // item, system and wave range are wave-uniform: scalar registers
     const int item = __builtin_amdgcn_readfirstlane(item_s);
@@ -347,12 +306,16 @@ extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, c
 
   // per-system levels, schedules and descriptors
   std::vector<BatchSys> hs(nsys);
-  const int nwv = opt.batch_waves == 0 ? kBatchWavesDefault : opt.batch_waves;
+  // Strips where every system has them, except at the caller's own levels
+  // (FIXED), which are per tile.
+  bool strips = opt.policy != MF_POLICY_FIXED;
+  for (int i = 0; i < nsys; ++i) strips = strips && systems[i]->strips.nstrips > 0;
+  const int nwv = opt.batch_waves == 0 ? (strips ? kStripWavesDefault : kBatchWavesDefault) : opt.batch_waves;
   if (nwv != 4 && nwv != 8 && nwv != 16)
     return fail(MF_ERR_ARG, "mf_batch_cg_solve: batch_waves must be 0, 4, 8 or 16");
   const int block = 64 * nwv;
   std::vector<int> htr((size_t)nsys * (nwv + 1));
-  int npad_max = 16;
+  int npad_max = 16, pieces_max = 0;
   for (int i = 0; i < nsys; ++i) {
     mf_tiled *t = systems[i];
     if (opt.policy == MF_POLICY_FIXED)
@@ -361,6 +324,7 @@ extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, c
     const std::vector<int> w = balance_tilerows(t, nwv);
     std::copy(w.begin(), w.end(), htr.begin() + (size_t)i * (nwv + 1));
     npad_max = std::max(npad_max, t->dev.npad);
+    pieces_max = std::max(pieces_max, t->strips.npieces);
   }
   int *d_tr = nullptr;
   MF_TRY(dalloc((void **)&d_tr, sizeof(int) * htr.size()));
@@ -369,6 +333,7 @@ extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, c
     for (int i = 0; i < nsys; ++i) MF_TRY(wave_uniform_levels(systems[i], d_tr + (size_t)i * (nwv + 1), nwv, st));
   for (int i = 0; i < nsys; ++i) {
     hs[i].A = view_of(systems[i]);
+    hs[i].S = strip_view_of(systems[i]);
     hs[i].wave_tr = d_tr + (size_t)i * (nwv + 1);
     hs[i].b = d_b[i];
     hs[i].x = d_x[i];
@@ -400,14 +365,15 @@ extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, c
 
   int ncu = 0, nb = 0;
   MF_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  const void *kern = nwv == 4 ? (const void *)k_batch_cg<256>
+  const void *kern = strips ? batch_strip_kernel(nwv, opt.policy != MF_POLICY_FP64)
+                   : nwv == 4 ? (const void *)k_batch_cg<256>
                    : nwv == 8 ? (const void *)k_batch_cg<512> : (const void *)k_batch_cg<1024>;
   MF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, block, 0));
   if (nb < 1) nb = 1;
   int G = std::min(nitems, ncu * nb);
   if (opt.blocks > 0) G = std::min(G, opt.blocks);
   // p32 needs npad_max floats: round the per-block stride up to whole doubles
-  const long long stride = 3LL * npad_max + (npad_max + 1) / 2 + 32;
+  const long long stride = 3LL * npad_max + std::max((npad_max + 1) / 2, pieces_max) + 32;
 
   BatchSys *d_sys = nullptr;
   int2 *d_items = nullptr;
@@ -435,6 +401,7 @@ extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, c
   args.head = d_head;
   args.work = d_work;
   args.stride = stride;
+  args.npad_max = npad_max;
   args.iters = d_iters;
   args.relres = d_rel;
   args.tstamp = d_ts;
@@ -447,12 +414,12 @@ extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, c
   // capture: queue reset (a kernel, not a memset node) + the persistent solve
   MF_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   k_batch_reset<<<(std::max(nitems, kQueues) + 255) / 256, 256, 0, st>>>(d_head, nitems, d_iters, d_rel);
-  if (nwv == 4) k_batch_cg<256><<<G, 256, 0, st>>>(args);
-  else if (nwv == 8) k_batch_cg<512><<<G, 512, 0, st>>>(args);
-  else k_batch_cg<1024><<<G, 1024, 0, st>>>(args);
+  void *kargs[] = {&args};
+  const hipError_t le = hipLaunchKernel(kern, dim3(G), dim3(block), kargs, 0, st);
   hipGraph_t g = nullptr;
   const hipError_t ce = hipStreamEndCapture(st, &g);
   own_res.g = g;
+  if (le != hipSuccess) return fail(MF_ERR_HIP, std::string("mf_batch_cg_solve: ") + hipGetErrorString(le));
   if (ce != hipSuccess) return fail(MF_ERR_HIP, std::string("mf_batch_cg_solve capture: ") + hipGetErrorString(ce));
   MF_HIP(hipGraphInstantiate(&own_res.ge, g, nullptr, nullptr, 0));
   MF_HIP(hipEventCreate(&own_res.e0));

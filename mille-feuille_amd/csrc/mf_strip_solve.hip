@@ -76,28 +76,20 @@ __device__ __forceinline__ void strip_product(const StripSolveArgs &a, const Str
     const int q1 = __builtin_amdgcn_readfirstlane(a.wave_piece[wid + 1]);
     for (int q = __builtin_amdgcn_readfirstlane(a.wave_piece[wid]); q < q1; ++q) {
       const int pc = __builtin_amdgcn_readfirstlane(a.piece_order[q]);
-      const double v[1] = {wave_sum(strip_sum(S, strip_desc(S, S.nstrips + pc), x, w.lane, 0.0, v32))};
+      const double v[1] = {piece_sum(S, pc, w.lane, MemVec<XT>{x}, v32)};
       if (w.lane == 0) mbox_post<1>(a.pmail + 2 * (size_t)pc, tag, v);
     }
   }
-#pragma unroll 1
-  for (int k = 0; k < w.n; ++k) {
-    const int s = w.s0 + k;
-    const StripDesc d = strip_desc(S, s);
-    bool lng;
-    const int row = strip_row(S, s, w.lane, lng);
-    const double own = row >= 0 ? (double)x[row] : 0.0;
-    double acc = 0.0;
-    if ((d.flags & kStripLead) && row >= 0)
-      acc = (v32 ? (double)S.lead32[64 * s + w.lane] : S.lead64[64 * s + w.lane]) * own;
-    acc = strip_sum(S, d, x, w.lane, acc, v32);
-    if ((d.flags & kStripLong) && lng) acc += take_pieces(a, S.lane_long[64 * s + w.lane], tag);
-    wl[64 * k + w.lane] = acc;
-    if (own_out) rl[64 * k + w.lane] = own;
-    g[0] += own * own;
-    g[1] += acc * own;
-    g[2] += acc * acc;
-  }
+  strips_run(S, w.lane, MemVec<XT>{x}, v32, w.n, [&](int k) { return w.s0 + k; },
+             [&](int s, const StripDesc &d, int, bool lng, double acc, double own) {
+               if ((d.flags & kStripLong) && lng) acc += take_pieces(a, S.lane_long[64 * s + w.lane], tag);
+               const int o = 64 * (s - w.s0) + w.lane;
+               wl[o] = acc;
+               if (own_out) rl[o] = own;
+               g[0] += own * own;
+               g[1] += acc * own;
+               g[2] += acc * acc;
+             });
 }
 
 // Tiles [t0, t1) counted per level (wave-uniform).

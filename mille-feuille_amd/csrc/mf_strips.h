@@ -68,6 +68,25 @@ __device__ __forceinline__ int strip_row(const StripView &S, int s, int lane, bo
   return r & (kLongBit - 1);
 }
 
+// The vector that a strip multiplies: in memory, or in the block's LDS.
+// rebase(d).get(i) is entry i + d.
+template <typename T>
+struct MemVec {
+  typedef T value;
+  const T *p;
+  __device__ __forceinline__ MemVec rebase(ptrdiff_t d) const { return MemVec{p + d}; }
+  __device__ __forceinline__ T get(uint32_t i) const { return ld_at<T>(p, i * (uint32_t)sizeof(T)); }
+};
+
+template <typename T>
+struct LdsVec {
+  typedef T value;
+  const T *p;
+  int off = 0;
+  __device__ __forceinline__ LdsVec rebase(ptrdiff_t d) const { return LdsVec{p, off + (int)d}; }
+  __device__ __forceinline__ T get(uint32_t i) const { return p[(int)i + off]; }
+};
+
 // The lane's N word pairs at byte offset vo of the strip's words.
 template <int N>
 __device__ __forceinline__ void strip_load_words(const uint32_t *__restrict__ w, uint32_t vo, uint2 (&r)[N]) {
@@ -75,16 +94,16 @@ __device__ __forceinline__ void strip_load_words(const uint32_t *__restrict__ w,
   for (int i = 0; i < N; ++i) r[i] = ld_at<uint2>(w, vo + 512u * i);
 }
 
-// Adds the products of N loaded word pairs to acc.  xb points 2^23 entries
+// Adds the products of N loaded word pairs to acc.  xb starts 2^23 entries
 // before the strip's base row (an address only: the packed column field is
 // biased by 2^23).
-template <int N, typename XT>
-__device__ __forceinline__ double strip_packed(const uint2 (&w)[N], const XT *xb, float sc, double acc) {
-  XT g[2 * N];
+template <int N, class X>
+__device__ __forceinline__ double strip_packed(const uint2 (&w)[N], const X &xb, float sc, double acc) {
+  typename X::value g[2 * N];
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    g[2 * i] = ld_at<XT>(xb, (w[i].x >> 8) * (uint32_t)sizeof(XT));
-    g[2 * i + 1] = ld_at<XT>(xb, (w[i].y >> 8) * (uint32_t)sizeof(XT));
+    g[2 * i] = xb.get(w[i].x >> 8);
+    g[2 * i + 1] = xb.get(w[i].y >> 8);
   }
 #pragma unroll
   for (int i = 0; i < 2 * N; ++i) {
@@ -97,9 +116,9 @@ __device__ __forceinline__ double strip_packed(const uint2 (&w)[N], const XT *xb
 }
 
 // The last pairs of a packed strip: four loaded ones and the np - k (< 4) after them.
-template <typename XT>
+template <class X>
 __device__ __forceinline__ double strip_packed_rest(const uint32_t *__restrict__ w, uint32_t vo, int k, int np,
-                                                    const uint2 (&a)[4], const XT *xb, float sc, double acc) {
+                                                    const uint2 (&a)[4], const X &xb, float sc, double acc) {
   if (np - k >= 2) {
     uint2 c[2];
     strip_load_words(w, vo + 512u * k, c);
@@ -118,13 +137,13 @@ __device__ __forceinline__ double strip_packed_rest(const uint32_t *__restrict__
 }
 
 // N value / column pairs of a full or near strip from the lane's entry e;
-// VT double or float.  Near columns: xb points 2^15 entries before the base.
-template <bool NEAR, int N, typename VT, typename XT>
+// VT double or float.  Near columns: xb starts 2^15 entries before the base.
+template <bool NEAR, int N, typename VT, class X>
 __device__ __forceinline__ double strip_full(const VT *__restrict__ v, const void *__restrict__ c, uint32_t e,
-                                             const XT *xb, double acc) {
+                                             const X &xb, double acc) {
   VT a[2 * N];
   uint32_t j[2 * N];
-  XT g[2 * N];
+  typename X::value g[2 * N];
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     struct alignas(2 * sizeof(VT)) Pair { VT x, y; };
@@ -145,15 +164,15 @@ __device__ __forceinline__ double strip_full(const VT *__restrict__ v, const voi
   auto pad = [](uint32_t q) { return NEAR ? q == 0u : (int)q < 0; };
 #pragma unroll
   for (int i = 0; i < 2 * N; ++i)
-    g[i] = ld_at<XT>(xb, (pad(j[i]) ? (NEAR ? 1u << 15 : 0u) : j[i]) * (uint32_t)sizeof(XT));
+    g[i] = xb.get(pad(j[i]) ? (NEAR ? 1u << 15 : 0u) : j[i]);
 #pragma unroll
   for (int i = 0; i < 2 * N; ++i) acc = __builtin_fma((double)a[i], pad(j[i]) ? 0.0 : (double)g[i], acc);
   return acc;
 }
 
-template <bool NEAR, typename VT, typename XT>
+template <bool NEAR, typename VT, class X>
 __device__ __forceinline__ double strip_full_sum(const VT *__restrict__ v, const void *__restrict__ c, int np,
-                                                 int lane, const XT *xb, double acc) {
+                                                 int lane, const X &xb, double acc) {
   const uint32_t e = 2u * lane;
   int k = 0;
   for (; k + 4 <= np; k += 4) acc = strip_full<NEAR, 4>(v, c, e + 128u * k, xb, acc);
@@ -165,16 +184,17 @@ __device__ __forceinline__ double strip_full_sum(const VT *__restrict__ v, const
 }
 
 // Sum of the lane's entries of a strip or piece (without the lead), added to
-// acc.  XT double or float: the vector; v32 (float vectors only): full and
+// acc.  X: the vector (MemVec or LdsVec); v32 (FP32 vectors only): full and
 // near strips multiply the FP32 payload.  Strips of more than four pairs load
-// the next four word pairs before the gathers of the current ones.
-template <typename XT>
-__device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc &d, const XT *__restrict__ x,
-                                            int lane, double acc, bool v32 = false) {
+// the next four word pairs before the gathers of the current ones (two
+// buffers in turn: a copy of words in flight would wait for them).
+template <class X>
+__device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc &d, const X &x, int lane,
+                                            double acc, bool v32 = false) {
   const int np = d.npair;
   if (d.cls == kStripPacked) {
     const uint32_t *w = S.words + (size_t)d.off * 128;
-    const XT *xb = x + ((ptrdiff_t)d.base - (1 << 23));
+    const X xb = x.rebase((ptrdiff_t)d.base - (1 << 23));
     const uint32_t vo = 8u * lane;
     if (np <= 4) {
       if (np == 1) {
@@ -199,7 +219,6 @@ __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc 
       }
       return acc;
     }
-    // (two buffers in turn: a copy of words in flight would wait for them)
     uint2 a[4], b[4];
     strip_load_words(w, vo, a);
     int k = 4;
@@ -215,8 +234,8 @@ __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc 
     }
   }
   const size_t o = (size_t)d.off * 128;
-  const XT *xn = x + ((ptrdiff_t)d.base - (1 << 15));
-  if (std::is_same<XT, float>::value && v32) {
+  const X xn = x.rebase((ptrdiff_t)d.base - (1 << 15));
+  if (std::is_same<typename X::value, float>::value && v32) {
     if (d.cls == kStripNear) return strip_full_sum<true>(S.vf + o, S.vh + o, np, lane, xn, acc);
     return strip_full_sum<false>(S.vf + o, S.vc + o, np, lane, x, acc);
   }
@@ -224,15 +243,49 @@ __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc 
   return strip_full_sum<false>(S.vv + o, S.vc + o, np, lane, x, acc);
 }
 
-// Descriptor i (wave-uniform), by a scalar load: descriptors do not change
-// while kernels run, which the constant address space tells the compiler.
-__device__ __forceinline__ StripDesc strip_desc(const StripView &S, int i) {
+// *p for a wave-uniform p by scalar loads: data that does not change while
+// kernels run, which the constant address space tells the compiler.
+template <typename T>
+__device__ __forceinline__ T load_uniform(const T *p) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
   typedef const __attribute__((address_space(4))) uint32_t *ConstPtr;
-  const ConstPtr q = (ConstPtr)(uintptr_t)(S.desc + i);
-  struct Raw { uint32_t w[4]; } u;
+  const ConstPtr q = (ConstPtr)(uintptr_t)p;
+  struct Raw { uint32_t w[sizeof(T) / 4]; } u;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) u.w[k] = q[k];
-  return __builtin_bit_cast(StripDesc, u);
+  for (int k = 0; k < (int)(sizeof(T) / 4); ++k) u.w[k] = q[k];
+  return __builtin_bit_cast(T, u);
+}
+
+// Descriptor i (wave-uniform).
+__device__ __forceinline__ StripDesc strip_desc(const StripView &S, int i) { return load_uniform(S.desc + i); }
+
+// Strips idx(0) .. idx(n - 1): f(strip, descriptor, row, long, sum with the
+// lead, own entry of x); row -1: the lane has none; long: the row's other
+// entries are in pieces.  (Loading the next strip's words and lead before the
+// gathers of the current one was slower: with four word pairs a strip always
+// loaded, 128^3 SpMV 17.4 -> 18.9 us, FP64 CG 28.9 -> 34.9 us an iteration.  The
+// waves of a CU hide the two trips; the loads themselves are what counts.)
+template <class X, class Idx, class F>
+__device__ __forceinline__ void strips_run(const StripView &S, int lane, const X &x, bool v32, int n, Idx idx, F f) {
+#pragma unroll 1
+  for (int k = 0; k < n; ++k) {
+    const int s = idx(k);
+    const StripDesc d = strip_desc(S, s);
+    bool lng;
+    const int row = strip_row(S, s, lane, lng);
+    const double own = row >= 0 ? (double)x.get((uint32_t)row) : 0.0;
+    double acc = 0.0;
+    if ((d.flags & kStripLead) && row >= 0)
+      acc = (v32 ? (double)S.lead32[64 * s + lane] : S.lead64[64 * s + lane]) * own;
+    acc = strip_sum(S, d, x, lane, acc, v32);
+    f(s, d, row, lng, acc, own);
+  }
+}
+
+// Sum over the wave of a piece's products.
+template <class X>
+__device__ __forceinline__ double piece_sum(const StripView &S, int piece, int lane, const X &x, bool v32) {
+  return wave_sum(strip_sum(S, strip_desc(S, S.nstrips + piece), x, lane, 0.0, v32));
 }
 
 }  // namespace mf

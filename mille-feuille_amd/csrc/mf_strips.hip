@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256, 8) void k_spmv_strip(StripView S, int pblocks,
       for (int k0 = 0; k0 < lr.n; k0 += 4) {
         double v = 0.0;
         if (k0 + wv < lr.n)
-          v = wave_sum(strip_sum(S, strip_desc(S, S.nstrips + lr.first + k0 + wv), x, lane, 0.0));
+          v = piece_sum(S, lr.first + k0 + wv, lane, MemVec<double>{x}, false);
         __syncthreads();
         if (lane == 0) part[wv] = v;
         __syncthreads();
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256, 8) void k_spmv_strip(StripView S, int pblocks,
       const int h = S.nmulti + (b - S.nmulti) * 4 + wv;
       if (h >= S.nlong) return;
       const LongRow lr = S.lrow[h];
-      const double v = wave_sum(strip_sum(S, strip_desc(S, S.nstrips + lr.first), x, lane, 0.0));
+      const double v = piece_sum(S, lr.first, lane, MemVec<double>{x}, false);
       if (lane == 0) store_long(S, lr, v, x, y);
     }
     return;
@@ -199,13 +199,10 @@ __global__ __launch_bounds__(256, 8) void k_spmv_strip(StripView S, int pblocks,
   const int per_xcd = (gridDim.x - (PIECES ? pblocks : 0)) >> 3;  // both counts are multiples of 8
   const int s = ((b & 7) * per_xcd + (b >> 3)) * 4 + wv;
   if (s >= S.nstrips) return;
-  const StripDesc d = strip_desc(S, s);
-  bool lng;
-  const int row = strip_row(S, s, lane, lng);
-  double acc = 0.0;
-  if ((d.flags & kStripLead) && row >= 0) acc = S.lead64[64 * s + lane] * x[row];
-  acc = strip_sum(S, d, x, lane, acc);
-  if (row >= 0 && !lng) y[row] = acc;
+  strips_run(S, lane, MemVec<double>{x}, false, 1, [&](int) { return s; },
+             [&](int, const StripDesc &, int row, bool lng, double acc, double) {
+               if (row >= 0 && !lng) y[row] = acc;
+             });
 }
 
 template <typename T>

@@ -307,20 +307,27 @@ def batch_cg(systems, bs, nrhs=1, x0=None, allow_not_converged=False, tune_iters
     timings under "tune")."""
     opts = solve_opts(**kw)
     nsys = len(systems)
-    db, dx = [], []
-    for tm, b in zip(systems, bs):
-        b = np.asarray(b, np.float64).reshape(nrhs, -1)
-        hb = np.zeros((nrhs, tm.npad))
-        hb[:, : b.shape[1]] = b
-        db.append(DeviceArray.from_host(hb.ravel()))
-        hx = np.zeros((nrhs, tm.npad))
-        if x0 is not None:
-            x = np.asarray(x0[len(dx)], np.float64).reshape(nrhs, -1)
-            hx[:, : x.shape[1]] = x
-        dx.append(DeviceArray.from_host(hx.ravel()))
+    # one device array each for the right-hand sides and the solutions, the
+    # systems one after another (a pair of allocations and copies per system
+    # took 5 ms for 48 systems)
+    off = np.concatenate([[0], np.cumsum([tm.npad * nrhs for tm in systems])]).astype(np.int64)
+
+    def pack(vs):
+        h = np.zeros(int(off[-1]))
+        for k, tm in enumerate(systems):
+            v = np.asarray(vs[k], np.float64).reshape(nrhs, -1)
+            h[off[k]:off[k + 1]].reshape(nrhs, tm.npad)[:, : v.shape[1]] = v
+        return DeviceArray.from_host(h)
+
+    db = pack(bs)
+    if x0 is None:
+        dx = DeviceArray(int(off[-1]), np.float64)
+        dx.zero()
+    else:
+        dx = pack(x0)
     hs = (C.c_void_p * nsys)(*[tm.h.value for tm in systems])
-    pb = (C.c_void_p * nsys)(*[d.ptr for d in db])
-    px = (C.c_void_p * nsys)(*[d.ptr for d in dx])
+    pb = (C.c_void_p * nsys)(*[db.ptr + 8 * int(o) for o in off[:-1]])
+    px = (C.c_void_p * nsys)(*[dx.ptr + 8 * int(o) for o in off[:-1]])
     tune = None
     if tune_iters > 0 and not kw.get("batch_waves"):
         rep = _lib.MfTuneReport()
@@ -335,7 +342,8 @@ def batch_cg(systems, bs, nrhs=1, x0=None, allow_not_converged=False, tune_iters
     code = lib.mf_batch_cg_solve(hs, nsys, nrhs, pb, px, C.byref(opts), _p(its), _p(rel), _p(per),
                                  C.byref(tot))
     check("mf_batch_cg_solve", code, allow=(0, 1) if allow_not_converged else (0,))
-    xs = [d.get().reshape(nrhs, tm.npad)[:, : tm.rowA] for d, tm in zip(dx, systems)]
+    x = dx.get()
+    xs = [x[off[k]:off[k + 1]].reshape(nrhs, tm.npad)[:, : tm.rowA] for k, tm in enumerate(systems)]
     return xs, {"status": code, "iterations": its.reshape(nsys, nrhs),
                 "rel_residual": rel.reshape(nsys, nrhs), "per_system_ms": per,
                 "total_ms": tot.value, "batch_waves": opts.batch_waves or 8, "tune": tune}

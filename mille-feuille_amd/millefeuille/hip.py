@@ -68,7 +68,8 @@ class DeviceArray:
         a = np.ascontiguousarray(a, dtype=dtype)
         n = len(a) if length is None else int(length)
         d = cls(n, a.dtype)
-        d.zero()
+        if n > len(a):
+            d.zero()
         if len(a):
             _ok("hipMemcpy", _hip.hipMemcpy(d.ptr, a.ctypes.data, a.nbytes, H2D))
         return d

@@ -81,6 +81,7 @@ struct SolveArgs {
   double ratio2;              // refresh_ratio^2
   int max_refresh;
   int refresh_every;
+  int stop64;                 // end at a fallback to FP64 (the host goes on over strips)
   // learned policy (MODE kPerTile; mlp == nullptr otherwise)
   const MlpDevice *mlp;
   const uint16_t *feat16;
@@ -421,6 +422,7 @@ __global__ __launch_bounds__(kBlock) void k_cg(SolveArgs a) {
   int trace_it = -1;
   (void)trace_it;
   while (!done) {
+    if (mixed && force64 && a.stop64) break;
     double gamma = 0.0, delta = 0.0;
     if (!pending) {
       ++trace_it;
@@ -724,6 +726,7 @@ __global__ __launch_bounds__(kBlock) void k_bicgstab(SolveArgs a) {
   double pp_last = rr;   // ||p||^2 at the last inference point
 
   while (!done) {
+    if (mixed && force64 && a.stop64) break;
     if (restart) {
       if (++restarts > kMaxRestart) { status = MF_ERR_BREAKDOWN; break; }
       // leaving the FP32 vectors: the FP64 recurrence restarts from here
@@ -1486,11 +1489,25 @@ static mf_status ensure_strip_schedule(mf_tiled *t, int nwaves) {
 // Blocks of a persistent solve without an override: a small system gets about
 // 1024 rows per block (at least 4 blocks; whole multiples of 8 from 8 on, for
 // the XCD-contiguous block order), so the grid-wide sums and syncs span fewer
-// blocks (one strip per wave).  From about 256k rows on, the full grid.
+// blocks.  From about 256k rows on, the full grid.
 static int want_blocks(const mf_tiled *t, const mf_solve_opts &opt) {
   if (opt.blocks > 0) return opt.blocks;
   const int rows = t->tilem * 16;
   const int want = std::max(4, (rows + 1023) / 1024);
+  return want >= 8 ? (want + 7) / 8 * 8 : want;
+}
+
+// Blocks of a strip solve without an override.  A wave's second strip costs
+// less than the synchronisation over twice the blocks up to 128 of them (us per
+// FP64 CG iteration on MI355X, 7-point Laplacians): 32^3 16 blocks 8.0, 32 6.3,
+// 64 6.6; 64^3 64 blocks 11.8, 128 9.8, 256 10.3; 80^3 128 blocks 12.8, 256 12.0.
+// Pieces of long rows want more waves: power law, 50k rows 48 blocks 20.4, 96
+// 16.6, 256 18.6; 200k rows 128 blocks 36.9, 200 30.2, 256 29.4.
+static int want_strip_blocks(const mf_tiled *t, const mf_solve_opts &opt) {
+  if (opt.blocks > 0) return opt.blocks;
+  const int rows = t->tilem * 16;
+  int want = t->strips.npieces > 0 ? (rows + 511) / 512 : std::min((rows + 1023) / 1024, std::max(128, (rows + 2047) / 2048));
+  want = std::max(4, want);
   return want >= 8 ? (want + 7) / 8 * 8 : want;
 }
 
@@ -1522,14 +1539,17 @@ static mf_status strip_grid(const mf_tiled *t, const mf_solve_opts &opt, bool bi
   if (!L.lean || opt.form == MF_FORM_MEMORY || 2 * L.npieces > t->rowA) return MF_OK;
   if (pol != MF_POLICY_FP64 && pol != MF_POLICY_ERRBOUND && !(pol == MF_POLICY_LEARNED && !L.sorted)) return MF_OK;
   int g = 0;
-  MF_TRY(grid_for(strip_solve_kernel(kMaxWaveStrips, bicg, pol != MF_POLICY_FP64), want_blocks(t, opt), &g, kBlock, true));
+  MF_TRY(grid_for(strip_solve_kernel(kMaxWaveStrips, bicg, pol != MF_POLICY_FP64), want_strip_blocks(t, opt), &g,
+                  kBlock, true));
   const int per = (L.nstrips + g * kWavesPerBlock - 1) / (g * kWavesPerBlock);
   if (per <= kMaxWaveStrips) *G = g;
   return MF_OK;
 }
 
+// before: the report of a tile solve that ended at its fallback to FP64 (x is
+// where it left off, opt its options); null: a solve from the start.
 static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solve_opts opt, mf_report *rep,
-                            int G, bool bicg, bool noalloc) {
+                            int G, bool bicg, bool noalloc, const mf_report *before = nullptr) {
   hipStream_t st = (hipStream_t)opt.stream;
   const StripLayout &L = t->strips;
   const int nwaves = G * kWavesPerBlock, per = (L.nstrips + nwaves - 1) / nwaves;
@@ -1575,7 +1595,7 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
     if (!nsched.piece_order.empty())
       MF_HIP(hipMemcpyAsync(nsched.d_piece_order, nsched.piece_order.data(), sizeof(int) * nsched.piece_order.size(), hipMemcpyHostToDevice, st));
   }
-  if (opt.policy == MF_POLICY_ERRBOUND && t->tilenum > 0) {
+  if (opt.policy == MF_POLICY_ERRBOUND && !before && t->tilenum > 0) {
     MF_TRY(apply_errbound_levels(t, st));
     MF_TRY(wave_uniform_levels(t, sc->d_wave_tr, nwaves, st));
   }
@@ -1628,7 +1648,12 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
   std::memset(&r, 0, sizeof(r));
   double stats[kStCount];
   mf_status ret = MF_OK;
-  bool mixed = opt.policy != MF_POLICY_FP64;
+  bool mixed = opt.policy != MF_POLICY_FP64 && !before;
+  if (before) {
+    r = *before;
+    a.maxiter -= r.iterations;
+    if (opt.fixed_iters > 0) a.fixed_iters -= r.iterations;
+  }
   for (;;) {
     if (ret == MF_OK) ret = fill_u32(z0, (size_t)(z1 - z0), 0u, st);
     if (ret == MF_OK) ret = fill_u32(w.mbox, (size_t)G * kMboxWords * 8, 0u, st);
@@ -1675,7 +1700,7 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
     float ms = 0.0f;
     if (ret == MF_OK && hipEventRecord(e1, st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
         hipEventElapsedTime(&ms, e0, e1) == hipSuccess)
-      r.time_ms = ms;
+      r.time_ms += ms;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
   }
@@ -1683,9 +1708,11 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
   const double bb = stats[kStBB];
   r.rel_residual = bb > 0 ? std::sqrt(stats[kStTrue] / bb) : std::sqrt(stats[kStTrue]);
   r.rel_residual_recursive = bb > 0 ? std::sqrt(stats[kStRecursive] / bb) : 0.0;
-  r.grid_blocks = G;
-  r.form_used = MF_FORM_RESIDENT;
-  r.policy_used = opt.policy;
+  if (!before) {
+    r.grid_blocks = G;
+    r.form_used = MF_FORM_RESIDENT;
+    r.policy_used = opt.policy;
+  }
   ret = (int)stats[kStStatus];
   if (ret == MF_OK && opt.fixed_iters <= 0 && !(r.rel_residual <= opt.tol)) ret = MF_NOT_CONVERGED;
   r.status = ret;
@@ -1836,6 +1863,15 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   a.seg2 = w.seg2;
   a.prec_rw = t->dev.prec;
   a.nseg = (int)segs;
+  // A fallback to FP64 goes on over strips where an FP64 solve would run on
+  // them (64^3, rule policy: 17 us an iteration over tiles, 9.8 over strips).
+  int G64 = 0;
+  if (mode != kAll64) {
+    mf_solve_opts o64 = opt;
+    o64.policy = MF_POLICY_FP64;
+    MF_TRY(strip_grid(t, o64, bicg, &G64));
+  }
+  a.stop64 = G64 > 0;
   if (learned && !noalloc) MF_HIP(hipMemsetAsync(w.seg2, 0, segs * 4, st));
 
 #ifdef MF_PHASE_TRACE
@@ -1906,6 +1942,10 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   r.form_used = resident_windows ? MF_FORM_RESIDENT : MF_FORM_MEMORY;
   r.policy_used = opt.policy;
   int ret = status;
+  if (a.stop64 && r.fell_back && status == MF_OK && r.iterations < opt.maxiter &&
+      !(opt.fixed_iters <= 0 && r.rel_residual <= opt.tol) &&
+      !(opt.fixed_iters > 0 && r.iterations >= opt.fixed_iters))
+    return run_strips(t, d_b, d_x, opt, rep, G64, bicg, noalloc, &r);
   if (ret == MF_OK && opt.fixed_iters <= 0 && !(r.rel_residual <= opt.tol)) ret = MF_NOT_CONVERGED;
   r.status = ret;
   if (rep) *rep = r;

@@ -195,9 +195,10 @@ mf_status mf_tile_set_spmv_kernel(mf_tiled *t, int kind);
 /* Sizes of a device handle's row strips: strips of 64 rows (0: the handle has
  * none), pieces of rows too long for a strip, whether rows are sorted by
  * length inside windows, and the entry slots (padding included) stored as one
- * 32-bit word and in full.  No reference counterpart. */
+ * 32-bit word, in full, and as diagonals of one value for the strip.  No
+ * reference counterpart. */
 mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pieces, int *sorted,
-                             int64_t *packed_slots, int64_t *full_slots);
+                             int64_t *packed_slots, int64_t *full_slots, int64_t *diag_slots);
 
 /* Schedule knob for the autotuner: entries per wave of the stand-alone SpMV
  * (the streamed kernel's nnz-balanced tile-row ranges are rebuilt, and a

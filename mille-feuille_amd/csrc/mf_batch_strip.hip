@@ -52,7 +52,7 @@ __device__ __forceinline__ void block_product(const StripView &S, int w, int lan
   }
   int n = (S.nstrips + NW - 1) / NW;
   if (n > 0 && wave_strip<NW>(w, n - 1) >= S.nstrips) --n;
-  strips_run(S, lane, x, v32, n, [&](int k) { return wave_strip<NW>(w, k); },
+  strips_run<false>(S, lane, x, v32, n, [&](int k) { return wave_strip<NW>(w, k); },
              [&](int s, const StripDesc &d, int row, bool lng, double acc, double own) {
                if ((d.flags & kStripLong) && lng) {
                  const LongRow lr = S.lrow[S.lane_long[64 * s + lane]];

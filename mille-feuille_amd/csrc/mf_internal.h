@@ -86,7 +86,7 @@ struct DeviceLayout {
 };
 
 // Row strips (mf_strips.h).
-constexpr int kStripPacked = 0, kStripFull = 1, kStripNear = 2;
+constexpr int kStripPacked = 0, kStripFull = 1, kStripNear = 2, kStripDiag = 3;
 constexpr int kStripLong = 1;  // flags: a lane of the strip holds a row with pieces
 constexpr int kStripLead = 2;  // flags: the rows' diagonals are in the lead arrays
 constexpr int kLongBit = 1 << 30;  // row map: the row's other entries are in pieces
@@ -123,12 +123,23 @@ struct RowInfo {
 
 constexpr int kNearCols = 31000;
 
+// One diagonal of a strip: `val` at column row + off in the rows of `mask`.
+struct DiagSlot {
+  uint64_t mask;
+  double val;
+  int off, pad;
+};
+
+// Most off-diagonal slots of a strip of the diagonal class.
+constexpr int kMaxDiagSlots = 64, kDiagLead = 128;
+
 // Host side of the layout: descriptors (strips, then pieces), the row order
 // of sorted layouts and the long rows.
 struct StripPlan {
   bool ok = false, sorted = false;
   int nstrips = 0, nmulti = 0;
   uint64_t npacked = 0, nfull = 0;   // pairs per lane in words; in values (full, near)
+  uint64_t ndiag = 0;                // diagonal slots
   bool any_full = false, any_near = false;
   std::vector<StripDesc> desc;
   std::vector<int> safe;  // per descriptor, a row of it (the column of its padding)
@@ -145,6 +156,7 @@ struct StripLayout {
   int nlong = 0;     // rows with pieces, those longer than a piece first
   int nmulti = 0;    // rows longer than a piece
   int sorted = 0;    // rows sorted by length inside windows of strips
+  int leads = 0;     // half of the strips or more have a lead
   bool lean = false; // a product over strips reads fewer bytes than over tiles (lean_strips)
   StripDesc *desc = nullptr;
   uint32_t *words = nullptr;
@@ -152,6 +164,7 @@ struct StripLayout {
   float *vf = nullptr;
   int *vc = nullptr;
   uint16_t *vh = nullptr;
+  DiagSlot *dslot = nullptr;
   double *lead64 = nullptr;
   float *lead32 = nullptr;
   int *rowmap = nullptr;
@@ -232,7 +245,10 @@ mf_status upload_tiles(mf_tiled *t, int device, const int *rowptr);
 // Row strips of an uploaded handle (mf_strips.hip); rowptr: the CSR row
 // pointers the handle was built from.
 mf_status build_strips(mf_tiled *t, const int *rowptr);
-void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info, StripPlan &p);
+// ndiag: off-diagonal slots that the diagonal class needs for each unsorted
+// strip (255: not possible), plus kDiagLead where its diagonal entries differ.
+void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info,
+                 const std::vector<uint8_t> &ndiag, StripPlan &p);
 void free_strips(mf_tiled *t);
 bool lean_strips(const mf_tiled *t);
 void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s);

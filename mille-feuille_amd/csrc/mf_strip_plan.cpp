@@ -17,7 +17,8 @@ constexpr int kStripWin = 16;
 // Longest row of a sorted layout kept in its strip.
 constexpr int kLongRow = 64;
 
-void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info, StripPlan &P) {
+void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info,
+                 const std::vector<uint8_t> &ndiag, StripPlan &P) {
   const int rows = t->rowA, nstr = (16 * t->tilem + 63) / 64;
   auto len = [&](int r) { return rowptr[r + 1] - rowptr[r]; };
   // Unsorted strips where padding every row to the longest of its 64 costs
@@ -84,7 +85,7 @@ void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo
 #pragma omp parallel for reduction(max : wide)
   for (int s = 0; s < nstr; ++s) {
     int lo = 127, hi = -127, m = 0, first = -1;
-    bool lead = true, packed = true, near = true, lng = false;
+    bool lead = true, packed = true, near = true, lng = false, exact = true;
     for (int i = 64 * s; i < 64 * s + 64; ++i) {
       const int r = row_of(i);
       if (r < 0) {
@@ -93,7 +94,7 @@ void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo
       }
       if (first < 0) first = r;
       lead = lead && info[r].diag;
-      packed = packed && (info[r].plain & 1);
+      exact = exact && (info[r].plain & 1);
       if (sorted && len(r) > kLongRow) {
         lng = true;
         continue;
@@ -103,15 +104,23 @@ void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo
       hi = std::max<int>(hi, info[r].hi);
       m = std::max(m, len(r));
     }
-    packed = packed && lead && narrow(lo, hi);
+    packed = exact && lead && narrow(lo, hi);
+    // Diagonals where they are no more than the entries that rows are padded
+    // to: a slot gathers x like an entry, with fewer instructions and no bytes
+    // of its own (mf_strips.h has both sides).
+    const int nd = ndiag[s] == 255 ? 255 : ndiag[s] & ~kDiagLead;
+    const bool own_diag = ndiag[s] & kDiagLead;  // the diagonals differ: a lead
+    const bool diag = !sorted && exact && (lead || !own_diag) && nd <= kMaxDiagSlots &&
+                      nd <= 2 * pairs(lead ? m - 1 : m);
+    if (diag) lead = own_diag;
     if (lead && m > 0) --m;
     wide = std::max(wide, m);
     StripDesc d;
     d.off = 0;
-    d.npair = (uint16_t)pairs(m);
-    d.cls = packed ? kStripPacked : near ? kStripNear : kStripFull;
+    d.npair = (uint16_t)(diag ? nd : pairs(m));
+    d.cls = diag ? kStripDiag : packed ? kStripPacked : near ? kStripNear : kStripFull;
     d.flags = (uint8_t)((lng ? kStripLong : 0) | (lead ? kStripLead : 0));
-    d.scale = packed ? scale_of(lo) : 1.0f;
+    d.scale = packed && !diag ? scale_of(lo) : 1.0f;
     d.base = sorted ? s / kStripWin * kStripWin * 64 : 64 * s;
     P.desc[s] = d;
     P.safe[s] = std::max(first, 0);
@@ -139,13 +148,13 @@ void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo
   }
   // offsets in each class's arrays
   for (StripDesc &d : P.desc) {
-    uint64_t &n = d.cls == kStripPacked ? P.npacked : P.nfull;
+    uint64_t &n = d.cls == kStripPacked ? P.npacked : d.cls == kStripDiag ? P.ndiag : P.nfull;
     d.off = (uint32_t)n;
-    n += d.npair;
+    n += d.npair + (d.cls == kStripDiag ? 1 : 0);
     P.any_full = P.any_full || (d.cls == kStripFull && d.npair > 0);
     P.any_near = P.any_near || d.cls == kStripNear;
   }
-  P.ok = P.npacked <= 0xffffffffull && P.nfull <= 0xffffffffull;
+  P.ok = P.ndiag <= 0xffffffffull && P.npacked <= 0xffffffffull && P.nfull <= 0xffffffffull;
 }
 
 void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s) {

@@ -42,9 +42,9 @@ __device__ __forceinline__ double sum16(double v) {
   return v;
 }
 
-// The wave's strips [s0, s0 + n).
+// The wave's strips s0 + k * step, k < n.
 struct StripWave {
-  int s0, n, lane;
+  int s0, step, n, lane;
 };
 
 // Sum of the pieces of lane's long row, posted by the waves that hold them
@@ -83,7 +83,7 @@ __device__ __forceinline__ double take_pieces(const StripSolveArgs &a, int h, un
 // strips: w and (own_out) the rows' own entries of x to wl and rl (lane's slot of
 // strip k at 64 k), and the sums of own^2, w * own and w^2.  Pieces never
 // wait, and an owner waits only after its own pieces, so every wait ends.
-template <typename XT>
+template <bool EARLY, typename XT>
 __device__ __forceinline__ void strip_product(const StripSolveArgs &a, const StripWave &w, const XT *__restrict__ x,
                                               unsigned tag, bool v32, bool own_out, double *wl, double *rl,
                                               double (&g)[3]) {
@@ -98,10 +98,11 @@ __device__ __forceinline__ void strip_product(const StripSolveArgs &a, const Str
       if (w.lane == 0) mbox_post<1>(a.pmail + 2 * (size_t)pc, tag, v);
     }
   }
-  strips_run(S, w.lane, MemVec<XT>{x}, v32, w.n, [&](int k) { return w.s0 + k; },
+  int o = w.lane - 64;
+  strips_run<EARLY>(S, w.lane, MemVec<XT>{x}, v32, w.n, [&](int k) { return w.s0 + k * w.step; },
              [&](int s, const StripDesc &d, int, bool lng, double acc, double own) {
                if ((d.flags & kStripLong) && lng) acc += take_pieces(a, S.lane_long[64 * s + w.lane], tag);
-               const int o = 64 * (s - w.s0) + w.lane;
+               o += 64;
                wl[o] = acc;
                if (own_out) rl[o] = own;
                g[0] += own * own;
@@ -122,23 +123,28 @@ __device__ __forceinline__ void count_levels(const uint8_t *prec, int t0, int t1
   }
 }
 
-// The wave's strips, and the tiles whose levels it counts (and infers: learned
-// solves run on unsorted strips, whose tile-rows are the wave's own).
+// The wave's strips, and the tiles whose levels it counts and infers.  Unsorted
+// strips go round the waves of their block, so that the block's waves gather
+// from neighbouring rows at the same time (L1; FP64 64^3 9.5 us an iteration
+// with contiguous strips, now 9.3; error bound 128^3 25.6 and 24.9).  Sorted
+// ones stay contiguous: a window's longest come first.
 template <bool MIXED>
 __device__ __forceinline__ void wave_share(const StripSolveArgs &a, int wid, int lane, StripWave &W, int &t0, int &t1) {
-  const int nw = gridDim.x * kWavesPerBlock;
+  const int nw = gridDim.x * kWavesPerBlock, wv = wid % kWavesPerBlock;
   W.lane = lane;
-  W.s0 = (int)((long long)a.S.nstrips * wid / nw);
-  W.n = (int)((long long)a.S.nstrips * (wid + 1) / nw) - W.s0;
-  t0 = t1 = 0;
-  if (!MIXED) return;
   if (a.S.rowmap) {
-    t0 = (int)((long long)a.A.tilenum * wid / nw);
-    t1 = (int)((long long)a.A.tilenum * (wid + 1) / nw);
+    W.s0 = (int)((long long)a.S.nstrips * wid / nw);
+    W.step = 1;
+    W.n = (int)((long long)a.S.nstrips * (wid + 1) / nw) - W.s0;
   } else {
-    t0 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * W.s0, a.A.tilem)]);
-    t1 = __builtin_amdgcn_readfirstlane(a.A.tile_ptr[min(4 * (W.s0 + W.n), a.A.tilem)]);
+    const int b = wid / kWavesPerBlock, G = gridDim.x;
+    const int b0 = (int)((long long)a.S.nstrips * b / G), b1 = (int)((long long)a.S.nstrips * (b + 1) / G);
+    W.s0 = b0 + wv;
+    W.step = kWavesPerBlock;
+    W.n = max(b1 - W.s0 + kWavesPerBlock - 1, 0) / kWavesPerBlock;
   }
+  t0 = (int)((long long)a.A.tilenum * wid / nw);
+  t1 = (int)((long long)a.A.tilenum * (wid + 1) / nw);
 }
 
 // Row of the lane in strip s0 + k.  The lane is hidden from the optimizer,
@@ -148,7 +154,7 @@ __device__ __forceinline__ int wave_row(const StripSolveArgs &a, const StripWave
   int l = W.lane;
   asm("" : "+v"(l));
   bool lng;
-  return strip_row(a.S, W.s0 + k, l, lng);
+  return strip_row(a.S, W.s0 + k * W.step, l, lng);
 }
 
 __device__ __forceinline__ void add_hist(unsigned long long c, unsigned long long *h, int lane) {
@@ -184,11 +190,11 @@ __device__ __noinline__ void infer_levels(const int *tile_col, InferCtx c, int t
 // needs FP64 ends, and the host starts an FP64 one from its x).
 //
 // Measured on MI355X, us per iteration, FP64 / error bound (streamed tiles with
-// the vectors in memory before): 7-point 128^3 28.9 / 29.9 (54.0 / 45.0), of
+// the vectors in memory before): 7-point 128^3 29.3 / 24.7 (54.0 / 45.0), of
 // which the product 15, the update's stores 6.5 and the two synchronisations
-// 7.6; 117 x 89 x 86 15.3 / 16.6 (30.0 / 29.4); 64^3 10.3 / 11.6 (16.7 / 18.7), of
-// which synchronisation 6; 5-point 64^2 5.6 / 6.9 (10.8 / 13.3); 200k-row power
-// law 28.0 / 30.1 (97 / 107).  The 128^3 product moves 84 MB.
+// 7.6; 117 x 89 x 86 13.8 / 15.8 (30.0 / 29.4); 64^3 9.4 / 10.7 (16.7 / 18.7), of
+// which synchronisation 6; 5-point 64^2 5.5 / 6.9 (10.8 / 13.3); 200k-row power
+// law 28.0 / 30.1 (97 / 107).  The 128^3 product moves 40 MB.
 //
 // Each round of the
 // loop is one product: of x for a residual (kRes), of r for an iteration
@@ -240,13 +246,13 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
       if (infer) {
         infer_levels(a.A.tile_col, infer_ctx(a, rr, rr, bb), t0, t1, lane);
         count_levels(a.prec_rw, t0, t1, lane, nlev);
-        full64 = nlev[0] > 0;
+        full64 = __syncthreads_or(nlev[0] > 0);  // (the block's strips hold these tiles)
         infer = false;
       }
-      strip_product(a, W, (const float *)a.r32, tag, !full64, true, wl, rl, gd3);
+      strip_product<!MIXED>(a, W, (const float *)a.r32, tag, !full64, true, wl, rl, gd3);
     } else {
       const double *v = round == kRes ? a.x : round == kIter ? a.r : a.p;
-      strip_product(a, W, v, tag, false, true, wl, rl, gd3);
+      strip_product<!MIXED>(a, W, v, tag, false, true, wl, rl, gd3);
     }
     if (round == kRes) {
       // r = b - A x of the wave's rows (stored unless it is the last)
@@ -499,13 +505,13 @@ __global__ __launch_bounds__(kBlock) void k_bicgstab_strip(StripSolveArgs a) {
       if (round == kP && infer) {
         infer_levels(a.A.tile_col, infer_ctx(a, pp_last, rr, bb), t0, t1, lane);
         count_levels(a.prec_rw, t0, t1, lane, nlev);
-        full64 = nlev[0] > 0;
+        full64 = __syncthreads_or(nlev[0] > 0);  // (the block's strips hold these tiles)
         infer = false;
       }
-      strip_product(a, W, (const float *)(round == kP ? gp : gs_), tag, !full64, round == kP, wl, rl, gd);
+      strip_product<false>(a, W, (const float *)(round == kP ? gp : gs_), tag, !full64, round == kP, wl, rl, gd);
     } else {
       const double *u = round == kRes ? a.x : (const double *)(round == kP ? gp : gs_);
-      strip_product(a, W, u, tag, false, round == kP, wl, rl, gd);
+      strip_product<false>(a, W, u, tag, false, round == kP, wl, rl, gd);
     }
     bool step = false;  // go on to p = r + beta (p - omega v)
     bool restart = false;

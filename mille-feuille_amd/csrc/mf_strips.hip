@@ -57,6 +57,95 @@ __global__ __launch_bounds__(256) void k_row_info(TileView A, int rows, RowInfo 
   if (lane == 0) info[row] = RowInfo{(int8_t)lo, (int8_t)hi, (uint8_t)diag, (uint8_t)plain};
 }
 
+// One wave per strip of 64 consecutive rows, a row per lane: merges the rows'
+// entries (in tile order) by column - row, smallest first, so each step takes
+// one entry of every row that has that offset next.  Entries are taken once
+// each whatever their order; where one step's values differ, the strip has no
+// diagonal form.  FILL: the slots (and leads) of the strips that the plan gave
+// this class; else the number of off-diagonal slots (255: none), plus
+// kDiagLead if the diagonal entries differ.
+template <bool FILL>
+__global__ __launch_bounds__(256) void k_diag_slots(TileView A, int rows, int nstrips, uint8_t *__restrict__ count,
+                                                    const StripDesc *__restrict__ desc,
+                                                    DiagSlot *__restrict__ out, double *__restrict__ lead64,
+                                                    float *__restrict__ lead32) {
+  const int s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (s >= nstrips) return;
+  if (FILL) {
+    if (desc[s].cls != kStripDiag) return;
+    out += desc[s].off;
+  }
+  const int row = 64 * s + lane, r = row & 15;
+  int t = 0, tend = 0, k = 0, e = 0;
+  if (row < rows) {
+    t = A.tile_ptr[row >> 4];
+    tend = A.tile_ptr[(row >> 4) + 1];
+  }
+  if (t < tend) {
+    int b;
+    tile_row_range(A, t, r, b, e);
+    k = A.tile_off[t] + b;
+    e += A.tile_off[t];
+  }
+  bool diag = false, live = true;
+  double dv = 0.0, v = 0.0;
+  int off = 0;
+  auto next = [&]() {  // the lane's next off-diagonal entry
+    for (;;) {
+      while (k >= e && t + 1 < tend) {
+        int b;
+        ++t;
+        tile_row_range(A, t, r, b, e);
+        k = A.tile_off[t] + b;
+        e += A.tile_off[t];
+      }
+      if (k >= e) {
+        live = false;
+        return;
+      }
+      off = (A.tile_col[t] << 4) + (A.rc[k] & 15) - row;
+      v = A.v64[k];
+      ++k;
+      if (off != 0 || diag) return;
+      diag = true;
+      dv = v;
+    }
+  };
+  // all lanes: whether the lanes of `in` hold one value, and that value
+  auto common = [&](unsigned long long in, double x, double &c) {
+    c = in ? __shfl(x, (int)__builtin_ctzll(in)) : 0.0;
+    const bool same = __builtin_bit_cast(unsigned long long, x) == __builtin_bit_cast(unsigned long long, c);
+    return (__ballot(!same) & in) == 0;
+  };
+  next();
+  int n = 0;
+  double c;
+  for (unsigned long long act; (act = __ballot(live)) != 0;) {
+    const int m = wave_min(live ? off : 0x7fffffff);
+    const bool mine = live && off == m;
+    const unsigned long long in = __ballot(mine);
+    if (n == kMaxDiagSlots || !common(in, v, c)) {
+      n = 255;
+      break;
+    }
+    ++n;
+    if (FILL && lane == 0) out[n] = DiagSlot{in, c, m, 0};
+    if (mine) next();
+  }
+  const unsigned long long in = __ballot(diag);
+  const bool same = common(in, dv, c);
+  if (FILL) {
+    const bool lead = desc[s].flags & kStripLead;
+    if (lane == 0) out[0] = lead ? DiagSlot{0, 0.0, 0, 0} : DiagSlot{in, c, 0, 0};
+    if (lead) {
+      lead64[row] = dv;
+      lead32[row] = (float)dv;  // (the payload of the rows of this class)
+    }
+  } else if (lane == 0) {
+    count[s] = (uint8_t)(n == 255 ? n : n | (same ? 0 : kDiagLead));
+  }
+}
+
 struct FillArgs {
   TileView A;
   const StripDesc *desc;
@@ -100,6 +189,7 @@ __global__ __launch_bounds__(256) void k_fill_strips(FillArgs a) {
   const int slot = a.slot ? a.slot[row] : row;
   const int h = a.long_of ? a.long_of[row] : -1;
   const StripDesc sd = a.desc[slot >> 6];
+  if (sd.cls == kStripDiag) return;
   const bool lead = sd.flags & kStripLead;  // the diagonal goes to the lead
   const int piece0 = h >= 0 ? a.lrow[h].first : 0;
   int pos = 0;  // off-diagonal (or all) entries before this batch of tiles
@@ -199,7 +289,7 @@ __global__ __launch_bounds__(256, 8) void k_spmv_strip(StripView S, int pblocks,
   const int per_xcd = (gridDim.x - (PIECES ? pblocks : 0)) >> 3;  // both counts are multiples of 8
   const int s = ((b & 7) * per_xcd + (b >> 3)) * 4 + wv;
   if (s >= S.nstrips) return;
-  strips_run(S, lane, MemVec<double>{x}, false, 1, [&](int) { return s; },
+  strips_run<true>(S, lane, MemVec<double>{x}, false, 1, [&](int) { return s; },
              [&](int, const StripDesc &, int row, bool lng, double acc, double) {
                if (row >= 0 && !lng) y[row] = acc;
              });
@@ -236,18 +326,27 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
   const int rows = t->rowA;
   if (rows == 0 || t->tilenum == 0) return MF_OK;
   const TileView A = view_of(t);
+  const int nstrips = (16 * t->tilem + 63) / 64;
   std::vector<RowInfo> info(rows);
+  std::vector<uint8_t> ndiag(nstrips);
   {
     RowInfo *d = nullptr;
-    MF_HIP(hipMalloc(&d, sizeof(RowInfo) * rows));
+    uint8_t *nd = nullptr;
+    Slab both;
+    void *mem = nullptr;
+    both.add(&d, rows);
+    both.add(&nd, nstrips);
+    MF_TRY(both.alloc(&mem));
     k_row_info<<<(rows + 3) / 4, 256>>>(A, rows, d);
+    k_diag_slots<false><<<(nstrips + 3) / 4, 256>>>(A, rows, nstrips, nd, nullptr, nullptr, nullptr, nullptr);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpy(info.data(), d, sizeof(RowInfo) * rows, hipMemcpyDeviceToHost);
-    (void)hipFree(d);
+    if (e == hipSuccess) e = hipMemcpy(ndiag.data(), nd, nstrips, hipMemcpyDeviceToHost);
+    (void)hipFree(mem);
     if (e != hipSuccess) return fail(MF_ERR_HIP, std::string("build_strips: ") + hipGetErrorString(e));
   }
   StripPlan P;
-  plan_strips(t, rowptr, info, P);
+  plan_strips(t, rowptr, info, ndiag, P);
   if (!P.ok) return MF_OK;
   const int nstr = P.nstrips;
   const uint64_t np = P.npacked, nf = P.nfull;
@@ -256,6 +355,9 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
   L.nlong = (int)P.lrow.size();
   L.nmulti = P.nmulti;
   L.hdesc = P.desc;
+  int leads = 0;
+  for (int s = 0; s < nstr; ++s) leads += (P.desc[s].flags & kStripLead) != 0;
+  L.leads = 2 * leads >= nstr;
   int *d_safe = nullptr, *d_slot = nullptr, *d_long = nullptr;
   Slab slab, tmp;
   slab.add(&L.desc, P.desc.size());
@@ -264,6 +366,7 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
   slab.add(&L.vf, 128 * nf);
   if (P.any_full) slab.add(&L.vc, 128 * nf);
   if (P.any_near) slab.add(&L.vh, 128 * nf);
+  if (P.ndiag) slab.add(&L.dslot, P.ndiag);
   slab.add(&L.lead64, 64 * (size_t)nstr);
   slab.add(&L.lead32, 64 * (size_t)nstr);
   if (P.sorted) slab.add(&L.rowmap, P.rowmap.size());
@@ -302,6 +405,7 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
     FillArgs a{A, L.desc, d_slot, d_long, L.lrow, L.words, L.vv, L.vf, L.vc, L.vh,
                L.lead64, L.lead32, rows, nstr};
     k_fill_strips<<<(rows + 3) / 4, 256>>>(a);
+    if (P.ndiag) k_diag_slots<true><<<(nstr + 3) / 4, 256>>>(A, rows, nstr, nullptr, L.desc, L.dslot, L.lead64, L.lead32);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) st = fail(MF_ERR_HIP, std::string("build_strips: ") + hipGetErrorString(e));
@@ -316,16 +420,23 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
 using namespace mf;
 
 extern "C" mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pieces, int *sorted,
-                                        int64_t *packed_slots, int64_t *full_slots) {
+                                        int64_t *packed_slots, int64_t *full_slots,
+                                        int64_t *diag_slots) {
   if (!t) return fail(MF_ERR_ARG, "mf_tile_strip_info: null handle");
   const StripLayout &L = t->strips;
-  int64_t n[2] = {0, 0};
+  int64_t n[3] = {0, 0, 0};
   if (L.nstrips > 0)
-    for (const StripDesc &d : L.hdesc) n[d.cls == kStripPacked ? 0 : 1] += 128 * (int64_t)d.npair;
+    for (const StripDesc &d : L.hdesc) {
+      if (d.cls == kStripDiag)
+        n[2] += 64 * ((int64_t)d.npair + 1);
+      else
+        n[d.cls == kStripPacked ? 0 : 1] += 128 * (int64_t)d.npair;
+    }
   if (strips) *strips = L.nstrips;
   if (pieces) *pieces = L.npieces;
   if (sorted) *sorted = L.sorted;
   if (packed_slots) *packed_slots = n[0];
   if (full_slots) *full_slots = n[1];
+  if (diag_slots) *diag_slots = n[2];
   return MF_OK;
 }

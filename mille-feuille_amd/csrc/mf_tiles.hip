@@ -272,8 +272,8 @@ bool lean_strips(const mf_tiled *t) {
   // value and column, a lead per row; tiles: value, byte and metadata), so the
   // fewer bytes win, with a margin for what strips save besides.  Measured on
   // MI355X, strips / streamed tiles, operands in the caches and not: 128^3
-  // 7-point Laplacian (packed, 67 against 151 MB) 17.5 / 30.2 and 36.7 / 68.9
-  // us; the same pattern with random values (near, 143 MB) 24.9 / 30.1 and
+  // 7-point Laplacian (diagonals, 23 against 151 MB) 16.1 / 30.2 and 30.6 / 68.9
+  // us, (packed, 67 MB) 17.5 and 36.7; the same pattern with random values (near, 143 MB) 24.9 / 30.1 and
   // 57.9 / 68.8; 64-entry bands of random values (near, 65 against 58 MB)
   // 12.3 / 13.2 and 26.3 / 28.6; 150k-row kNN graph, random values (17
   // against 19 MB) 5.7 / 6.2 and 16.4 / 13.9; 200k-row power-law graph (packed,
@@ -282,7 +282,8 @@ bool lean_strips(const mf_tiled *t) {
   if (L.nstrips == 0) return false;
   double strip = 8.0 * 64.0 * L.nstrips;
   for (const StripDesc &d : L.hdesc)
-    strip += 128.0 * d.npair * (d.cls == kStripPacked ? 4.0 : d.cls == kStripNear ? 10.0 : 12.0);
+    strip += d.cls == kStripDiag ? 24.0 * (d.npair + 1)
+                                 : 128.0 * d.npair * (d.cls == kStripPacked ? 4.0 : d.cls == kStripNear ? 10.0 : 12.0);
   const double tiles = 9.0 * t->dev.npay + 13.0 * t->tilenum;
   return strip <= 1.2 * tiles;
 }

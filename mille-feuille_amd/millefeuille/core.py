@@ -207,10 +207,12 @@ class TiledMatrix:
     def strips(self):
         """Sizes of the handle's row-strip layout: strips (0: none), pieces of
         long rows, whether rows are sorted, and the entry slots
-        stored packed (one 32-bit word each) and in full."""
-        v = [C.c_int(), C.c_int(), C.c_int(), C.c_int64(), C.c_int64()]
+        stored packed (one 32-bit word each), in full, and as diagonals of one
+        value."""
+        v = [C.c_int(), C.c_int(), C.c_int(), C.c_int64(), C.c_int64(), C.c_int64()]
         check("mf_tile_strip_info", lib.mf_tile_strip_info(self.h, *[C.byref(q) for q in v]))
-        return dict(zip(("strips", "pieces", "sorted", "packed_slots", "full_slots"), [q.value for q in v]))
+        return dict(zip(("strips", "pieces", "sorted", "packed_slots", "full_slots", "diag_slots"),
+                        [q.value for q in v]))
 
     def set_spmv_kernel(self, kind):
         """'auto', 'stream', 'rowgroup' or 'strip' (or the MF_SPMV_* value)."""

@@ -111,3 +111,68 @@ def test_non_finite_x_reaches_only_coupled_rows(mf, oracle, kind, bad):
     hit = np.zeros(n, bool)
     hit[rows[np.isin(ci, [0, 77])]] = True
     np.testing.assert_array_equal(~np.isfinite(dy.get()[:n]), hit)
+
+
+def _stencil(n, offs, vals, diag, rng, shuffle=False):
+    """CSR with value vals[k] at offset offs[k] wherever the column exists;
+    diag: "same", "each" (its own value per row) or "some" (every third row)."""
+    rp, ci, va = [0], [], []
+    for i in range(n):
+        row = [(i + o, v) for o, v in zip(offs, vals) if 0 <= i + o < n]
+        if diag != "some" or i % 3 == 0:
+            row.append((i, 5.5 if diag != "each" else 0.3 + i))
+        row.sort()
+        if shuffle:
+            rng.shuffle(row)
+        ci += [c for c, _ in row]
+        va += [v for _, v in row]
+        rp.append(len(ci))
+    return np.array(rp, np.int32), np.array(ci, np.int32), np.array(va, np.float64)
+
+
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 130, 1025])
+@pytest.mark.parametrize("diag", ["same", "each", "some"])
+@pytest.mark.parametrize("shuffle", [False, True])
+def test_diagonals(mf, oracle, n, diag, shuffle):
+    """One value for each diagonal of a strip; the first and last rows lack
+    entries, as does the last strip."""
+    rng = np.random.default_rng(n)
+    rp, ci, va = _stencil(n, [-90, -64, -17, -1, 1, 17, 64, 90], [-0.1, 1 / 3, 0.0, -1, -1.7, 2, 1e-3, 1e6], diag, rng, shuffle)
+    tm = _check(mf, oracle, rp, ci, va)
+    if n == 1025 and not shuffle:
+        assert tm.strips()["diag_slots"] > 0
+    # the streamed kernel over the same payload
+    x = rng.uniform(-1, 1, n)
+    dx, ys, yt = tm.vector(x), tm.vector(), tm.vector()
+    tm.spmv(dx, ys)
+    tm.set_spmv_kernel("stream")
+    tm.spmv(dx, yt)
+    bound = oracle.csr_spmv(rp, ci, np.abs(va), np.abs(x))
+    assert np.all(np.abs(ys.get() - yt.get())[:n] <= 1e-14 * bound + 1e-300)
+
+
+@pytest.mark.parametrize("slots", list(range(0, 15)) + [63, 64, 65])
+def test_diagonal_counts(mf, oracle, slots):
+    """Every remainder of the groups of gathers, and the most slots of a strip."""
+    n, rng = 600, np.random.default_rng(slots)
+    offs = sorted(rng.choice([o for o in range(-150, 151) if o], slots, replace=False))
+    rp, ci, va = _stencil(n, offs, list(rng.standard_normal(slots)), "same", rng)
+    tm = _check(mf, oracle, rp, ci, va)
+    # (strips at the ends have fewer diagonals)
+    assert tm.strips()["diag_slots"] > 0 and (tm.strips()["full_slots"] > 0 or slots <= 64)
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_diagonals_non_finite_x(mf, oracle, bad):
+    n = 1280
+    rp, ci, va = _stencil(n, [-65, -1, 1, 65], [1.0] * 4, "some", None)
+    tm = mf.TiledMatrix(rp, ci, va)
+    tm.set_spmv_kernel("strip")
+    x = np.random.default_rng(2).uniform(1, 2, n)
+    x[[0, 77]] = bad
+    dx, dy = tm.vector(x), tm.vector()
+    tm.spmv(dx, dy)
+    assert tm.strips()["diag_slots"] > 0
+    hit = np.zeros(n, bool)
+    hit[np.repeat(np.arange(n), np.diff(rp))[np.isin(ci, [0, 77])]] = True
+    np.testing.assert_array_equal(~np.isfinite(dy.get()[:n]), hit)

@@ -181,7 +181,7 @@ __device__ __forceinline__ InferCtx infer_ctx(const StripSolveArgs &a, double v2
 __device__ __noinline__ void infer_levels(const int *tile_col, InferCtx c, int t0, int t1, int lane) {
   TileView A;
   A.tile_col = tile_col;
-  wave_infer_tiles(A, c, t0, t1, lane);
+  wave_infer_tiles<false>(A, c, t0, t1, lane);
 }
 
 // Chronopoulos-Gear CG: w = A r with gamma = r.r and delta = w.r, one fused

@@ -77,15 +77,25 @@ _VEC_BYTES = {("cg", False): 72, ("cg", True): 44, ("bicgstab", False): 128, ("b
 
 
 def _iteration_roofline(tm, res, method, levels=None):
-    """Modeled HBM bytes per iteration (the SpMV formula at the tile levels
-    the mixed solve ran with -- `levels`, else the handle's after the solve --
-    or all FP64, plus the vector passes) and the rate they imply at each
-    solve's measured kernel time per iteration."""
+    """Modeled HBM bytes per iteration and the rate they imply at each solve's
+    measured kernel time per iteration.  Over row strips: the layout's bytes
+    and, per product, one read and one write of the vector it gathers (the
+    others stay on chip).  Over tiles: the SpMV formula at the tile levels the
+    mixed solve ran with -- `levels`, else the handle's after the solve -- or
+    all FP64, plus the vector passes."""
     import millefeuille as mf
     spmvs = 2 if method == "bicgstab" else 1
     out = {}
     for pol, r in res.items():
         mixed = pol != "fp64" and not r["fell_back"]
+        if pol != "rule" and tm.strips()["lean"]:
+            b_it = spmvs * (tm.strips()["bytes"] + (8 if mixed else 16) * tm.rowA)
+            us = 1e3 * r["kernel_ms"] / max(r["iterations"], 1)
+            gbs = b_it / (us * 1e-6) / 1e9
+            out[pol] = {"bytes_per_iteration": int(b_it), "us_per_iteration": round(us, 2),
+                        "achieved_gbs": round(gbs, 1), "frac_of_8tbs": round(gbs / HBM_PEAK_GBS, 4),
+                        "levels": "row strips, FP32 vectors" if mixed else "row strips, FP64"}
+            continue
         lv = (tm.get_precision() if levels is None else levels) if mixed else None
         b_spmv = mf.spmv_bytes(tm, levels=lv, x_bytes=4 if mixed else 8)
         b_it = spmvs * b_spmv + _VEC_BYTES[(method, mixed)] * tm.rowA
@@ -355,6 +365,23 @@ def main():
     xs = np.random.default_rng(0).uniform(-1, 1, n)
     dxs, dys = tm.vector(xs), tm.vector()
     tune = None
+    strip = None
+    if tm.strips()["lean"]:
+        # the default kernel; its bytes are those of the strip layout, x and y
+        timer = mf.Timer()
+        for _ in range(10):
+            tm.spmv(dxs, dys)
+        runs = []
+        for _ in range(5):
+            timer.start()
+            for _ in range(args.spmv_runs):
+                tm.spmv(dxs, dys)
+            runs.append(timer.stop() / args.spmv_runs)
+        sb = tm.strips()["bytes"] + 16 * n
+        strip = {"kernel": tm.spmv_kernel_name(), "us_per_launch": round(1e3 * float(np.median(runs)), 2),
+                 "bytes": sb, "GBps": round(sb / (float(np.median(runs)) * 1e-3) / 1e9, 1)}
+        log(f"spmv over strips: {strip}")
+    # the streamed tiles' roofline (a schedule selects that kernel)
     if args.wave_nnz > 0:
         tm.set_schedule(args.wave_nnz)
         wave_nnz = args.wave_nnz
@@ -449,7 +476,8 @@ def main():
         "speedup_vs_rule": round(others["rule"]["ms"] / mixed_ms, 3),
         "spmv": {"us_per_launch": round(t_spmv * 1e3, 2), "us_single_launch": round(t_single * 1e3, 2),
                  "bytes": bytes_spmv, "GBps": round(gbs, 1), "wave_nnz": wave_nnz, "tune": tune,
-                 "kernel": tm.spmv_kernel_name(), "copy_GBps_measured": round(copy_gbs, 1)},
+                 "kernel": tm.spmv_kernel_name(), "strips": strip,
+                 "copy_GBps_measured": round(copy_gbs, 1)},
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": traffic},
         "cpu_baseline": cpu_baseline,

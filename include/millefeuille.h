@@ -183,8 +183,8 @@ mf_status mf_spmv(mf_tiled *t, const double *d_x, const float *d_x32,
  * ranges, LDS row accumulators; any sparsity), MF_SPMV_ROWGROUP (one row per
  * lane, four tile-rows per wave; regular sparsity), MF_SPMV_STRIP (mode 0: a
  * layout of row strips built with the handle, one row per lane; mode 1 runs
- * the streamed kernel) or MF_SPMV_AUTO (the default: strips where the handle
- * has them, else streamed).
+ * the streamed kernel) or MF_SPMV_AUTO (the default: strips where they are
+ * lean, see mf_tile_strip_info, else streamed).
  * No reference counterpart (one kernel form there, src/Mille-feuille-cg.h:97-166). */
 #define MF_SPMV_AUTO (-1)
 #define MF_SPMV_STREAM 0
@@ -195,10 +195,12 @@ mf_status mf_tile_set_spmv_kernel(mf_tiled *t, int kind);
 /* Sizes of a device handle's row strips: strips of 64 rows (0: the handle has
  * none), pieces of rows too long for a strip, whether rows are sorted by
  * length inside windows, and the entry slots (padding included) stored as one
- * 32-bit word, in full, and as diagonals of one value for the strip.  No
- * reference counterpart. */
+ * 32-bit word, in full, and as diagonals of one value for the strip; bytes: what
+ * an FP64 product reads of the layout; lean: that is little enough next to the
+ * tiles for strips to be the default.  No reference counterpart. */
 mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pieces, int *sorted,
-                             int64_t *packed_slots, int64_t *full_slots, int64_t *diag_slots);
+                             int64_t *packed_slots, int64_t *full_slots, int64_t *diag_slots,
+                             int64_t *bytes, int *lean);
 
 /* Schedule knob for the autotuner: entries per wave of the stand-alone SpMV
  * (the streamed kernel's nnz-balanced tile-row ranges are rebuilt, and a
@@ -224,10 +226,14 @@ mf_status mf_stream_copy(const double *d_src, double *d_dst, int64_t n,
 #define MF_POLICY_FIXED 2   /* use the levels set with mf_tile_set_precision */
 #define MF_POLICY_LEARNED 3 /* MLP over per-tile features (mf_policy_*); the
                                FP32 / FP16 / INT8 classes of a solver wave's
-                               tiles run at the most precise of them */
+                               tiles run at the most precise of them.  Over
+                               row strips: the FP32 payload wherever no tile of
+                               the block is FP64, else its FP64 payload */
 #define MF_POLICY_ERRBOUND 4 /* analytic per-tile quantisation error bound;
                                 the FP32 / FP16 / INT8 levels of a solver
-                                wave's tiles run at the most precise of them */
+                                wave's tiles run at the most precise of them
+                                (over row strips the FP32 payload multiplies
+                                at every narrow level) */
 
 typedef struct mf_solve_opts {
   double tol;           /* stop at ||b - A x||_2 <= tol * ||b||_2 (FP64) */
@@ -242,20 +248,25 @@ typedef struct mf_solve_opts {
                            check -> FP64 fallback and restart (0 -> 64) */
   int blocks;           /* persistent grid size override (0: about 1024 rows
                            per block, at least 4 blocks, at most one block of
-                           16 waves per CU) */
+                           16 waves per CU; over row strips 2048 rows per block
+                           from 128 blocks on, 512 with pieces of long rows) */
   int fixed_iters;      /* >0: run exactly this many iterations, no test
                            (reference timing mode, src/Mille-feuille-cg.h:426) */
   int form;             /* solver SpMV form: MF_FORM_MEMORY (every SpMV reads
                            the tile metadata of each wave's windows from HBM),
-                           MF_FORM_RESIDENT or MF_FORM_AUTO (each wave keeps
-                           its share's tile metadata in LDS for the whole
-                           solve when every share fits a window of 40
+                           MF_FORM_RESIDENT or MF_FORM_AUTO (FP64, ERRBOUND
+                           and LEARNED on a handle whose row strips are no
+                           larger than its tiles: strips, each wave's vectors
+                           in registers, up to 8 strips a wave.  Else each wave
+                           keeps its share's tile metadata in LDS for the
+                           whole solve when every share fits a window of 40
                            tile-rows, 256 tiles and 1024 chunks with no heavy
                            tile-row; else as MEMORY).  The report's form_used
-                           says which ran. */
+                           says which ran; strips count as RESIDENT. */
   int batch_waves;      /* mf_batch_cg_solve: waves per (system, right-hand
-                           side) item, 4, 8 or 16 (0 -> 8; mf_tune_batch
-                           picks one) */
+                           side) item, 4, 8 or 16 (0 -> 16 where every system
+                           has row strips and the policy is not FIXED, else 8;
+                           mf_tune_batch picks one) */
   void *stream;         /* hipStream_t */
 } mf_solve_opts;
 

@@ -250,6 +250,7 @@ mf_status build_strips(mf_tiled *t, const int *rowptr);
 void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo> &info,
                  const std::vector<uint8_t> &ndiag, StripPlan &p);
 void free_strips(mf_tiled *t);
+int64_t strip_bytes(const StripLayout &L);  // of the layout that an FP64 product reads
 bool lean_strips(const mf_tiled *t);
 void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s);
 void free_device(mf_tiled *t);

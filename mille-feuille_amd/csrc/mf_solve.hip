@@ -1,4 +1,6 @@
-// mf_solve.hip -- single-kernel (persistent, cooperative) CG and BiCGSTAB.
+// mf_solve.hip -- single-kernel (persistent, cooperative) CG and BiCGSTAB
+// over tiles, and the host side of all single-kernel solves (strip_grid says
+// which run over row strips, mf_strip_solve.hip).
 //
 // One launch runs the whole solve.  The grid is sized to the occupancy of
 // the kernel on every CU and launched cooperatively, so all blocks are

@@ -321,6 +321,18 @@ void free_strips(mf_tiled *t) {
   s = StripLayout();
 }
 
+int64_t strip_bytes(const StripLayout &L) {
+  int64_t b = (int64_t)(sizeof(StripDesc) * L.hdesc.size()) + (L.sorted ? 256 * (int64_t)L.nstrips : 0);
+  for (const StripDesc &d : L.hdesc) {
+    if (d.flags & kStripLead) b += 8 * 64;
+    if (d.cls == kStripDiag)
+      b += (int64_t)sizeof(DiagSlot) * (d.npair + 1);
+    else
+      b += 128 * (int64_t)d.npair * (d.cls == kStripPacked ? 4 : d.cls == kStripNear ? 10 : 12);
+  }
+  return b;
+}
+
 mf_status build_strips(mf_tiled *t, const int *rowptr) {
   StripLayout &L = t->strips;
   const int rows = t->rowA;
@@ -421,7 +433,7 @@ using namespace mf;
 
 extern "C" mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pieces, int *sorted,
                                         int64_t *packed_slots, int64_t *full_slots,
-                                        int64_t *diag_slots) {
+                                        int64_t *diag_slots, int64_t *bytes, int *lean) {
   if (!t) return fail(MF_ERR_ARG, "mf_tile_strip_info: null handle");
   const StripLayout &L = t->strips;
   int64_t n[3] = {0, 0, 0};
@@ -438,5 +450,7 @@ extern "C" mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pie
   if (packed_slots) *packed_slots = n[0];
   if (full_slots) *full_slots = n[1];
   if (diag_slots) *diag_slots = n[2];
+  if (bytes) *bytes = L.nstrips > 0 ? strip_bytes(L) : 0;
+  if (lean) *lean = L.lean;
   return MF_OK;
 }

@@ -280,12 +280,8 @@ bool lean_strips(const mf_tiled *t) {
   // pieces; 16 against 135 MB) 25.8 / 149 and 41 / 215.
   const StripLayout &L = t->strips;
   if (L.nstrips == 0) return false;
-  double strip = 8.0 * 64.0 * L.nstrips;
-  for (const StripDesc &d : L.hdesc)
-    strip += d.cls == kStripDiag ? 24.0 * (d.npair + 1)
-                                 : 128.0 * d.npair * (d.cls == kStripPacked ? 4.0 : d.cls == kStripNear ? 10.0 : 12.0);
   const double tiles = 9.0 * t->dev.npay + 13.0 * t->tilenum;
-  return strip <= 1.2 * tiles;
+  return (double)strip_bytes(L) <= 1.2 * tiles;
 }
 
 int default_spmv_kernel(const mf_tiled *t) { return t->strips.lean ? MF_SPMV_STRIP : MF_SPMV_STREAM; }

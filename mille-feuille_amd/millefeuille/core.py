@@ -195,7 +195,7 @@ class TiledMatrix:
         if self._spmv_kernel == _lib.SPMV_ROWGROUP:
             return "mf::k_spmv_rg<0>"
         d = self.strips()
-        if d["strips"] and self._spmv_kernel != _lib.SPMV_STREAM:
+        if self._spmv_kernel == _lib.SPMV_STRIP or (d["lean"] and self._spmv_kernel == _lib.SPMV_AUTO):
             return f"mf::k_spmv_strip<{'true' if d['pieces'] else 'false'}>"
         a = self.arrays()
         slots = (np.diff(a["csr_offset"]).astype(np.int64) + 3) // 4 * 4
@@ -208,10 +208,11 @@ class TiledMatrix:
         """Sizes of the handle's row-strip layout: strips (0: none), pieces of
         long rows, whether rows are sorted, and the entry slots
         stored packed (one 32-bit word each), in full, and as diagonals of one
-        value."""
-        v = [C.c_int(), C.c_int(), C.c_int(), C.c_int64(), C.c_int64(), C.c_int64()]
+        value; the bytes of it that an FP64 product reads; and whether
+        strips are the default (lean)."""
+        v = [C.c_int(), C.c_int(), C.c_int()] + [C.c_int64() for _ in range(4)] + [C.c_int()]
         check("mf_tile_strip_info", lib.mf_tile_strip_info(self.h, *[C.byref(q) for q in v]))
-        return dict(zip(("strips", "pieces", "sorted", "packed_slots", "full_slots", "diag_slots"),
+        return dict(zip(("strips", "pieces", "sorted", "packed_slots", "full_slots", "diag_slots", "bytes", "lean"),
                         [q.value for q in v]))
 
     def set_spmv_kernel(self, kind):

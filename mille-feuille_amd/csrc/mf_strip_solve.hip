@@ -50,40 +50,50 @@ struct StripWave {
 // Sum of the pieces of lane's long row, posted by the waves that hold them
 // (values tagged with the product's ordinal, as in grid_sum_values; waits are
 // bounded).
-// Eight pieces are awaited at a time: one by one, a row of 32 pieces cost 32
+// 2 D pieces are awaited at a time: one by one, a row of 32 pieces cost 32
 // trips through memory (200k-row power law: 30.6 us an iteration, now 28.0).
+template <int N>
 __device__ __forceinline__ double take_pieces(const StripSolveArgs &a, int h, unsigned tag) {
   const LongRow lr = a.S.lrow[h];
   double sum = 0.0;
-  for (int j = 0; j < lr.n; j += 8) {
-    unsigned long long q[16];
+  for (int j = 0; j < lr.n; j += N) {
+    unsigned long long q[2 * N];
     unsigned spins = 0;
     for (;;) {
       bool ok = true;
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
+      for (int u = 0; u < 2 * N; ++u) {
         // (past the last piece: the last again, not added)
         const int i = min(j + u / 2, lr.n - 1);
         q[u] = __hip_atomic_load(a.pmail + 2 * (size_t)(lr.first + i) + (u & 1), __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
       }
 #pragma unroll
-      for (int u = 0; u < 16; ++u) ok = ok && (unsigned)(q[u] >> 32) == tag;
+      for (int u = 0; u < 2 * N; ++u) ok = ok && (unsigned)(q[u] >> 32) == tag;
       if (ok || !spin_on(spins, a.gs)) break;
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < N; ++u)
       if (j + u < lr.n)
         sum += __builtin_bit_cast(double, (q[2 * u + 1] & 0xffffffffull) << 32 | (q[2 * u] & 0xffffffffull));
   }
   return sum;
 }
 
+// Pairs of entries in flight in a product.  Eight strips of FP64 vectors are 48
+// (BiCGSTAB 64) of a lane's 128 registers: with four pairs in flight besides, 12 of them
+// went to memory and back in every iteration (128^3, 25 MB).  CG with two 26.2 us an
+// iteration, with four 29.2; random values 39.8 / 41.2, 21 entries a row 50.0 / 50.3.
+// At four strips a wave the two are mixed (900k rows of 21 packed entries 27.8 /
+// 26.0, 7 diagonals 13.9 / 14.1), and the mixed kernels lose (128^3 29.9 / 24.5).
+template <int KS, bool MIXED>
+constexpr int kDepth = KS == 8 && !MIXED ? 2 : 4;
+
 // Products of the wave's pieces (posted for the rows' owners), then of its
 // strips: w and (own_out) the rows' own entries of x to wl and rl (lane's slot of
 // strip k at 64 k), and the sums of own^2, w * own and w^2.  Pieces never
 // wait, and an owner waits only after its own pieces, so every wait ends.
-template <bool EARLY, typename XT>
+template <bool EARLY, int D, typename XT>
 __device__ __forceinline__ void strip_product(const StripSolveArgs &a, const StripWave &w, const XT *__restrict__ x,
                                               unsigned tag, bool v32, bool own_out, double *wl, double *rl,
                                               double (&g)[3]) {
@@ -94,14 +104,14 @@ __device__ __forceinline__ void strip_product(const StripSolveArgs &a, const Str
     const int q1 = __builtin_amdgcn_readfirstlane(a.wave_piece[wid + 1]);
     for (int q = __builtin_amdgcn_readfirstlane(a.wave_piece[wid]); q < q1; ++q) {
       const int pc = __builtin_amdgcn_readfirstlane(a.piece_order[q]);
-      const double v[1] = {piece_sum(S, pc, w.lane, MemVec<XT>{x}, v32)};
+      const double v[1] = {piece_sum<D>(S, pc, w.lane, MemVec<XT>{x}, v32)};
       if (w.lane == 0) mbox_post<1>(a.pmail + 2 * (size_t)pc, tag, v);
     }
   }
   int o = w.lane - 64;
-  strips_run<EARLY>(S, w.lane, MemVec<XT>{x}, v32, w.n, [&](int k) { return w.s0 + k * w.step; },
+  strips_run<EARLY, D>(S, w.lane, MemVec<XT>{x}, v32, w.n, [&](int k) { return w.s0 + k * w.step; },
              [&](int s, const StripDesc &d, int, bool lng, double acc, double own) {
-               if ((d.flags & kStripLong) && lng) acc += take_pieces(a, S.lane_long[64 * s + w.lane], tag);
+               if ((d.flags & kStripLong) && lng) acc += take_pieces<2 * D>(a, S.lane_long[64 * s + w.lane], tag);
                o += 64;
                wl[o] = acc;
                if (own_out) rl[o] = own;
@@ -190,11 +200,11 @@ __device__ __noinline__ void infer_levels(const int *tile_col, InferCtx c, int t
 // needs FP64 ends, and the host starts an FP64 one from its x).
 //
 // Measured on MI355X, us per iteration, FP64 / error bound (streamed tiles with
-// the vectors in memory before): 7-point 128^3 29.3 / 24.7 (54.0 / 45.0), of
-// which the product 15, the update's stores 6.5 and the two synchronisations
-// 7.6; 117 x 89 x 86 13.8 / 15.8 (30.0 / 29.4); 64^3 9.4 / 10.7 (16.7 / 18.7), of
-// which synchronisation 6; 5-point 64^2 5.5 / 6.9 (10.8 / 13.3); 200k-row power
-// law 28.0 / 30.1 (97 / 107).  The 128^3 product moves 40 MB.
+// the vectors in memory before): 7-point 128^3 26.2 / 24.5 (54.0 / 45.0), of
+// which the update's stores 6.5 and the two synchronisations 7.6;
+// 117 x 89 x 86 14.1 / 16.0 (30.0 / 29.4); 64^3 9.3 / 10.7 (16.7 / 18.7), of
+// which synchronisation 6; 5-point 64^2 5.1 / 6.4 (10.8 / 13.3); 200k-row power
+// law 27.5 / 26.4 (97 / 107).  The 128^3 product moves 40 MB.
 //
 // Each round of the
 // loop is one product: of x for a residual (kRes), of r for an iteration
@@ -249,10 +259,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
         full64 = __syncthreads_or(nlev[0] > 0);  // (the block's strips hold these tiles)
         infer = false;
       }
-      strip_product<!MIXED>(a, W, (const float *)a.r32, tag, !full64, true, wl, rl, gd3);
+      strip_product<!MIXED, kDepth<KS, MIXED>>(a, W, (const float *)a.r32, tag, !full64, true, wl, rl, gd3);
     } else {
       const double *v = round == kRes ? a.x : round == kIter ? a.r : a.p;
-      strip_product<!MIXED>(a, W, v, tag, false, true, wl, rl, gd3);
+      strip_product<!MIXED, kDepth<KS, MIXED>>(a, W, v, tag, false, true, wl, rl, gd3);
     }
     if (round == kRes) {
       // r = b - A x of the wave's rows (stored unless it is the last)
@@ -443,9 +453,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
 // one product: of x (kRes), p or s.  A mixed solve that breaks down or
 // stagnates ends, and the host starts an FP64 one from its x.
 //
-// Measured on MI355X, convection-diffusion 100^3, us per iteration: FP64 37.2,
-// error bound 39.3 (tiles with the vectors in memory: 67.8 and 59.7): two
-// products of about 8 us, three sums and two barriers of 15 us together.
+// Measured on MI355X, convection-diffusion 100^3, us per iteration: FP64 32.4,
+// error bound 34.0 (tiles with the vectors in memory: 67.8 and 59.7): two
+// products of about 7 us, three sums and two barriers of 15 us together.
 constexpr int kStripRestarts = 8;
 
 template <int KS, bool MIXED>
@@ -508,10 +518,10 @@ __global__ __launch_bounds__(kBlock) void k_bicgstab_strip(StripSolveArgs a) {
         full64 = __syncthreads_or(nlev[0] > 0);  // (the block's strips hold these tiles)
         infer = false;
       }
-      strip_product<false>(a, W, (const float *)(round == kP ? gp : gs_), tag, !full64, round == kP, wl, rl, gd);
+      strip_product<false, kDepth<KS, MIXED>>(a, W, (const float *)(round == kP ? gp : gs_), tag, !full64, round == kP, wl, rl, gd);
     } else {
       const double *u = round == kRes ? a.x : (const double *)(round == kP ? gp : gs_);
-      strip_product<false>(a, W, u, tag, false, round == kP, wl, rl, gd);
+      strip_product<false, kDepth<KS, MIXED>>(a, W, u, tag, false, round == kP, wl, rl, gd);
     }
     bool step = false;  // go on to p = r + beta (p - omega v)
     bool restart = false;

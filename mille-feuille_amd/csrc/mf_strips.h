@@ -192,14 +192,15 @@ __device__ __forceinline__ double strip_full(const VT *__restrict__ v, const voi
   return acc;
 }
 
-template <bool NEAR, typename VT, class X>
+template <bool NEAR, int D, typename VT, class X>
 __device__ __forceinline__ double strip_full_sum(const VT *__restrict__ v, const void *__restrict__ c, int np,
                                                  int lane, const X &xb, double acc) {
   const uint32_t e = 2u * lane;
   int k = 0;
-  for (; k + 4 <= np; k += 4) acc = strip_full<NEAR, 4>(v, c, e + 128u * k, xb, acc);
+  for (; k + D <= np; k += D) acc = strip_full<NEAR, D>(v, c, e + 128u * k, xb, acc);
   const int rest = np - k;
-  if (rest == 3) return strip_full<NEAR, 3>(v, c, e + 128u * k, xb, acc);
+  if constexpr (D > 3)
+    if (rest == 3) return strip_full<NEAR, 3>(v, c, e + 128u * k, xb, acc);
   if (rest == 2) return strip_full<NEAR, 2>(v, c, e + 128u * k, xb, acc);
   if (rest == 1) return strip_full<NEAR, 1>(v, c, e + 128u * k, xb, acc);
   return acc;
@@ -207,10 +208,11 @@ __device__ __forceinline__ double strip_full_sum(const VT *__restrict__ v, const
 
 // Sum of the lane's entries of a strip or piece (without the lead), added to
 // acc.  X: the vector (MemVec or LdsVec); v32 (FP32 vectors only): full and
-// near strips multiply the FP32 payload.  Strips of more than four pairs load
+// near strips multiply the FP32 payload.  D: pairs in flight.  At four, packed
+// strips of more than four pairs load
 // the next four word pairs before the gathers of the current ones (two
 // buffers in turn: a copy of words in flight would wait for them).
-template <class X>
+template <int D = 4, class X>
 __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc &d, const X &x, int lane,
                                             double acc, bool v32 = false) {
   const int np = d.npair;
@@ -241,6 +243,20 @@ __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc 
       }
       return acc;
     }
+    if constexpr (D < 4) {
+      int k = 0;
+      for (; k + D <= np; k += D) {
+        uint2 a[D];
+        strip_load_words(w, vo + 512u * k, a);
+        acc = strip_packed(a, xb, d.scale, acc);
+      }
+      for (; k < np; ++k) {
+        uint2 a[1];
+        strip_load_words(w, vo + 512u * k, a);
+        acc = strip_packed(a, xb, d.scale, acc);
+      }
+      return acc;
+    }
     uint2 a[4], b[4];
     strip_load_words(w, vo, a);
     int k = 4;
@@ -258,11 +274,11 @@ __device__ __forceinline__ double strip_sum(const StripView &S, const StripDesc 
   const size_t o = (size_t)d.off * 128;
   const X xn = x.rebase((ptrdiff_t)d.base - (1 << 15));
   if (std::is_same<typename X::value, float>::value && v32) {
-    if (d.cls == kStripNear) return strip_full_sum<true>(S.vf + o, S.vh + o, np, lane, xn, acc);
-    return strip_full_sum<false>(S.vf + o, S.vc + o, np, lane, x, acc);
+    if (d.cls == kStripNear) return strip_full_sum<true, D>(S.vf + o, S.vh + o, np, lane, xn, acc);
+    return strip_full_sum<false, D>(S.vf + o, S.vc + o, np, lane, x, acc);
   }
-  if (d.cls == kStripNear) return strip_full_sum<true>(S.vv + o, S.vh + o, np, lane, xn, acc);
-  return strip_full_sum<false>(S.vv + o, S.vc + o, np, lane, x, acc);
+  if (d.cls == kStripNear) return strip_full_sum<true, D>(S.vv + o, S.vh + o, np, lane, xn, acc);
+  return strip_full_sum<false, D>(S.vv + o, S.vc + o, np, lane, x, acc);
 }
 
 // Descriptor i (wave-uniform).
@@ -316,7 +332,7 @@ __device__ __forceinline__ double strip_diag_sum(const StripView &S, const Strip
 // gathers of the current one was slower: with four word pairs a strip always
 // loaded, 128^3 SpMV 17.4 -> 18.9 us, FP64 CG 28.9 -> 34.9 us an iteration.  The
 // waves of a CU hide the two trips; the loads themselves are what counts.)
-template <bool EARLY, class X, class Idx, class F>
+template <bool EARLY, int D = 4, class X, class Idx, class F>
 __device__ __forceinline__ void strips_run(const StripView &S, int lane, const X &x, bool v32, int n, Idx idx, F f) {
 #pragma unroll 1
   for (int k = 0; k < n; ++k) {
@@ -330,15 +346,15 @@ __device__ __forceinline__ void strips_run(const StripView &S, int lane, const X
     double acc = 0.0;
     if ((d.flags & kStripLead) && row >= 0)
       acc = (EARLY && S.leads ? ld : lead()) * own;
-    acc = d.cls == kStripDiag ? strip_diag_sum(S, d, x, row, own, v32, acc) : strip_sum(S, d, x, lane, acc, v32);
+    acc = d.cls == kStripDiag ? strip_diag_sum(S, d, x, row, own, v32, acc) : strip_sum<D>(S, d, x, lane, acc, v32);
     f(s, d, row, lng, acc, own);
   }
 }
 
 // Sum over the wave of a piece's products.
-template <class X>
+template <int D = 4, class X>
 __device__ __forceinline__ double piece_sum(const StripView &S, int piece, int lane, const X &x, bool v32) {
-  return wave_sum(strip_sum(S, strip_desc(S, S.nstrips + piece), x, lane, 0.0, v32));
+  return wave_sum(strip_sum<D>(S, strip_desc(S, S.nstrips + piece), x, lane, 0.0, v32));
 }
 
 }  // namespace mf

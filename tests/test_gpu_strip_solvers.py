@@ -158,3 +158,32 @@ def test_batch_sorted_rows_pieces_and_fallback(mf, oracle, policy, waves, refres
     xs, rep = mf.batch_cg([tm], [b], nrhs=3, tol=TOL, policy=policy, batch_waves=waves, max_refresh=refresh)
     for j in range(3):
         assert oracle.rel_residual(*m, b[j], xs[0][j]) <= TOL
+
+
+@pytest.mark.parametrize("offs", [4, 5, 6, 7, 9])
+@pytest.mark.parametrize("kind", ["packed", "near"])
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+def test_wide_rows_at_eight_strips_a_wave(mf, oracle, offs, kind, method):
+    """Two pairs of entries in flight: every remainder of 4 to 9 pairs."""
+    n, rng = 8150, np.random.default_rng(offs)
+    r, c, v = [np.arange(n)], [np.arange(n)], [rng.uniform(2 * offs + 1, 2 * offs + 2, n)]
+    for o in (1, 2, 3, 17, 64, 65, 200, 901, 3000)[:offs]:
+        i = np.arange(n - o)
+        w = -(2.0 ** -rng.integers(0, 4, n - o)) if kind == "packed" else -rng.uniform(0.1, 1, n - o)
+        r += [i, i + o]
+        c += [i + o, i]
+        v += [w, w]
+    r, c, v = np.concatenate(r), np.concatenate(c), np.concatenate(v)
+    k = np.lexsort((c, r))
+    m = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]).astype(np.int32), c[k].astype(np.int32), v[k]
+    _check(mf, oracle, m, method, blocks=1)
+    y = [_run(mf, m, method, fixed_iters=8, blocks=1, form=f)[3] for f in ("auto", "memory")]
+    assert np.max(np.abs(y[0] - y[1])) <= 1e-9 * np.max(np.abs(y[1]))
+
+
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+def test_pieces_at_eight_strips_a_wave(mf, oracle, method):
+    from millefeuille import gen
+    m = gen.powerlaw_laplacian(8100, 120000, seed=7)
+    tm, _, _ = _check(mf, oracle, m, method, blocks=1)
+    assert tm.strips()["pieces"] > 0

@@ -1699,10 +1699,9 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 
 // Grid-wide deterministic sum of NV values per thread, also a full barrier.
 // Each block writes its NV block sums to partials[slot][block][i] and
-// arrives; once block 0 has seen every arrival and published the barrier,
-// every block reads all the partials and adds them in block order with the
-// same fixed-order tree, so every block gets the same totals without a
-// second broadcast.  The two slots alternate so that storage is never
+// arrives; once it has seen every arrival, every block reads all the partials
+// and adds them in block order with the same fixed-order tree, so every block
+// gets the same totals without a second broadcast.  The two slots alternate so that storage is never
 // reused while a slower block may still read it (two sync points always
 // separate two uses of one slot).  `lds` must hold NV * blockDim.x/64
 // doubles.
@@ -1733,6 +1732,9 @@ __device__ __forceinline__ void grid_sum(double (&v)[NV], double *partials, Grid
     for (int i = 0; i < NV; ++i) s[i] += t[i];
   }
   block_sum_n<NV>(s, lds);
+  // (grid_sum_values writes lds at once: a wave with no rows in between would
+  // overwrite the sums that slower waves of its block still read)
+  lds_barrier();
 #pragma unroll
   for (int i = 0; i < NV; ++i) v[i] = s[i];
   slot ^= 1;

@@ -133,12 +133,14 @@ __device__ __forceinline__ void count_levels(const uint8_t *prec, int t0, int t1
   }
 }
 
-// The wave's strips, and the tiles whose levels it counts and infers.  Unsorted
-// strips go round the waves of their block, so that the block's waves gather
-// from neighbouring rows at the same time (L1; FP64 64^3 9.5 us an iteration
+// The wave's strips, and the tiles whose levels it counts and infers: of
+// unsorted strips, its share of the tiles that the block's strips hold (learned
+// levels are inferred there, and a block with an FP64 tile multiplies FP64); of
+// sorted ones, which no learned solve takes, an equal share of all.
+// Unsorted strips go round the waves of their block, so that the block's waves
+// gather from neighbouring rows at the same time (L1; FP64 64^3 9.5 us an iteration
 // with contiguous strips, now 9.3; error bound 128^3 25.6 and 24.9).  Sorted
 // ones stay contiguous: a window's longest come first.
-template <bool MIXED>
 __device__ __forceinline__ void wave_share(const StripSolveArgs &a, int wid, int lane, StripWave &W, int &t0, int &t1) {
   const int nw = gridDim.x * kWavesPerBlock, wv = wid % kWavesPerBlock;
   W.lane = lane;
@@ -146,15 +148,20 @@ __device__ __forceinline__ void wave_share(const StripSolveArgs &a, int wid, int
     W.s0 = (int)((long long)a.S.nstrips * wid / nw);
     W.step = 1;
     W.n = (int)((long long)a.S.nstrips * (wid + 1) / nw) - W.s0;
+    t0 = (int)((long long)a.A.tilenum * wid / nw);
+    t1 = (int)((long long)a.A.tilenum * (wid + 1) / nw);
   } else {
     const int b = wid / kWavesPerBlock, G = gridDim.x;
     const int b0 = (int)((long long)a.S.nstrips * b / G), b1 = (int)((long long)a.S.nstrips * (b + 1) / G);
     W.s0 = b0 + wv;
     W.step = kWavesPerBlock;
     W.n = max(b1 - W.s0 + kWavesPerBlock - 1, 0) / kWavesPerBlock;
+    // (a strip is four tile-rows)
+    const int u0 = load_uniform(a.A.tile_ptr + min(4 * b0, a.A.tilem));
+    const int u1 = load_uniform(a.A.tile_ptr + min(4 * b1, a.A.tilem));
+    t0 = u0 + (int)((long long)(u1 - u0) * wv / kWavesPerBlock);
+    t1 = u0 + (int)((long long)(u1 - u0) * (wv + 1) / kWavesPerBlock);
   }
-  t0 = (int)((long long)a.A.tilenum * wid / nw);
-  t1 = (int)((long long)a.A.tilenum * (wid + 1) / nw);
 }
 
 // Row of the lane in strip s0 + k.  The lane is hidden from the optimizer,
@@ -221,7 +228,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_strip(StripSolveArgs a) {
   const int lane = threadIdx.x & 63;
   StripWave W;
   int t0, t1;
-  wave_share<MIXED>(a, wid, lane, W, t0, t1);
+  wave_share(a, wid, lane, W, t0, t1);
   auto row_of = [&](int k) { return wave_row(a, W, k); };
   unsigned epoch = 0, tag = 0;
   int slot = 0, lds_i = 0;
@@ -470,7 +477,7 @@ __global__ __launch_bounds__(kBlock) void k_bicgstab_strip(StripSolveArgs a) {
   const int lane = threadIdx.x & 63;
   StripWave W;
   int t0, t1;
-  wave_share<MIXED>(a, wid, lane, W, t0, t1);
+  wave_share(a, wid, lane, W, t0, t1);
   auto row_of = [&](int k) { return wave_row(a, W, k); };
   VT *const gp = MIXED ? (VT *)a.p32 : (VT *)a.p, *const gs_ = MIXED ? (VT *)a.r32 : (VT *)a.r;
   unsigned epoch = 0, tag = 0;

@@ -1442,8 +1442,8 @@ __device__ __forceinline__ void rowgroup_passes(const TileView &A, int tr0, int 
 
 // Learned tile levels for tiles [t0, t1): the MLP runs on 16 tiles per MFMA
 // batch and the levels go to ic.prec_out, where the next per-tile SpMV pass
-// of the same wave reads them (the closing workgroup fence orders the stores
-// before those loads).  Callers infer exactly the tiles their own SpMV reads,
+// of the same wave reads them (a workgroup fence after the last stores orders
+// them before those loads).  Callers infer exactly the tiles their own SpMV reads,
 // so no level is written while another wave may read it.  Returns (alike in
 // every lane) whether any of the tiles changed level; without CMP it does not
 // read the previous levels (a byte's trip through memory in every batch), and
@@ -1490,8 +1490,8 @@ __device__ __forceinline__ bool wave_infer_tiles(const TileView &A, const InferC
   // run as predicted.
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) narrow = min(narrow, __shfl_xor(narrow, m));
-  if (!CMP && __ballot(widest > narrow) == 0) return true;
   __threadfence_block();  // the first pass's level bytes, for every lane
+  if (!CMP && __ballot(widest > narrow) == 0) return true;
   for (int u = t0 + lane; u < t1; u += kWave) {
     const int v = ic.prec_out[u];
     const int cls = v & 15, old = CMP ? v >> 4 : -1;

@@ -137,3 +137,63 @@ def test_grid_sums_order_their_lds_words(tmp_path):
     assert n == 1
     r = _run(tmp_path, PRELUDE + fns + MAIN)
     assert r.returncode == 0, r.stdout
+
+
+INFER = r"""
+#include <algorithm>
+#include <cstdint>
+#include <cstdio>
+using std::max;
+using std::min;
+#define __device__
+#define __forceinline__ inline
+constexpr int kWave = 64, MF_PREC_FP32 = 1, MF_PREC_INT8 = 3, MF_PREC_SKIP = 4;
+static int open_stores;  // level bytes written since the last fence
+static void __threadfence_block() { open_stores = 0; }
+static unsigned long long __ballot(bool v) { return v; }
+static int __shfl_xor(int v, int) { return v; }
+struct Byte {
+  uint8_t v = 0;
+  operator int() const { return v; }
+  Byte &operator=(uint8_t x) { v = x; ++open_stores; return *this; }
+};
+struct TileView { const int *tile_col; };
+struct InferCtx { const int *w; Byte *prec_out; };
+struct MlpRegs {};
+typedef int half4_t;
+typedef int float4_t;
+static const int *classes;
+static void mlp_load(const int *, int, MlpRegs &) {}
+static half4_t infer_features(const InferCtx &, int t, int, int, bool) { return t; }
+static float4_t mlp_eval16r(const MlpRegs &, half4_t t) { return classes[t]; }
+static int mlp_argmax(float4_t c) { return c; }
+"""
+
+INFER_MAIN = r"""
+template <bool CMP> int check(const int *cls, int n) {
+  Byte prec[64];
+  for (int t = 0; t < n; ++t) prec[t].v = 1;
+  classes = cls;
+  open_stores = 0;
+  wave_infer_tiles<CMP>(TileView{nullptr}, InferCtx{nullptr, prec}, 0, n, 0);
+  return open_stores;
+}
+int main() {
+  int same[64], mixed[64], wide[64], bad = 0;
+  for (int t = 0; t < 64; ++t) { same[t] = 2; mixed[t] = 1 + t / 16 % 3; wide[t] = 0; }
+  for (const int *c : {same, mixed, wide})
+    for (int n : {1, 17, 64}) {
+      bad += check<true>(c, n) != 0;
+      bad += check<false>(c, n) != 0;
+    }
+  std::printf("%d returns with unfenced level stores\n", bad);
+  return bad != 0;
+}
+"""
+
+
+def test_inferred_levels_are_fenced_before_their_reader(tmp_path):
+    """The lanes that store a wave's levels are not those that read them."""
+    text = open(HEADER).read()
+    r = _run(tmp_path, INFER + _function(text, "wave_infer_tiles") + INFER_MAIN)
+    assert r.returncode == 0, r.stdout

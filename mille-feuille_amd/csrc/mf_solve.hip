@@ -1651,10 +1651,15 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
   double stats[kStCount];
   mf_status ret = MF_OK;
   bool mixed = opt.policy != MF_POLICY_FP64 && !before;
+  // What a fallback leaves of the caller's limits.  At least one iteration:
+  // BiCGSTAB counts the step that failed, so none may seem to be left.
+  auto go_on = [&] {
+    a.maxiter = std::max(opt.maxiter - r.iterations, 1);
+    if (opt.fixed_iters > 0) a.fixed_iters = std::max(opt.fixed_iters - r.iterations, 1);
+  };
   if (before) {
     r = *before;
-    a.maxiter -= r.iterations;
-    if (opt.fixed_iters > 0) a.fixed_iters -= r.iterations;
+    go_on();
   }
   for (;;) {
     if (ret == MF_OK) ret = fill_u32(z0, (size_t)(z1 - z0), 0u, st);
@@ -1691,12 +1696,7 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
     // FP64 from the x that the mixed solve reached
     mixed = false;
     r.fell_back = 1;
-    a.maxiter = opt.maxiter - r.iterations;
-    if (a.maxiter <= 0) {
-      stats[kStStatus] = MF_NOT_CONVERGED;
-      break;
-    }
-    if (opt.fixed_iters > 0) a.fixed_iters = opt.fixed_iters - r.iterations;
+    go_on();
   }
   if (e0) {
     float ms = 0.0f;
@@ -1944,9 +1944,7 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   r.form_used = resident_windows ? MF_FORM_RESIDENT : MF_FORM_MEMORY;
   r.policy_used = opt.policy;
   int ret = status;
-  if (a.stop64 && r.fell_back && status == MF_OK && r.iterations < opt.maxiter &&
-      !(opt.fixed_iters <= 0 && r.rel_residual <= opt.tol) &&
-      !(opt.fixed_iters > 0 && r.iterations >= opt.fixed_iters))
+  if (a.stop64 && r.fell_back && status == MF_OK && !(opt.fixed_iters <= 0 && r.rel_residual <= opt.tol))
     return run_strips(t, d_b, d_x, opt, rep, G64, bicg, noalloc, &r);
   if (ret == MF_OK && opt.fixed_iters <= 0 && !(r.rel_residual <= opt.tol)) ret = MF_NOT_CONVERGED;
   r.status = ret;

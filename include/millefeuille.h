@@ -287,6 +287,8 @@ typedef struct mf_report {
   int form_used;        /* MF_FORM_MEMORY or MF_FORM_RESIDENT */
   int policy_used;      /* MF_POLICY_* that ran (LEARNED without an installed
                            MLP runs the rule policy) */
+  int strips_per_wave;  /* most row strips that a wave of the solve's last
+                           kernel held; 0: that kernel ran over tiles */
 } mf_report;
 
 void mf_solve_opts_default(mf_solve_opts *o);

@@ -25,6 +25,7 @@
 #include <mutex>
 #include <string>
 #include <cmath>
+#include <cstddef>
 #include <cstdlib>
 #include <cstring>
 #include <cstdio>
@@ -1715,6 +1716,7 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
     r.form_used = MF_FORM_RESIDENT;
     r.policy_used = opt.policy;
   }
+  r.strips_per_wave = per;
   ret = (int)stats[kStStatus];
   if (ret == MF_OK && opt.fixed_iters <= 0 && !(r.rel_residual <= opt.tol)) ret = MF_NOT_CONVERGED;
   r.status = ret;
@@ -1723,6 +1725,10 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
   if (ret == MF_NOT_CONVERGED) set_error("solve: tolerance not reached");
   return ret;
 }
+
+// (strips_per_wave lies in what was the report's tail padding, so a caller built
+// without it has room for it)
+static_assert(sizeof(mf_report) == 96 && offsetof(mf_report, strips_per_wave) == 92, "report layout");
 
 mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_solve_opts *o,
                          mf_report *rep, bool bicg, bool noalloc = false) {

@@ -59,7 +59,7 @@ class MfReport(C.Structure):
                 ("status", C.c_int), ("rel_residual", C.c_double),
                 ("rel_residual_recursive", C.c_double), ("time_ms", C.c_double),
                 ("prec_hist", C.c_longlong * 5), ("grid_blocks", C.c_int),
-                ("form_used", C.c_int), ("policy_used", C.c_int)]
+                ("form_used", C.c_int), ("policy_used", C.c_int), ("strips_per_wave", C.c_int)]
 
     def as_dict(self):
         return {"iterations": self.iterations, "refreshes": self.refreshes,
@@ -68,7 +68,7 @@ class MfReport(C.Structure):
                 "rel_residual_recursive": self.rel_residual_recursive,
                 "time_ms": self.time_ms, "prec_hist": list(self.prec_hist),
                 "grid_blocks": self.grid_blocks, "form_used": self.form_used,
-                "policy_used": self.policy_used}
+                "policy_used": self.policy_used, "strips_per_wave": self.strips_per_wave}
 
 
 class MfTuneReport(C.Structure):

@@ -61,9 +61,14 @@ class Slab {
     parts_.push_back({(void **)p, bytes_});
     bytes_ += (n * sizeof(T) + 255) & ~(size_t)255;
   }
+  hipError_t try_alloc(void **base) {
+    const hipError_t e = hipMalloc(base, bytes_ > 0 ? bytes_ : 256);
+    if (e == hipSuccess)
+      for (auto &q : parts_) *q.first = (char *)*base + q.second;
+    return e;
+  }
   mf_status alloc(void **base) {
-    MF_HIP(hipMalloc(base, bytes_ > 0 ? bytes_ : 256));
-    for (auto &q : parts_) *q.first = (char *)*base + q.second;
+    MF_HIP(try_alloc(base));
     return MF_OK;
   }
 

@@ -333,7 +333,17 @@ int64_t strip_bytes(const StripLayout &L) {
   return b;
 }
 
-mf_status build_strips(mf_tiled *t, const int *rowptr) {
+// (no_memory: an allocation failed for want of memory, with MF_OK returned)
+static mf_status make_strips(mf_tiled *t, const int *rowptr, bool &no_memory) {
+  auto alloc = [&](Slab &s, void **base) {
+    const hipError_t e = s.try_alloc(base);
+    if (e == hipSuccess) return MF_OK;
+    *base = nullptr;
+    if (e != hipErrorOutOfMemory) return fail(MF_ERR_HIP, std::string("build_strips: ") + hipGetErrorString(e));
+    (void)hipGetLastError();
+    no_memory = true;
+    return MF_OK;
+  };
   StripLayout &L = t->strips;
   const int rows = t->rowA;
   if (rows == 0 || t->tilenum == 0) return MF_OK;
@@ -348,7 +358,8 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
     void *mem = nullptr;
     both.add(&d, rows);
     both.add(&nd, nstrips);
-    MF_TRY(both.alloc(&mem));
+    MF_TRY(alloc(both, &mem));
+    if (no_memory) return MF_OK;
     k_row_info<<<(rows + 3) / 4, 256>>>(A, rows, d);
     k_diag_slots<false><<<(nstrips + 3) / 4, 256>>>(A, rows, nstrips, nd, nullptr, nullptr, nullptr, nullptr);
     hipError_t e = hipGetLastError();
@@ -390,7 +401,10 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
   tmp.add(&d_safe, P.safe.size());
   if (P.sorted) tmp.add(&d_slot, P.slot.size());
   if (L.nlong > 0) tmp.add(&d_long, P.long_of.size());
-  MF_TRY(slab.alloc(&L.slab));
+  void *scratch = nullptr;  // temporaries of the fill
+  MF_TRY(alloc(slab, &L.slab));
+  if (!no_memory) MF_TRY(alloc(tmp, &scratch));
+  if (no_memory) return MF_OK;
   MF_HIP(hipMemset(L.lead64, 0, sizeof(double) * 64 * (size_t)nstr));
   MF_HIP(hipMemset(L.lead32, 0, sizeof(float) * 64 * (size_t)nstr));
   if (nf > 0) {
@@ -399,9 +413,6 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
     if (L.vc) MF_HIP(hipMemset(L.vc, 0xff, sizeof(int) * 128 * nf));
     if (L.vh) MF_HIP(hipMemset(L.vh, 0, sizeof(uint16_t) * 128 * nf));
   }
-  // temporaries of the fill
-  void *scratch = nullptr;
-  MF_TRY(tmp.alloc(&scratch));
   mf_status st = upload(L.desc, P.desc);
   if (st == MF_OK) st = upload(d_safe, P.safe);
   if (st == MF_OK && P.sorted) st = upload(L.rowmap, P.rowmap);
@@ -424,6 +435,14 @@ mf_status build_strips(mf_tiled *t, const int *rowptr) {
   }
   (void)hipFree(scratch);
   if (st == MF_OK) L.nstrips = nstr;
+  return st;
+}
+
+// Without memory for them a handle has no strips and runs on its tiles.
+mf_status build_strips(mf_tiled *t, const int *rowptr) {
+  bool no_memory = false;
+  const mf_status st = make_strips(t, rowptr, no_memory);
+  if (no_memory) free_strips(t);
   return st;
 }
 

@@ -1,0 +1,101 @@
+"""The library's host code on the CPU, over a stand-in for the HIP runtime
+(fake_hip.cpp): allocation failures, which kernels are launched, what lives how
+long.  Each snippet runs in a process of its own."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, sys
+fake = C.CDLL({shim!r}, mode=C.RTLD_GLOBAL)
+fake.fake_log.restype = C.c_char_p
+fake.fake_in_use.restype = C.c_size_t
+fake.fake_budget.argtypes = [C.c_size_t]
+fake.fake_cost.argtypes = [C.c_char_p, C.c_float]
+sys.path[:0] = [{pkg!r}]
+import numpy as np
+import millefeuille as mf
+from millefeuille import gen
+from millefeuille._lib import lib, MfReport, MfSolveOpts, MfTuneReport
+
+ALL = 2 ** 64 - 1
+
+def log():
+    out = fake.fake_log().decode().splitlines()
+    fake.fake_clear()
+    return out
+
+def launched(name):
+    return [l for l in log() if l.startswith("launch mf::" + name)]
+
+class Vec:  # a device array
+    def __init__(self, n):
+        self.a = np.zeros(n)
+        self.ptr = self.a.ctypes.data
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    d = tmp_path_factory.mktemp("fake_hip")
+    shim = str(d / "libfakehip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", shim, os.path.join(HERE, "fake_hip.cpp")],
+                   check=True)
+    prelude = PRELUDE.format(shim=shim, pkg=os.path.join(ROOT, "mille-feuille_amd"))
+
+    def go(body):
+        env = dict(os.environ, MALLOC_PERTURB_="165")  # freed memory is overwritten
+        r = subprocess.run([sys.executable, "-c", prelude + textwrap.dedent(body)], capture_output=True, text=True,
+                           env=env)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+    return go
+
+
+def test_handles_without_room_for_strips_run_on_tiles(run):
+    """Every budget from nothing to all: either the tiles do not fit and the
+    creation fails, or there is a handle, with strips if they fit too."""
+    run("""
+    m = gen.laplace3d(12)
+    tm = mf.TiledMatrix(*m)
+    full = fake.fake_in_use()
+    assert tm.strips()["strips"] > 0
+    tm.free()
+    assert fake.fake_in_use() == 0
+    sizes = [int(l.split()[1]) for l in log() if l.startswith("malloc")]
+    made = failed = without = 0
+    for budget in range(0, sum(sizes), 4096):
+        fake.fake_budget(budget)
+        try:
+            tm = mf.TiledMatrix(*m)
+        except mf.MfError as e:
+            assert e.code == -4, e  # MF_ERR_HIP
+            assert made == 0, "a larger budget failed"
+            failed += 1
+            assert fake.fake_in_use() == 0
+            continue
+        made += 1
+        if tm.strips()["strips"] == 0:
+            without += 1
+            fake.fake_budget(ALL)
+            log()
+            x, y = Vec(tm.npad), Vec(tm.npad)
+            tm.spmv(x, y)
+            assert launched("k_spmv<")
+            tm.cg(x, y)
+            assert launched("k_cg<")
+            try:
+                tm.set_spmv_kernel("strip")
+                assert False
+            except mf.MfError as e:
+                assert e.code == -1
+        tm.free()
+        assert fake.fake_in_use() == 0
+    assert failed and without and made > without, (failed, without, made)
+    """)

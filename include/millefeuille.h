@@ -191,6 +191,8 @@ mf_status mf_spmv(mf_tiled *t, const double *d_x, const float *d_x32,
 #define MF_SPMV_ROWGROUP 1
 #define MF_SPMV_STRIP 2
 mf_status mf_tile_set_spmv_kernel(mf_tiled *t, int kind);
+/* Kernel that mf_spmv launches for `mode` (0 or 1). */
+mf_status mf_tile_get_spmv_kernel(const mf_tiled *t, int mode, int *kind);
 
 /* Sizes of a device handle's row strips: strips of 64 rows (0: the handle has
  * none), pieces of rows too long for a strip, whether rows are sorted by

@@ -54,7 +54,8 @@ struct DeviceLayout {
   uint8_t *rc = nullptr;       // npay (+pad): (row << 4) | col inside the tile
   uint8_t *rp16 = nullptr;     // 16*tilenum: row starts inside each tile
   int max_tiles_per_row = 0;   // largest tile count of a tile-row
-  int spmv_kernel = 0;         // MF_SPMV_STREAM or MF_SPMV_ROWGROUP
+  int spmv_kernel = 0;         // MF_SPMV_* of mode 0 ...
+  int spmv_level_kernel = 0;   // ... and of mode 1 (MF_SPMV_STREAM or MF_SPMV_ROWGROUP)
   double *v64 = nullptr;       // npay FP64 payload
   float *v32 = nullptr;        // npay FP32 payload
   uint16_t *v16 = nullptr;     // npay FP16 payload (bits), scaled by s16

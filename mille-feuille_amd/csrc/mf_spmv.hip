@@ -67,9 +67,10 @@ mf_status launch_spmv_strip(const mf_tiled *t, const double *d_x, double *d_y, h
 mf_status launch_spmv(const mf_tiled *t, const double *d_x, const float *d_x32, double *d_y,
                       int mode, hipStream_t s) {
   const TileView A = view_of(t);
-  if (mode == kAll64 && t->dev.spmv_kernel == MF_SPMV_STRIP) {
+  const int kind = mode == kAll64 ? t->dev.spmv_kernel : t->dev.spmv_level_kernel;
+  if (kind == MF_SPMV_STRIP) {
     MF_TRY(launch_spmv_strip(t, d_x, d_y, s));
-  } else if (t->dev.spmv_kernel == MF_SPMV_ROWGROUP) {
+  } else if (kind == MF_SPMV_ROWGROUP) {
     const int nwv = (A.tilem + 3) / 4;
     const int blocks = ((nwv + 3) / 4 + 7) / 8 * 8;
     if (A.tilem > 0) {
@@ -145,6 +146,14 @@ extern "C" mf_status mf_tile_set_spmv_kernel(mf_tiled *t, int kind) {
   if (kind != MF_SPMV_STREAM && kind != MF_SPMV_ROWGROUP && kind != MF_SPMV_STRIP)
     return fail(MF_ERR_ARG, "mf_tile_set_spmv_kernel: unknown kernel");
   t->dev.spmv_kernel = kind;
+  t->dev.spmv_level_kernel = kind == MF_SPMV_STRIP ? MF_SPMV_STREAM : kind;
+  return MF_OK;
+}
+
+extern "C" mf_status mf_tile_get_spmv_kernel(const mf_tiled *t, int mode, int *kind) {
+  if (!t || !kind) return fail(MF_ERR_ARG, "mf_tile_get_spmv_kernel: null argument");
+  if (mode != kAll64 && mode != kPerTile) return fail(MF_ERR_ARG, "mf_tile_get_spmv_kernel: bad mode");
+  *kind = mode == kAll64 ? t->dev.spmv_kernel : t->dev.spmv_level_kernel;
   return MF_OK;
 }
 

@@ -78,7 +78,11 @@ extern "C" mf_status mf_tune_spmv(mf_tiled *t, int mode, mf_tune_report *rep) {
   MF_TRY(buf.alloc((void **)&x32, sizeof(float) * np));
   MF_HIP(hipMemset(x, 0, sizeof(double) * np));
   MF_HIP(hipMemset(x32, 0, sizeof(float) * np));
-  const int old_nnz = t->dev.spmv_wave_nnz, old_kernel = t->dev.spmv_kernel;
+  const int old_nnz = t->dev.spmv_wave_nnz, old_kernel = t->dev.spmv_kernel, old_level = t->dev.spmv_level_kernel;
+  auto use = [&](int kernel, int level) {
+    t->dev.spmv_kernel = kernel;
+    t->dev.spmv_level_kernel = level;
+  };
   std::vector<int> cand = {384, 512, 768, 1024, 1536, 2048};
   if (regular_tilerows(t)) cand.push_back(0);
   if (mode == kAll64 && t->strips.nstrips > 0) cand.push_back(-1);
@@ -89,15 +93,15 @@ extern "C" mf_status mf_tune_spmv(mf_tiled *t, int mode, mf_tune_report *rep) {
   for (size_t i = 0; i < cand.size(); ++i) {
     if (cand[i] > 0) {
       MF_TRY(mf_tile_set_schedule(t, cand[i]));
-      t->dev.spmv_kernel = MF_SPMV_STREAM;
+      use(MF_SPMV_STREAM, MF_SPMV_STREAM);
     } else {
-      t->dev.spmv_kernel = cand[i] < 0 ? MF_SPMV_STRIP : MF_SPMV_ROWGROUP;
+      use(cand[i] < 0 ? MF_SPMV_STRIP : MF_SPMV_ROWGROUP, MF_SPMV_ROWGROUP);
     }
     float us = 0.0f;
     const mf_status st = time_median([&] { return mf_spmv(t, x, x32, y, mode, nullptr); }, 5, 25, &us);
     if (st != MF_OK) {
       (void)mf_tile_set_schedule(t, old_nnz);
-      t->dev.spmv_kernel = old_kernel;
+      use(old_kernel, old_level);
       return st;
     }
     rep->cand[i] = cand[i];
@@ -108,14 +112,11 @@ extern "C" mf_status mf_tune_spmv(mf_tiled *t, int mode, mf_tune_report *rep) {
     }
   }
   rep->best = cand[bi];
-  if (cand[bi] > 0) {
-    MF_TRY(mf_tile_set_schedule(t, cand[bi]));
-    // (mode 1 of a handle on strips runs the streamed kernel already)
-    t->dev.spmv_kernel = mode == kPerTile && old_kernel == MF_SPMV_STRIP ? MF_SPMV_STRIP : MF_SPMV_STREAM;
-  } else {
-    MF_TRY(mf_tile_set_schedule(t, old_nnz));
-    t->dev.spmv_kernel = cand[bi] < 0 ? MF_SPMV_STRIP : MF_SPMV_ROWGROUP;
-  }
+  MF_TRY(mf_tile_set_schedule(t, cand[bi] > 0 ? cand[bi] : old_nnz));
+  // Strips are mode 0's alone: the choice for one mode leaves the other's
+  // kernel where strips are on either side of it, else it holds for both.
+  const int k = cand[bi] > 0 ? MF_SPMV_STREAM : cand[bi] < 0 ? MF_SPMV_STRIP : MF_SPMV_ROWGROUP;
+  use(mode == kPerTile && old_kernel == MF_SPMV_STRIP ? MF_SPMV_STRIP : k, k == MF_SPMV_STRIP ? old_level : k);
   return MF_OK;
 }
 

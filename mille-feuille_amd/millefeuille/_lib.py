@@ -118,6 +118,7 @@ SIGNATURES = {
     "mf_stream_copy": (C.c_int, [_vp, _vp, C.c_int64, _vp]),
     "mf_tile_set_schedule": (C.c_int, [_vp, C.c_int]),
     "mf_tile_set_spmv_kernel": (C.c_int, [_vp, C.c_int]),
+    "mf_tile_get_spmv_kernel": (C.c_int, [_vp, C.c_int, _ip]),
     "mf_tile_strip_info": (C.c_int, [_vp, _ip, _ip, _ip] + [C.POINTER(C.c_int64)] * 4 + [_ip]),
     "mf_solve_opts_default": (None, [C.POINTER(MfSolveOpts)]),
     "mf_cg_solve": (C.c_int, [_vp, _vp, _vp, C.POINTER(MfSolveOpts), C.POINTER(MfReport)]),

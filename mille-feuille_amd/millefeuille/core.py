@@ -75,7 +75,6 @@ class TiledMatrix:
         vals = [C.c_int() for _ in range(6)]
         check("mf_tile_info", lib.mf_tile_info(h, *[C.byref(v) for v in vals]))
         self.tilem, self.tilen, self.tilenum, self.csrsize, self.csrptrlen, self.npad = [v.value for v in vals]
-        self._spmv_kernel = _lib.SPMV_AUTO
 
     def free(self):
         if getattr(self, "h", None):
@@ -168,8 +167,6 @@ class TiledMatrix:
         check("mf_tile_set_schedule", lib.mf_tile_set_schedule(self.h, int(spmv_wave_nnz)))
         if int(spmv_wave_nnz) > 0:
             self._wave_nnz = int(spmv_wave_nnz)
-            if self._spmv_kernel not in (_lib.SPMV_STREAM, _lib.SPMV_ROWGROUP):
-                self._spmv_kernel = _lib.SPMV_STREAM  # as the library does
 
     def tune_spmv(self, mode=0):
         """Autotunes the stand-alone SpMV (mf_tune_spmv) for `mode` at the
@@ -178,13 +175,15 @@ class TiledMatrix:
         rep = _lib.MfTuneReport()
         check("mf_tune_spmv", lib.mf_tune_spmv(self.h, int(mode), C.byref(rep)))
         d = rep.as_dict()
-        if d["best"] <= 0:
-            self._spmv_kernel = _lib.SPMV_ROWGROUP if d["best"] == 0 else _lib.SPMV_STRIP
-        elif int(mode) == 0 or self._spmv_kernel == _lib.SPMV_ROWGROUP:
-            self._spmv_kernel = _lib.SPMV_STREAM
         if d["best"] > 0:
             self._wave_nnz = int(d["best"])
         return d
+
+    def spmv_kernel(self, mode=0):
+        """SPMV_* kernel that spmv launches for `mode` (mf_tile_get_spmv_kernel)."""
+        k = C.c_int()
+        check("mf_tile_get_spmv_kernel", lib.mf_tile_get_spmv_kernel(self.h, int(mode), C.byref(k)))
+        return k.value
 
     def spmv_kernel_name(self):
         """Device kernel that mf_spmv launches for this handle (mode 0): the
@@ -192,11 +191,11 @@ class TiledMatrix:
         long rows), or the streamed one, instantiated with piece bookkeeping
         when a tile-row holds more than 4*max(wave_nnz, 4096) padded payload
         slots (the library's heavy tile-row rule)."""
-        if self._spmv_kernel == _lib.SPMV_ROWGROUP:
+        kind = self.spmv_kernel()
+        if kind == _lib.SPMV_ROWGROUP:
             return "mf::k_spmv_rg<0>"
-        d = self.strips()
-        if self._spmv_kernel == _lib.SPMV_STRIP or (d["lean"] and self._spmv_kernel == _lib.SPMV_AUTO):
-            return f"mf::k_spmv_strip<{'true' if d['pieces'] else 'false'}>"
+        if kind == _lib.SPMV_STRIP:
+            return f"mf::k_spmv_strip<{'true' if self.strips()['pieces'] else 'false'}>"
         a = self.arrays()
         slots = (np.diff(a["csr_offset"]).astype(np.int64) + 3) // 4 * 4
         pre = np.concatenate([[0], np.cumsum(slots)])
@@ -221,7 +220,6 @@ class TiledMatrix:
              "strip": _lib.SPMV_STRIP}
         kind = k.get(kind, kind)
         check("mf_tile_set_spmv_kernel", lib.mf_tile_set_spmv_kernel(self.h, kind))
-        self._spmv_kernel = kind
 
     def get_precision(self):
         out = np.zeros(max(self.tilenum, 1), np.uint8)

@@ -64,12 +64,14 @@ void __hipRegisterFunction(void **, const void *f, char *, const char *name, uns
   std::string s = d && !st ? d : name;
   std::free(d);
   if (s.rfind("void ", 0) == 0) s = s.substr(5);
+  const std::string anon = "(anonymous namespace)::";
+  for (size_t i; (i = s.find(anon)) != std::string::npos;) s.erase(i, anon.size());
   // the arguments' list, after the template's
   int depth = 0;
   for (size_t i = 0; i < s.size(); ++i) {
     if (s[i] == '<') ++depth;
     if (s[i] == '>') --depth;
-    if (s[i] == '(' && depth == 0 && s.compare(i, 11, "(anonymous ") != 0) { s = s.substr(0, i); break; }
+    if (s[i] == '(' && depth == 0) { s = s.substr(0, i); break; }
   }
   for (size_t i; (i = s.find(' ')) != std::string::npos;) s.erase(i, 1);
   names[f] = s;

@@ -99,3 +99,33 @@ def test_handles_without_room_for_strips_run_on_tiles(run):
         assert fake.fake_in_use() == 0
     assert failed and without and made > without, (failed, without, made)
     """)
+
+
+def test_tuning_one_mode_leaves_strips_to_the_other(run):
+    """The stand-in's event times make the row-group kernel, then the strip
+    kernel, then the streamed one the fastest candidate."""
+    run("""
+    tm = mf.TiledMatrix(*gen.laplace3d(12))
+    tm.set_spmv_kernel("strip")
+    x, y, x32 = Vec(tm.npad), Vec(tm.npad), Vec(tm.npad)
+
+    def kernels():
+        log()
+        tm.spmv(x, y)
+        tm.spmv(x, y, mode=1, d_x32=x32)
+        return [l.split()[1] for l in log() if l.startswith("launch")]
+
+    assert kernels() == ["mf::k_spmv_strip<false>", "mf::k_spmv<1,false>"], kernels()
+    fake.fake_cost(b"k_spmv_rg", 0.5)
+    assert tm.tune_spmv(mode=1)["best"] == 0
+    assert kernels() == ["mf::k_spmv_strip<false>", "mf::k_spmv_rg<1>"], kernels()
+    fake.fake_cost(b"k_spmv_strip", 0.25)
+    assert tm.tune_spmv(mode=0)["best"] == -1
+    assert kernels() == ["mf::k_spmv_strip<false>", "mf::k_spmv_rg<1>"], kernels()
+    fake.fake_cost(b"k_spmv<", 0.125)
+    assert tm.tune_spmv(mode=1)["best"] > 0
+    assert kernels() == ["mf::k_spmv_strip<false>", "mf::k_spmv<1,false>"], kernels()
+    assert tm.tune_spmv(mode=0)["best"] > 0
+    assert kernels() == ["mf::k_spmv<0,false>", "mf::k_spmv<1,false>"], kernels()
+    assert tm.spmv_kernel() == tm.spmv_kernel(1) == mf._lib.SPMV_STREAM
+    """)

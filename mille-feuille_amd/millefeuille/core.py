@@ -307,6 +307,7 @@ def batch_cg(systems, bs, nrhs=1, x0=None, allow_not_converged=False, tune_iters
     iterations, relative residuals, per-system and total ms (and the tuner's
     timings under "tune")."""
     opts = solve_opts(**kw)
+    systems, bs = list(systems), list(bs)
     nsys = len(systems)
     # one device array each for the right-hand sides and the solutions, the
     # systems one after another (a pair of allocations and copies per system

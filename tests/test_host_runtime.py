@@ -129,3 +129,39 @@ def test_tuning_one_mode_leaves_strips_to_the_other(run):
     assert kernels() == ["mf::k_spmv<0,false>", "mf::k_spmv<1,false>"], kernels()
     assert tm.spmv_kernel() == tm.spmv_kernel(1) == mf._lib.SPMV_STREAM
     """)
+
+
+def test_batch_takes_any_iterable_of_right_hand_sides(run):
+    run("""
+    from millefeuille import core
+
+    class Dev(Vec):
+        made = []
+
+        def __init__(self, n, dtype=np.float64):
+            super().__init__(n)
+            Dev.made.append(self)
+
+        @classmethod
+        def from_host(cls, a, dtype=None, length=None):
+            d = cls(len(a))
+            d.a[:] = a
+            return d
+
+        def zero(self):
+            self.a[:] = 0
+
+        def get(self, n=None):
+            return self.a.copy()
+
+    core.DeviceArray = Dev
+    tms = [mf.TiledMatrix(*gen.laplace2d(e)) for e in (5, 8)]
+    bs = [np.arange(2 * t.rowA).reshape(2, -1) + 1.0 for t in tms]
+    want = None
+    for v in (bs, tuple(bs), (b for b in bs), iter(bs), map(np.asarray, bs), {k: b for k, b in enumerate(bs)}.values()):
+        Dev.made.clear()
+        xs, rep = mf.batch_cg(tms, v, nrhs=2, allow_not_converged=True)
+        assert [x.shape for x in xs] == [(2, 25), (2, 64)]
+        want = Dev.made[0].a if want is None else want
+        np.testing.assert_array_equal(Dev.made[0].a, want)
+    """)

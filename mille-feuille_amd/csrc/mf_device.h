@@ -77,6 +77,12 @@ class Slab {
   std::vector<std::pair<void **, size_t>> parts_;
 };
 
+// y = A x by the handle's kernel for `mode` (mf_spmv.hip).  stateless: by one that
+// writes nothing but y, so that a product of the handle on another stream may
+// run at the same time.
+mf_status launch_spmv(const mf_tiled *t, const double *d_x, const float *d_x32, double *d_y, int mode, hipStream_t s,
+                      bool stateless = false);
+
 inline TileView view_of(const mf_tiled *t) {
   const DeviceLayout &d = t->dev;
   return TileView{d.tile_ptr, d.tile_col, d.tile_off, d.tile_row, d.tile_nz, d.rc, d.rp16,

@@ -30,8 +30,6 @@ using namespace mf;
 
 namespace mf {
 
-mf_status launch_spmv(const mf_tiled *t, const double *d_x, const float *d_x32, double *d_y, int mode, hipStream_t s);
-
 constexpr int kGS = 128;                 // samples per gradient block (= threads)
 constexpr int kGSP = kGS + 1;            // padded LDS row (no bank conflicts)
 constexpr int kPartial = kMlpParams + 1; // gradient partials + loss per block
@@ -632,7 +630,7 @@ extern "C" mf_status mf_policy_labels(mf_tiled *t, const double *d_p, double the
   double *y = (double *)w, *part = y + t->dev.npad, *sum = part + kSqBlocks;
   double w2 = 0.0;
   if (n > 0) {
-    MF_TRY(launch_spmv(t, d_p, nullptr, y, kAll64, st));
+    MF_TRY(launch_spmv(t, d_p, nullptr, y, kAll64, st, true));
     k_sum_squares<<<kSqBlocks, 256, 0, st>>>(y, n, part);
     k_sum_one_block<<<1, 1024, 0, st>>>(part, kSqBlocks, sum);
     MF_HIP(hipGetLastError());

@@ -12,9 +12,6 @@
 
 namespace mf {
 
-mf_status launch_spmv(const mf_tiled *t, const double *d_x, const float *d_x32, double *d_y,
-                      int mode, hipStream_t s);
-
 namespace {
 
 constexpr int kDotBlocks = 1024;

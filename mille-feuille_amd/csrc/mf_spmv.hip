@@ -65,9 +65,12 @@ __global__ void k_zero_tail(double *y, int from, int to) {
 mf_status launch_spmv_strip(const mf_tiled *t, const double *d_x, double *d_y, hipStream_t s);
 
 mf_status launch_spmv(const mf_tiled *t, const double *d_x, const float *d_x32, double *d_y,
-                      int mode, hipStream_t s) {
+                      int mode, hipStream_t s, bool stateless) {
   const TileView A = view_of(t);
-  const int kind = mode == kAll64 ? t->dev.spmv_kernel : t->dev.spmv_level_kernel;
+  int kind = mode == kAll64 ? t->dev.spmv_kernel : t->dev.spmv_level_kernel;
+  // (the streamed kernel counts the pieces of heavy tile-rows in the handle)
+  if (stateless && kind == MF_SPMV_STREAM && t->dev.spmv_nheavy > 0)
+    kind = mode == kAll64 && t->strips.nstrips > 0 ? MF_SPMV_STRIP : MF_SPMV_ROWGROUP;
   if (kind == MF_SPMV_STRIP) {
     MF_TRY(launch_spmv_strip(t, d_x, d_y, s));
   } else if (kind == MF_SPMV_ROWGROUP) {

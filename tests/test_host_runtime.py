@@ -165,3 +165,28 @@ def test_batch_takes_any_iterable_of_right_hand_sides(run):
         want = Dev.made[0].a if want is None else want
         np.testing.assert_array_equal(Dev.made[0].a, want)
     """)
+
+
+def test_policy_labels_share_no_state_with_products(run):
+    """A product on another stream may be under way: the labels' own product is
+    not the streamed kernel's form that counts pieces in the handle."""
+    run("""
+    from millefeuille import policy
+    n = 20000
+    r = np.concatenate([np.zeros(n - 1, np.int64), np.arange(1, n), np.arange(n)])
+    c = np.concatenate([np.arange(1, n), np.zeros(n - 1, np.int64), np.arange(n)])
+    k = np.lexsort((c, r))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]).astype(np.int32)
+    tm = mf.TiledMatrix(rp, c[k].astype(np.int32), np.ones(len(k)))
+    x, y, lab = Vec(tm.npad), Vec(tm.npad), Vec(tm.tilenum)
+    for kernel in ("auto", "stream", "strip", "rowgroup"):
+        tm.set_spmv_kernel(kernel)
+        log()
+        assert lib.mf_policy_labels(tm.h, x.ptr, 1e-5, lab.ptr, None) == 0
+        l = log()
+        assert any("launch mf::k_labels" in q for q in l)
+        assert any("k_spmv_" in q for q in l) and not any("k_spmv<" in q for q in l), l
+    tm.set_spmv_kernel("stream")
+    tm.spmv(x, y)
+    assert launched("k_spmv<0,true>")
+    """)

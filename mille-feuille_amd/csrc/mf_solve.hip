@@ -1559,13 +1559,13 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
   const size_t n = t->dev.npad, rows = 16 * (size_t)t->tilem;
   const size_t segs = std::max(t->tilen, t->tilem);
   Workspace w;
-  StripSchedule nsched;
+  StripSchedule nsched;  // (these two outlive the asynchronous copies from them)
+  HostSchedule hs;
   const StripSchedule *sc = &t->strip_sched;
   unsigned char *spare = nullptr;
   size_t spare_bytes = 0;
   if (noalloc) {
     // the tile solver's layout, so that the same systems fit
-    HostSchedule hs;
     build_schedule(t, nwaves, hs);
     Schedule unused;
     unsigned char *base = nullptr;

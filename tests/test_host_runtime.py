@@ -190,3 +190,36 @@ def test_policy_labels_share_no_state_with_products(run):
     tm.spmv(x, y)
     assert launched("k_spmv<0,true>")
     """)
+
+
+NOALLOC = """
+def system(n):
+    # diagonal, two scattered entries a row, every 997th row of 600: strips with pieces
+    rng = np.random.default_rng(n)
+    L = np.full(n, 2)
+    L[::997] = 600
+    r = np.concatenate([np.repeat(np.arange(n), L), np.arange(n)])
+    c = np.concatenate([rng.integers(0, n, L.sum()), np.arange(n)])
+    k = np.unique(r * n + c)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(k // n, minlength=n))]).astype(np.int32)
+    tm = mf.TiledMatrix(rp, (k % n).astype(np.int32), np.ones(len(k)))
+    assert tm.strips()["pieces"] > 0
+    return tm, Vec(tm.npad), Vec(tm.npad)
+"""
+
+
+def test_noalloc_schedules_outlive_their_copies(run):
+    """Copies of host arrays wait until the stream is synchronised; the arrays
+    must still be there then (freed memory is overwritten)."""
+    run(NOALLOC + textwrap.dedent("""
+    for n in (2000, 20000):
+        tm, b, x = system(n)
+        for kw in ({}, {"form": "memory"}, {"policy": "errbound"}, {"policy": "rule"}):
+            log()
+            tm.cg_noalloc(b, x, **kw)
+            l = log()
+            assert any("k_cg_strip" in q for q in l) == (kw in ({}, {"policy": "errbound"})), (kw, l)
+            assert not any(q.startswith("malloc") for q in l), l
+            assert fake.fake_stale_copies() == 0, kw
+        tm.free()
+    """))

@@ -1,7 +1,7 @@
 // The HIP runtime functions that libmillefeuille_hip.so calls, on host memory,
 // for CPU tests of the library's host code: allocations come from a budget,
-// kernels are logged and not run (device memory starts at zero), asynchronous
-// copies happen at the next synchronisation, and event times follow a cost per
+// kernels are logged and not run but for the fill (device memory starts at
+// zero), asynchronous copies happen at the next synchronisation, and event times follow a cost per
 // kernel name.  Loaded with RTLD_GLOBAL before the library, so the library's calls
 // resolve here.
 #include <cstdint>
@@ -16,6 +16,7 @@
 namespace {
 struct Dim3 { uint32_t x, y, z; };
 struct Copy { void *dst; const void *src; std::vector<char> then; int kind; };
+constexpr int kFill = -1;  // (of dst, then.size() bytes, with the word in src)
 std::map<const void *, std::string> names;
 std::map<void *, size_t> live;
 std::vector<Copy> queue;
@@ -29,19 +30,26 @@ alignas(256) char symbol[12 << 20];
 
 void drain() {
   for (Copy &c : queue) {
+    if (c.kind == kFill) {
+      for (size_t i = 0; i < c.then.size(); i += 4) std::memcpy((char *)c.dst + i, &c.src, 4);
+      continue;
+    }
     if (c.kind == 1 && std::memcmp(c.src, c.then.data(), c.then.size())) ++stale;
     std::memcpy(c.dst, c.kind == 1 ? c.then.data() : c.src, c.then.size());
   }
   queue.clear();
 }
 
-int launch(const void *f, Dim3 grid) {
+int launch(const void *f, Dim3 grid, void **args) {
   const std::string &n = names[f];
   log_ += "launch " + n + " " + std::to_string(grid.x) + "\n";
   float us = 1.0f;
   for (auto &c : costs)
     if (n.find(c.first) != std::string::npos) us = c.second;
   clock_us += us;
+  if (n == "mf::k_fill_u32")
+    queue.push_back({*(void **)args[0], (const void *)(uintptr_t)*(uint32_t *)args[2],
+                     std::vector<char>(4 * *(size_t *)args[1]), kFill});
   return 0;
 }
 }  // namespace
@@ -85,8 +93,8 @@ int __hipPopCallConfiguration(Dim3 *g, Dim3 *b, size_t *m, void **s) {
   *s = nullptr;
   return 0;
 }
-int hipLaunchKernel(const void *f, Dim3 g, Dim3, void **, size_t, void *) { return launch(f, g); }
-int hipLaunchCooperativeKernel(const void *f, Dim3 g, Dim3, void **, unsigned, void *) { return launch(f, g); }
+int hipLaunchKernel(const void *f, Dim3 g, Dim3, void **a, size_t, void *) { return launch(f, g, a); }
+int hipLaunchCooperativeKernel(const void *f, Dim3 g, Dim3, void **a, unsigned, void *) { return launch(f, g, a); }
 
 int hipMalloc(void **p, size_t n) {
   log_ += "malloc " + std::to_string(n) + "\n";

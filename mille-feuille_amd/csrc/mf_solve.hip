@@ -1385,10 +1385,11 @@ mf_status fill_u32(void *p, size_t bytes, uint32_t v, hipStream_t st) {
   return MF_OK;
 }
 
-// Carves the workspace and the schedule of a solve out of the scratch array;
-// fails when they do not fit.  Host schedule arrays are copied in.
+// Carves the workspace and the schedule of a tile solve out of the scratch
+// array; fails when they do not fit.  Host schedule arrays are copied in.
+// base == nullptr: only says whether they fit.
 mf_status scratch_layout(const mf_tiled *t, int G, const HostSchedule &hs, unsigned char *base,
-                         Workspace &w, Schedule &sc, hipStream_t st, unsigned char **spare, size_t *spare_bytes) {
+                         Workspace &w, Schedule &sc, hipStream_t st) {
   const size_t n = t->dev.npad, segs = t->tilen > t->tilem ? t->tilen : t->tilem;
   const int nwaves = (int)hs.b.size() - 1, nh = (int)hs.hn.size();
   size_t off = 0;
@@ -1414,9 +1415,7 @@ mf_status scratch_layout(const mf_tiled *t, int G, const HostSchedule &hs, unsig
   const size_t o_mbox = off + mbox_bytes <= kScratchBytes ? off : o_vec + 5 * align256(n * 8);
   if (o_mbox != off && mbox_bytes > n * 8)
     return fail(MF_ERR_ARG, "mf_cg_solve_noalloc: no room for the grid sums' mailboxes");
-  if (o_mbox == off) take(mbox_bytes);
-  *spare = base + off;
-  *spare_bytes = off < kScratchBytes ? kScratchBytes - off : 0;
+  if (!base) return MF_OK;
   unsigned char *v = base + o_vec;
   w.r = (double *)v; v += align256(n * 8);
   w.p = (double *)v; v += align256(n * 8);
@@ -1466,6 +1465,41 @@ mf_status scratch_layout(const mf_tiled *t, int G, const HostSchedule &hs, unsig
   MF_TRY(fill_u32(base + o_mbox, mbox_bytes, 0u, st));
   MF_TRY(fill_u32(base + o_gs, o_tr - o_gs, 0u, st));  // barrier, stats, histogram
   MF_TRY(fill_u32(base + o_hcnt, align256(sizeof(unsigned) * std::max(nh, 1)), 0u, st));
+  return MF_OK;
+}
+
+// Carves what a strip CG and its schedule need out of the scratch array.  Every
+// system whose tile solve fits has room for it: of r, p, r32, p32 (24 bytes a
+// row), the piece sums and their order (20 bytes a piece, half as many pieces as
+// rows at most) it takes 34 bytes a row, of which a tile solve takes 64.
+mf_status strip_scratch(const mf_tiled *t, int G, Workspace &w, StripSchedule &sc, unsigned long long **pmail,
+                        hipStream_t st) {
+  unsigned char *base = nullptr;
+  MF_TRY(scratch_address(t->dev.device, &base));
+  const size_t n = t->dev.npad, segs = std::max(t->tilen, t->tilem), np = sc.piece_order.size();
+  size_t off = 0;
+  auto take = [&](size_t bytes) { const size_t o = off; off += align256(bytes); return base + o; };
+  w.r = (double *)take(n * 8);
+  w.p = (double *)take(n * 8);
+  w.r32 = (float *)take(n * 4);
+  w.p32 = (float *)take(n * 4);
+  w.seg2 = (float *)take(segs * 4);
+  w.partials = (double *)take(2 * kMaxGridSum * (size_t)G * 8);
+  w.mbox = (unsigned long long *)take((size_t)G * kMboxWords * 8);
+  w.gs = (GridSync *)take(sizeof(GridSync));
+  w.stats = (double *)take(kStCount * 8);
+  w.hist = (unsigned long long *)take(5 * 8);
+  *pmail = (unsigned long long *)take(16 * np);
+  sc.d_wave_tr = (int *)take(sizeof(int) * sc.wave_tr.size());
+  sc.d_wave_piece = (int *)take(sizeof(int) * sc.wave_piece.size());
+  sc.d_piece_order = (int *)take(sizeof(int) * np);
+  if (off > kScratchBytes) return fail(MF_ERR_ARG, "mf_cg_solve_noalloc: no room for the row strips' workspace");
+  auto up = [&](int *d, const std::vector<int> &h) {
+    return h.empty() ? hipSuccess : hipMemcpyAsync(d, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice, st);
+  };
+  MF_HIP(up(sc.d_wave_tr, sc.wave_tr));
+  MF_HIP(up(sc.d_wave_piece, sc.wave_piece));
+  MF_HIP(up(sc.d_piece_order, sc.piece_order));
   return MF_OK;
 }
 
@@ -1559,44 +1593,21 @@ static mf_status run_strips(mf_tiled *t, const double *d_b, double *d_x, mf_solv
   const size_t n = t->dev.npad, rows = 16 * (size_t)t->tilem;
   const size_t segs = std::max(t->tilen, t->tilem);
   Workspace w;
-  StripSchedule nsched;  // (these two outlive the asynchronous copies from them)
-  HostSchedule hs;
+  StripSchedule nsched;  // (outlives the asynchronous copies from it)
   const StripSchedule *sc = &t->strip_sched;
-  unsigned char *spare = nullptr;
-  size_t spare_bytes = 0;
+  // Piece sums: in the place of vectors that only the tile solvers use (q .. s:
+  // 24 bytes a row).
+  const size_t mail_bytes = sizeof(unsigned long long) * 2 * (size_t)L.npieces;
+  unsigned long long *pmail = nullptr;
   if (noalloc) {
-    // the tile solver's layout, so that the same systems fit
-    build_schedule(t, nwaves, hs);
-    Schedule unused;
-    unsigned char *base = nullptr;
-    MF_TRY(scratch_address(t->dev.device, &base));
-    MF_TRY(scratch_layout(t, G, hs, base, w, unused, st, &spare, &spare_bytes));
     plan_strip_schedule(t, nwaves, nsched);
     sc = &nsched;
+    MF_TRY(strip_scratch(t, G, w, nsched, &pmail, st));
   } else {
     MF_TRY(ensure_strip_schedule(t, nwaves));
     MF_TRY(get_workspace(t, G, w));
-  }
-  // Piece sums and the allocation-free schedule: behind the scratch layout
-  // where they fit, else in the place of vectors that only the tile solvers
-  // use (q .. s: 24 bytes a row, of at least 100,000 rows then).
-  const size_t mail_bytes = sizeof(unsigned long long) * 2 * (size_t)L.npieces;
-  const size_t need = align256(mail_bytes) + 2 * align256(sizeof(int) * (nwaves + 1)) +
-                      align256(sizeof(int) * (size_t)std::max(L.npieces, 1));
-  unsigned char *c = (unsigned char *)w.q;
-  if (noalloc && need <= spare_bytes) c = spare;
-  else if ((noalloc ? need : mail_bytes) > 24 * n)
-    return fail(MF_ERR_ARG, "solve: no room for the long rows' piece sums");
-  auto take = [&](size_t bytes) { unsigned char *p = c; c += align256(bytes); return p; };
-  unsigned long long *pmail = (unsigned long long *)take(mail_bytes);
-  if (noalloc) {
-    nsched.d_wave_tr = (int *)take(sizeof(int) * (nwaves + 1));
-    nsched.d_wave_piece = (int *)take(sizeof(int) * (nwaves + 1));
-    nsched.d_piece_order = (int *)take(sizeof(int) * std::max<size_t>(nsched.piece_order.size(), 1));
-    MF_HIP(hipMemcpyAsync(nsched.d_wave_tr, nsched.wave_tr.data(), sizeof(int) * (nwaves + 1), hipMemcpyHostToDevice, st));
-    MF_HIP(hipMemcpyAsync(nsched.d_wave_piece, nsched.wave_piece.data(), sizeof(int) * (nwaves + 1), hipMemcpyHostToDevice, st));
-    if (!nsched.piece_order.empty())
-      MF_HIP(hipMemcpyAsync(nsched.d_piece_order, nsched.piece_order.data(), sizeof(int) * nsched.piece_order.size(), hipMemcpyHostToDevice, st));
+    pmail = (unsigned long long *)w.q;
+    if (mail_bytes > 24 * n) return fail(MF_ERR_ARG, "solve: no room for the long rows' piece sums");
   }
   if (opt.policy == MF_POLICY_ERRBOUND && !before && t->tilenum > 0) {
     MF_TRY(apply_errbound_levels(t, st));
@@ -1751,11 +1762,9 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   hipStream_t st = (hipStream_t)opt.stream;
   const int mode = spmv_mode_for(opt.policy);
   if (opt.form < MF_FORM_AUTO || opt.form > MF_FORM_RESIDENT) return fail(MF_ERR_ARG, "solve: unknown form");
-  {
-    int Gs = 0;
-    MF_TRY(strip_grid(t, opt, bicg, &Gs));
-    if (Gs > 0) return run_strips(t, d_b, d_x, opt, rep, Gs, bicg, noalloc);
-  }
+  int Gs = 0;
+  MF_TRY(strip_grid(t, opt, bicg, &Gs));
+  if (Gs > 0 && !noalloc) return run_strips(t, d_b, d_x, opt, rep, Gs, bicg, false);
 
   const void *kern;
   int G = 0;
@@ -1779,6 +1788,13 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
     if (sst != MF_OK) return sst;
     if (noalloc) {
       build_schedule(t, G * kWavesPerBlock, nsched);
+      if (Gs > 0) {
+        // (the limit is the tile solve's, whichever kernel runs)
+        Workspace none;
+        Schedule no_schedule;
+        MF_TRY(scratch_layout(t, G, nsched, nullptr, none, no_schedule, st));
+        return run_strips(t, d_b, d_x, opt, rep, Gs, bicg, true);
+      }
     } else {
       sst = ensure_schedule(t, G * kWavesPerBlock);
       if (sst != MF_OK) return sst;
@@ -1807,9 +1823,7 @@ mf_status run_persistent(mf_tiled *t, const double *d_b, double *d_x, const mf_s
   if (noalloc) {
     unsigned char *base = nullptr;
     MF_TRY(scratch_address(t->dev.device, &base));
-    unsigned char *spare = nullptr;
-    size_t spare_bytes = 0;
-    MF_TRY(scratch_layout(t, G, nsched, base, w, scr_sched, st, &spare, &spare_bytes));
+    MF_TRY(scratch_layout(t, G, nsched, base, w, scr_sched, st));
     sch = &scr_sched;
   } else {
     sst = get_workspace(t, G, w);

@@ -223,3 +223,30 @@ def test_noalloc_schedules_outlive_their_copies(run):
             assert fake.fake_stale_copies() == 0, kw
         tm.free()
     """))
+
+
+def test_noalloc_takes_the_same_systems_over_strips_as_over_tiles(run):
+    """On both sides of the largest system whose tile solve fits the scratch."""
+    run(NOALLOC + textwrap.dedent("""
+    def accepted(n, **kw):
+        tm, b, x = system(n)
+        log()
+        try:
+            tm.cg_noalloc(b, x, **kw)
+            l = log()
+            assert any("k_cg_strip" in q for q in l) == (not kw), l
+            return True
+        except mf.MfError as e:
+            assert e.code == -1, e
+            return False
+        finally:
+            tm.free()
+
+    lo, hi = 120000, 200000  # fits, does not
+    assert accepted(lo, form="memory") and not accepted(hi, form="memory")
+    while hi - lo > 32:
+        n = (lo + hi) // 2
+        lo, hi = (n, hi) if accepted(n, form="memory") else (lo, n)
+    for n in range(lo - 64, hi + 64, 16):
+        assert accepted(n) == accepted(n, form="memory"), n
+    """))

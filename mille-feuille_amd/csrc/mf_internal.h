@@ -158,7 +158,7 @@ struct StripLayout {
   int nmulti = 0;    // rows longer than a piece
   int sorted = 0;    // rows sorted by length inside windows of strips
   int leads = 0;     // half of the strips or more have a lead
-  bool lean = false; // a product over strips reads fewer bytes than over tiles (lean_strips)
+  bool lean = false; // an FP64 product reads at most 1.2 times the tiles' bytes (lean_strips)
   StripDesc *desc = nullptr;
   uint32_t *words = nullptr;
   double *vv = nullptr;
@@ -253,6 +253,7 @@ void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo
 void free_strips(mf_tiled *t);
 int64_t strip_bytes(const StripLayout &L);  // of the layout that an FP64 product reads
 bool lean_strips(const mf_tiled *t);
+bool strips_for_product(const mf_tiled *t);
 void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s);
 void free_device(mf_tiled *t);
 // nnz-balanced contiguous tile-row partition for `nwaves` waves.
@@ -278,7 +279,7 @@ int cut_pieces(const mf_tiled *t, int r, int h, int max_tiles, int max_slots, in
 // them (such a descriptor walks several windows).
 void window_partition_range(const mf_tiled *t, int r0, int r1, int target_nnz,
                             std::vector<WaveDesc> &out);
-// Default stand-alone SpMV kernel (MF_SPMV_STREAM or MF_SPMV_ROWGROUP).
+// Default stand-alone SpMV kernel of mode 0 (MF_SPMV_STREAM or MF_SPMV_STRIP).
 int default_spmv_kernel(const mf_tiled *t);
 // No tile-row holds more than 4x the mean tile count + 8 (the row-group
 // kernel, one tile-row per 16 lanes, wastes little on such matrices).

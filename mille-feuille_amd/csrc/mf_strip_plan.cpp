@@ -157,6 +157,37 @@ void plan_strips(const mf_tiled *t, const int *rowptr, const std::vector<RowInfo
   P.ok = P.ndiag <= 0xffffffffull && P.npacked <= 0xffffffffull && P.nfull <= 0xffffffffull;
 }
 
+// Bytes that an FP64 product reads of the tiles.
+static double tile_bytes(const mf_tiled *t) { return 9.0 * t->dev.npay + 13.0 * t->tilenum; }
+
+bool lean_strips(const mf_tiled *t) {
+  return t->strips.nstrips > 0 && (double)strip_bytes(t->strips) <= 1.2 * tile_bytes(t);
+}
+
+// The stand-alone FP64 product: each side takes the longer of what its bytes
+// take at 5.5 TB/s and what its longest wave takes.  Streamed tiles: a wave walks
+// a whole tile-row or about 1024 slots, 3.2 us for each 1024 (a tile-row of over
+// 16384 is cut).  Strips: a lane walks its row, 0.12 us a pair of entries; a piece
+// of a long row costs as much as 2 KB.  Fitted to 226 products of kNN graphs, bands
+// and scattered rows of 6 to 700 entries, 8,000 to 500,000 rows, hot and cold:
+// two that it gives to strips lose more than 5% (7%), two that it keeps from
+// them would gain more than 10%.  Both sides on MI355X, us, strips / streamed
+// tiles, hot (cold): 128^3 Laplacian 16.0 / 30.2 (30.6 / 68.9); 160k-row kNN graph
+// 5.0 / 6.2 (11.0 / 12.8), with random values 5.6 / 6.2 (14.2 / 12.7); 200k-row power law
+// 25.8 / 149; bands of 48 entries a row whose longest are cut, 160k rows 29.8 / 17.3;
+// of 75 random ones 23.8 / 22.6 (47.8 / 42.3); of 110, 8,000 rows 9.8 / 7.2.
+bool strips_for_product(const mf_tiled *t) {
+  const StripLayout &L = t->strips;
+  if (!L.lean) return false;
+  int slots = 0, pairs = 0;
+  for (int r = 0; r < t->tilem; ++r)
+    slots = std::max(slots, t->pay_off[t->tile_ptr[r + 1]] - t->pay_off[t->tile_ptr[r]]);
+  for (const StripDesc &d : L.hdesc) pairs = std::max<int>(pairs, d.cls == kStripDiag ? (d.npair + 1) / 2 : d.npair);
+  const double tiles = std::max(1.3 + 3.2 * std::max(1.0, std::min(slots, 16384) / 1024.0), 1.5 + tile_bytes(t) / 5.5e6);
+  const double strips = std::max(1.5 + 0.12 * pairs, 1.5 + (strip_bytes(L) + 2000.0 * L.npieces) / 5.5e6);
+  return 1.06 * strips <= tiles;
+}
+
 void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s) {
   const StripLayout &L = t->strips;
   s.nwaves = nwaves;

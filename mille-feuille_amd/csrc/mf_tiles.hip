@@ -267,24 +267,7 @@ bool regular_tilerows(const mf_tiled *t) {
   return t->dev.max_tiles_per_row <= 4.0 * mean + 8.0;
 }
 
-bool lean_strips(const mf_tiled *t) {
-  // Both kernels run at the rate of their bytes (strips: an entry's word or
-  // value and column, a lead per row; tiles: value, byte and metadata), so the
-  // fewer bytes win, with a margin for what strips save besides.  Measured on
-  // MI355X, strips / streamed tiles, operands in the caches and not: 128^3
-  // 7-point Laplacian (diagonals, 23 against 151 MB) 16.1 / 30.2 and 30.6 / 68.9
-  // us, (packed, 67 MB) 17.5 and 36.7; the same pattern with random values (near, 143 MB) 24.9 / 30.1 and
-  // 57.9 / 68.8; 64-entry bands of random values (near, 65 against 58 MB)
-  // 12.3 / 13.2 and 26.3 / 28.6; 150k-row kNN graph, random values (17
-  // against 19 MB) 5.7 / 6.2 and 16.4 / 13.9; 200k-row power-law graph (packed,
-  // pieces; 16 against 135 MB) 25.8 / 149 and 41 / 215.
-  const StripLayout &L = t->strips;
-  if (L.nstrips == 0) return false;
-  const double tiles = 9.0 * t->dev.npay + 13.0 * t->tilenum;
-  return (double)strip_bytes(L) <= 1.2 * tiles;
-}
-
-int default_spmv_kernel(const mf_tiled *t) { return t->strips.lean ? MF_SPMV_STRIP : MF_SPMV_STREAM; }
+int default_spmv_kernel(const mf_tiled *t) { return strips_for_product(t) ? MF_SPMV_STRIP : MF_SPMV_STREAM; }
 
 // Stand-alone SpMV schedule of about wave_nnz payload slots per wave, heavy
 // tile-rows cut into one-window pieces, uploaded in place of the previous one.

@@ -85,3 +85,65 @@ def test_per_tile_levels_run_on_tiles_and_fall_back_to_strips(mf, oracle, method
     assert rep["fell_back"] == 1 and rep["strips_per_wave"] > 0, rep
     rep = _solve(mf, oracle, tm, m, method, policy=policy, max_refresh=1, refresh_every=2, form="memory")
     assert rep["fell_back"] == 1 and rep["strips_per_wave"] == 0, rep
+
+
+def _rows(n, lens, cols, values, seed=0):
+    """Symmetric matrix: row i gets lens[i] couplings at cols(rng, i-array);
+    diagonally dominant."""
+    rng = np.random.default_rng(seed)
+    r = np.repeat(np.arange(n), lens)
+    c = cols(rng, r)
+    k = np.unique(np.concatenate([r * np.int64(n) + c, c * np.int64(n) + r]))
+    r, c = k // n, k % n
+    up = c > r
+    v = -np.ones(up.sum()) if values == "ones" else -rng.uniform(0.1, 1, up.sum())
+    r, c, v = np.concatenate([r[up], c[up]]), np.concatenate([c[up], r[up]]), np.concatenate([v, v])
+    d = np.bincount(r, -v, minlength=n) + 1.0
+    r, c, v = np.concatenate([r, np.arange(n)]), np.concatenate([c, np.arange(n)]), np.concatenate([v, d])
+    k = np.lexsort((c, r))
+    return np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]).astype(np.int32), c[k].astype(np.int32), v[k]
+
+
+def _matrix(name):
+    from millefeuille import gen
+    rng = np.random.default_rng(1)
+
+    def band(w):
+        return lambda g, r: np.clip(r + g.integers(-w, w + 1, len(r)), 0, r.max())
+
+    return {
+        "lap2d": lambda: gen.laplace2d(64),
+        "lap3d": lambda: gen.laplace3d_scaled(32, seed=2),
+        "convdiff": lambda: gen.convdiff3d(24),
+        "knn": lambda: gen.knn_laplacian(20000, 8, seed=4),
+        "powerlaw": lambda: gen.powerlaw_laplacian(20000, 300000, seed=5),
+        "scattered": lambda: _rows(20000, rng.integers(5, 16, 20000), lambda g, r: g.integers(0, 20000, len(r)), "random"),
+        # rows of 20 to 70 entries around the diagonal, the longest in pieces
+        "wide band, pieces": lambda: _rows(40000, rng.integers(10, 50, 40000), band(160), "ones"),
+        # two rows of 64 run longer than the rest of the chip needs for them all
+        "few long rows": lambda: _rows(8000, np.full(8000, 60), band(240), "ones"),
+        # as many bytes as the tiles, in another order
+        "random band": lambda: _rows(160000, rng.integers(5, 18, 160000), band(60), "random"),
+    }[name]()
+
+
+# kernel of the FP64 product
+@pytest.mark.parametrize("name,strips", [("lap2d", True), ("lap3d", True), ("convdiff", True), ("knn", True),
+                                         ("powerlaw", True), ("scattered", True), ("wide band, pieces", False),
+                                         ("few long rows", False), ("random band", False)])
+def test_default_product(mf, oracle, name, strips):
+    m = _matrix(name)
+    n = len(m[0]) - 1
+    tm = mf.TiledMatrix(*m)
+    assert tm.strips()["strips"] > 0
+    assert tm.spmv_kernel() == (mf._lib.SPMV_STRIP if strips else mf._lib.SPMV_STREAM), tm.strips()
+    assert tm.spmv_kernel(1) == mf._lib.SPMV_STREAM
+    x = np.random.default_rng(0).uniform(-1, 1, n)
+    dx, dy = tm.vector(x), tm.vector()
+    bound = oracle.csr_spmv(m[0], m[1], np.abs(m[2]), np.abs(x))
+    for kernel in ("auto", "strip", "stream"):
+        tm.set_spmv_kernel(kernel)
+        tm.spmv(dx, dy)
+        # (sums of up to 4,000 terms in any order: 2^-53 a term)
+        err = np.abs(dy.get()[:n] - oracle.csr_spmv(*m, x))
+        assert np.all(err <= np.maximum(1e-14, 2.3e-16 * np.diff(m[0])) * bound), kernel

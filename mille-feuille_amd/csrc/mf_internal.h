@@ -158,6 +158,7 @@ struct StripLayout {
   int nmulti = 0;    // rows longer than a piece
   int sorted = 0;    // rows sorted by length inside windows of strips
   int leads = 0;     // half of the strips or more have a lead
+  double work = 0.0; // strip_work
   bool lean = false; // an FP64 product reads at most 1.2 times the tiles' bytes (lean_strips)
   StripDesc *desc = nullptr;
   uint32_t *words = nullptr;
@@ -254,6 +255,10 @@ void free_strips(mf_tiled *t);
 int64_t strip_bytes(const StripLayout &L);  // of the layout that an FP64 product reads
 bool lean_strips(const mf_tiled *t);
 bool strips_for_product(const mf_tiled *t);
+// Microseconds that one block of a persistent solver takes for a product of the
+// whole matrix, over strips and over tiles.
+double strip_work(const StripLayout &L);
+double tile_work(const mf_tiled *t, bool mixed);
 void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s);
 void free_device(mf_tiled *t);
 // nnz-balanced contiguous tile-row partition for `nwaves` waves.

@@ -1539,12 +1539,14 @@ static int want_blocks(const mf_tiled *t, const mf_solve_opts &opt) {
 // FP64 CG iteration on MI355X, 7-point Laplacians): 32^3 16 blocks 8.0, 32 6.3,
 // 64 6.6; 64^3 64 blocks 11.8, 128 9.8, 256 10.3; 80^3 128 blocks 12.8, 256 12.0.
 // Pieces of long rows want more waves: power law, 50k rows 48 blocks 20.4, 96
-// 16.6, 256 18.6; 200k rows 128 blocks 36.9, 200 30.2, 256 29.4.
+// 16.6, 256 18.6; 200k rows 128 blocks 36.9, 200 30.2, 256 29.4.  So do wide rows:
+// a block gets at most 4 us of a product's work (8,000 rows of 40 entries 18.8 us
+// an iteration on 8 blocks, 10.6 on 64; 160k rows of 30 22.6 on 128, 18.0 on 256).
 static int want_strip_blocks(const mf_tiled *t, const mf_solve_opts &opt) {
   if (opt.blocks > 0) return opt.blocks;
   const int rows = t->tilem * 16;
   int want = t->strips.npieces > 0 ? (rows + 511) / 512 : std::min((rows + 1023) / 1024, std::max(128, (rows + 2047) / 2048));
-  want = std::max(4, want);
+  want = std::max({4, want, (int)std::min(t->strips.work / 4.0, (double)kMaxBlocks)});
   return want >= 8 ? (want + 7) / 8 * 8 : want;
 }
 
@@ -1562,13 +1564,19 @@ static hipError_t launch_grid(const void *kern, int G, void **args, hipStream_t 
   return le;
 }
 
-// Grid of a strip solve, or 0 where the tile solver runs: the memory form and
-// per-tile or per-segment levels (FIXED, RULE) need tiles; a handle whose
-// strips read more bytes than its tiles keeps them; rows sorted across
-// tile-rows cannot be inferred per wave (LEARNED); and a wave holds the
-// vectors of at most kMaxWaveStrips strips (2.1M rows on 256 CUs: three FP64
-// vectors of 8 strips are 48 of a lane's 128 registers).  Both sides are
-// measured at k_cg_strip.
+// Grid of a strip solve, or 0 where the tile solver runs.  Tiles take:
+// - the memory form, and per-tile or per-segment levels (FIXED, RULE);
+// - LEARNED on sorted rows: 16 lanes add the segment norms that its features
+//   need, and sorted lanes do not hold a segment's rows;
+// - more strips than the waves hold the vectors of, kMaxWaveStrips each (2,097,152
+//   rows on 256 CUs: three FP64 vectors of 8 strips are 48 of a lane's 128
+//   registers; one strip more and an FP64 iteration takes 56 us instead of 30);
+// - matrices whose product takes a block longer over strips than over tiles
+//   (strip_work), beyond what the vectors on chip save: 0.25 us and 0.3 us per
+//   100k rows.  On MI355X, us an iteration, strips / tiles: 160k rows of 48
+//   entries with pieces 29.7 / 22.2, of 63 50 / 33; error bound, 500k sorted rows of 24
+//   37.9 / 28.5; 1M rows of 13 random ones FP64 43.7 / 39.3.  Both sides on stencils and
+//   graphs are at k_cg_strip.
 static mf_status strip_grid(const mf_tiled *t, const mf_solve_opts &opt, bool bicg, int *G) {
   *G = 0;
   const StripLayout &L = t->strips;
@@ -1579,7 +1587,12 @@ static mf_status strip_grid(const mf_tiled *t, const mf_solve_opts &opt, bool bi
   MF_TRY(grid_for(strip_solve_kernel(kMaxWaveStrips, bicg, pol != MF_POLICY_FP64), want_strip_blocks(t, opt), &g,
                   kBlock, true));
   const int per = (L.nstrips + g * kWavesPerBlock - 1) / (g * kWavesPerBlock);
-  if (per <= kMaxWaveStrips) *G = g;
+  if (per > kMaxWaveStrips) return MF_OK;
+  int ncu = 0, dev = 0;
+  MF_HIP(hipGetDevice(&dev));
+  MF_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  const double tiles = tile_work(t, pol != MF_POLICY_FP64) / std::min(want_blocks(t, opt), ncu);
+  if (L.work / g <= tiles + 0.25 + 3e-6 * t->rowA) *G = g;
   return MF_OK;
 }
 

@@ -170,8 +170,8 @@ bool lean_strips(const mf_tiled *t) {
 // 16384 is cut).  Strips: a lane walks its row, 0.12 us a pair of entries; a piece
 // of a long row costs as much as 2 KB.  Fitted to 226 products of kNN graphs, bands
 // and scattered rows of 6 to 700 entries, 8,000 to 500,000 rows, hot and cold:
-// two that it gives to strips lose more than 5% (7%), two that it keeps from
-// them would gain more than 10%.  Both sides on MI355X, us, strips / streamed
+// three that it gives to strips lose 5 to 9%, two that it keeps from them would
+// gain more than 10%.  Both sides on MI355X, us, strips / streamed
 // tiles, hot (cold): 128^3 Laplacian 16.0 / 30.2 (30.6 / 68.9); 160k-row kNN graph
 // 5.0 / 6.2 (11.0 / 12.8), with random values 5.6 / 6.2 (14.2 / 12.7); 200k-row power law
 // 25.8 / 149; bands of 48 entries a row whose longest are cut, 160k rows 29.8 / 17.3;
@@ -186,6 +186,27 @@ bool strips_for_product(const mf_tiled *t) {
   const double tiles = std::max(1.3 + 3.2 * std::max(1.0, std::min(slots, 16384) / 1024.0), 1.5 + tile_bytes(t) / 5.5e6);
   const double strips = std::max(1.5 + 0.12 * pairs, 1.5 + (strip_bytes(L) + 2000.0 * L.npieces) / 5.5e6);
   return 1.06 * strips <= tiles;
+}
+
+// Fitted to CG on 150 matrices (kNN graphs and bands of 6 to 700 entries a row,
+// 8,000 to 1,000,000 rows) at 8 to 256 blocks, ns: an entry slot 0.24, with its
+// value and column 0.29, half as much again where the rows of a strip come from
+// a sorted window and its lanes gather from 64 lines; a diagonal's slot 0.12; a piece
+// 56 besides its slots.  Tiles: a payload slot 0.28, a tile 0.95; under the mixed
+// policies 0.13 and 2.2, which put the line where the two sides meet.
+double strip_work(const StripLayout &L) {
+  double ns = 56.0 * L.npieces;
+  for (const StripDesc &d : L.hdesc) {
+    if (d.cls == kStripDiag)
+      ns += 64 * 0.12 * (d.npair + 1);
+    else
+      ns += 128 * d.npair * (d.cls == kStripPacked ? 0.24 : 0.29) * (L.sorted ? 1.5 : 1.0);
+  }
+  return 1e-3 * ns;
+}
+
+double tile_work(const mf_tiled *t, bool mixed) {
+  return 1e-3 * (mixed ? 0.13 * t->dev.npay + 2.2 * t->tilenum : 0.28 * t->dev.npay + 0.95 * t->tilenum);
 }
 
 void plan_strip_schedule(const mf_tiled *t, int nwaves, StripSchedule &s) {

@@ -256,6 +256,7 @@ mf_status upload_tiles(mf_tiled *t, int device, const int *rowptr) {
   }
   MF_TRY(build_strips(t, rowptr));
   t->strips.lean = lean_strips(t);
+  t->strips.work = strip_work(t->strips);
   d.spmv_kernel = default_spmv_kernel(t);
   return MF_OK;
 }

@@ -120,7 +120,7 @@ def _matrix(name):
         "scattered": lambda: _rows(20000, rng.integers(5, 16, 20000), lambda g, r: g.integers(0, 20000, len(r)), "random"),
         # rows of 20 to 70 entries around the diagonal, the longest in pieces
         "wide band, pieces": lambda: _rows(40000, rng.integers(10, 50, 40000), band(160), "ones"),
-        # two rows of 64 run longer than the rest of the chip needs for them all
+        # 125 strips whose lanes walk 120 entries each
         "few long rows": lambda: _rows(8000, np.full(8000, 60), band(240), "ones"),
         # as many bytes as the tiles, in another order
         "random band": lambda: _rows(160000, rng.integers(5, 18, 160000), band(60), "random"),
@@ -147,3 +147,31 @@ def test_default_product(mf, oracle, name, strips):
         # (sums of up to 4,000 terms in any order: 2^-53 a term)
         err = np.abs(dy.get()[:n] - oracle.csr_spmv(*m, x))
         assert np.all(err <= np.maximum(1e-14, 2.3e-16 * np.diff(m[0])) * bound), kernel
+
+
+# strips at (FP64, error bound); the last two: rows of 40 to 100 entries in full
+# tiles, half of them in pieces, at as many blocks over strips as over tiles
+@pytest.mark.parametrize("name,blocks,fp64,errbound", [
+    ("lap2d", 0, True, True), ("lap3d", 0, True, True), ("knn", 0, True, True), ("powerlaw", 0, True, True),
+    ("scattered", 0, True, True), ("few long rows", 0, True, True), ("random band", 0, True, False),
+    ("cut rows", 8, False, False), ("cut rows", 16, False, False)])
+def test_solver_of_a_matrix(mf, oracle, name, blocks, fp64, errbound):
+    if name == "cut rows":
+        rng = np.random.default_rng(2)
+        m = _rows(16000, rng.integers(20, 60, 16000), lambda g, r: (r // 64 * 64 + g.integers(0, 64, len(r))), "ones")
+    else:
+        m = _matrix(name)
+    tm = mf.TiledMatrix(*m)
+    for policy, strips in (("fp64", fp64), ("errbound", errbound)):
+        for method in ("cg", "bicgstab"):
+            rep = _solve(mf, oracle, tm, m, method, policy=policy, blocks=blocks)
+            assert (rep["strips_per_wave"] > 0) == strips, (method, policy, rep, tm.strips())
+
+
+def test_wide_rows_get_more_blocks(mf, oracle):
+    """8,000 rows: one for each 1024 rows, and where they are wide as many as their products need."""
+    m = _band(8000, "near")
+    assert _solve(mf, oracle, mf.TiledMatrix(*m), m, "cg", policy="fp64")["grid_blocks"] == 8
+    m = _matrix("few long rows")
+    rep = _solve(mf, oracle, mf.TiledMatrix(*m), m, "cg", policy="fp64")
+    assert rep["grid_blocks"] >= 24 and rep["strips_per_wave"] == 1, rep

@@ -266,8 +266,9 @@ typedef struct mf_solve_opts {
                            tile-row; else as MEMORY).  The report's form_used
                            says which ran; strips count as RESIDENT. */
   int batch_waves;      /* mf_batch_cg_solve: waves per (system, right-hand
-                           side) item, 4, 8 or 16 (0 -> 16 where every system
-                           has row strips and the policy is not FIXED, else 8;
+                           side) item, 4, 8 or 16 (0 -> 16 where the batch
+                           runs over row strips, else 8, see
+                           mf_batch_default_waves;
                            mf_tune_batch picks one) */
   void *stream;         /* hipStream_t */
 } mf_solve_opts;
@@ -441,6 +442,10 @@ mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs,
                             const mf_solve_opts *opts, int *iterations,
                             double *rel_residual, double *per_system_ms,
                             double *total_ms);
+/* Waves per item that mf_batch_cg_solve takes for batch_waves 0: 16 where the
+ * batch runs over row strips, 8 over tiles (0: null argument). */
+int mf_batch_default_waves(mf_tiled *const *systems, int nsys,
+                           const mf_solve_opts *opts);
 
 /* ---------------------------------------------------------------------- */
 /* Autotuner                                                               */

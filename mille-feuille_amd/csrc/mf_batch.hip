@@ -41,6 +41,27 @@ namespace mf {
 constexpr int kBatchWavesDefault = 8;
 constexpr int kStripWavesDefault = 16;
 
+// Strips where every system has them, except at the caller's own levels
+// (FIXED), which are per tile, and where the batch's products cost a block more
+// than over tiles.  An item in its CU: strip_work for strips (four fifths of it
+// with the vectors on chip), 0.58 ns a payload slot and 6.8 a tile for tiles.  Both sides on MI355X, FP64, us an iteration of an
+// item, strips / tiles: 8,000 rows in bands of 39 entries 40 / 156, of 61 of which half the
+// rows are cut into pieces 168 / 232, at 40,000 rows 1741 / 1219; 40,000 scattered
+// rows of 80 2581 / 19782.  (The layout's bytes do not matter: strips that are
+// not lean, without pieces, win as well, 40,000 rows of 59 entries 814 / 955.)
+static bool batch_on_strips(mf_tiled *const *systems, int nsys, int policy) {
+  if (policy == MF_POLICY_FIXED) return false;
+  double strips = 0.0, tiles = 0.0;
+  for (int i = 0; i < nsys; ++i) {
+    const mf_tiled *t = systems[i];
+    if (t->strips.nstrips == 0) return false;
+    const bool on_chip = t->strips.nstrips <= kStripWavesDefault * (policy == MF_POLICY_FP64 ? 8 : 16);
+    strips += (on_chip ? 0.8 : 1.0) * t->strips.work;
+    tiles += 1e-3 * (0.58 * t->dev.npay + 6.8 * t->tilenum);
+  }
+  return strips <= tiles;
+}
+
 __global__ void k_batch_reset(int *head, int nitems, int *iters, double *relres) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < kQueues) head[i] = 0;
@@ -251,6 +272,13 @@ __global__ __launch_bounds__(BLOCK) void k_batch_cg(BatchArgs a) {
 
 using namespace mf;
 
+extern "C" int mf_batch_default_waves(mf_tiled *const *systems, int nsys, const mf_solve_opts *o) {
+  if (!systems || nsys <= 0) return 0;
+  for (int i = 0; i < nsys; ++i)
+    if (!systems[i]) return 0;
+  return batch_on_strips(systems, nsys, o ? o->policy : MF_POLICY_FP64) ? kStripWavesDefault : kBatchWavesDefault;
+}
+
 extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, const double **d_b,
                                        double **d_x, const mf_solve_opts *o, int *iterations,
                                        double *rel_residual, double *per_system_ms,
@@ -306,11 +334,8 @@ extern "C" mf_status mf_batch_cg_solve(mf_tiled **systems, int nsys, int nrhs, c
 
   // per-system levels, schedules and descriptors
   std::vector<BatchSys> hs(nsys);
-  // Strips where every system has them, except at the caller's own levels
-  // (FIXED), which are per tile.
-  bool strips = opt.policy != MF_POLICY_FIXED;
-  for (int i = 0; i < nsys; ++i) strips = strips && systems[i]->strips.nstrips > 0;
-  const int nwv = opt.batch_waves == 0 ? (strips ? kStripWavesDefault : kBatchWavesDefault) : opt.batch_waves;
+  const bool strips = batch_on_strips(systems, nsys, opt.policy);
+  const int nwv = opt.batch_waves == 0 ? mf_batch_default_waves(systems, nsys, &opt) : opt.batch_waves;
   if (nwv != 4 && nwv != 8 && nwv != 16)
     return fail(MF_ERR_ARG, "mf_batch_cg_solve: batch_waves must be 0, 4, 8 or 16");
   const int block = 64 * nwv;

@@ -145,6 +145,7 @@ SIGNATURES = {
     "mf_tune_spmv": (C.c_int, [_vp, C.c_int, C.POINTER(MfTuneReport)]),
     "mf_tune_batch": (C.c_int, [_vp, C.c_int, C.c_int, _vp, _vp, C.POINTER(MfSolveOpts), C.c_int,
                                 C.POINTER(MfTuneReport)]),
+    "mf_batch_default_waves": (C.c_int, [_vp, C.c_int, C.POINTER(MfSolveOpts)]),
     "mf_batch_cg_solve": (C.c_int, [_vp, C.c_int, C.c_int, _vp, _vp, C.POINTER(MfSolveOpts), _vp,
                                     _vp, _vp, C.POINTER(C.c_double)]),
     "mf_last_error": (C.c_char_p, []),

@@ -344,10 +344,9 @@ def batch_cg(systems, bs, nrhs=1, x0=None, allow_not_converged=False, tune_iters
     code = lib.mf_batch_cg_solve(hs, nsys, nrhs, pb, px, C.byref(opts), _p(its), _p(rel), _p(per),
                                  C.byref(tot))
     check("mf_batch_cg_solve", code, allow=(0, 1) if allow_not_converged else (0,))
-    # (the library's default: 16 where the items run on strips)
-    strips = opts.policy != _lib.POLICY_FIXED and all(tm.strips()["strips"] > 0 for tm in systems)
     x = dx.get()
     xs = [x[off[k]:off[k + 1]].reshape(nrhs, tm.npad)[:, : tm.rowA] for k, tm in enumerate(systems)]
     return xs, {"status": code, "iterations": its.reshape(nsys, nrhs),
                 "rel_residual": rel.reshape(nsys, nrhs), "per_system_ms": per,
-                "total_ms": tot.value, "batch_waves": opts.batch_waves or (16 if strips else 8), "tune": tune}
+                "total_ms": tot.value, "batch_waves": opts.batch_waves or lib.mf_batch_default_waves(hs, nsys, C.byref(opts)),
+                "tune": tune}

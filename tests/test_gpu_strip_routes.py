@@ -158,7 +158,7 @@ def test_default_product(mf, oracle, name, strips):
 def test_solver_of_a_matrix(mf, oracle, name, blocks, fp64, errbound):
     if name == "cut rows":
         rng = np.random.default_rng(2)
-        m = _rows(16000, rng.integers(20, 60, 16000), lambda g, r: (r // 64 * 64 + g.integers(0, 64, len(r))), "ones")
+        m = _rows(16000, rng.integers(20, 60, 16000), lambda g, r: (r // 128 * 128 + g.integers(0, 128, len(r))), "ones")
     else:
         m = _matrix(name)
     tm = mf.TiledMatrix(*m)
@@ -175,3 +175,23 @@ def test_wide_rows_get_more_blocks(mf, oracle):
     m = _matrix("few long rows")
     rep = _solve(mf, oracle, mf.TiledMatrix(*m), m, "cg", policy="fp64")
     assert rep["grid_blocks"] >= 24 and rep["strips_per_wave"] == 1, rep
+
+
+@pytest.mark.parametrize("name,policy,strips", [("knn", "fp64", True), ("knn", "errbound", True), ("knn", "fixed", False),
+                                                ("powerlaw", "fp64", True), ("scattered", "errbound", True),
+                                                ("few long rows", "fp64", True), ("wide band, pieces", "errbound", True),
+                                                ("cut rows", "fp64", False), ("cut rows", "errbound", True)])
+def test_batch_of_a_matrix(mf, oracle, name, policy, strips):
+    """Strips unless the pieces of cut rows cost more (16,000 rows fit on chip at the
+    mixed policies); every wave count on both."""
+    rng = np.random.default_rng(2)
+    m = (_rows(16000, rng.integers(20, 60, 16000), lambda g, r: (r // 128 * 128 + g.integers(0, 128, len(r))), "ones")
+         if name == "cut rows" else _matrix(name))
+    n = len(m[0]) - 1
+    tms = [mf.TiledMatrix(*m) for _ in range(2)]
+    bs = [np.random.default_rng(k).uniform(-1, 1, n) for k in range(2)]
+    for waves in (0, 4, 16):
+        xs, rep = mf.batch_cg(tms, bs, tol=TOL, policy=policy, batch_waves=waves)
+        assert rep["batch_waves"] == (waves or (16 if strips else 8)), rep
+        for k in range(2):
+            assert oracle.rel_residual(*m, bs[k], xs[k][0]) <= TOL

@@ -67,6 +67,7 @@ class Slab {
       for (auto &q : parts_) *q.first = (char *)*base + q.second;
     return e;
   }
+  size_t bytes() const { return bytes_; }
   mf_status alloc(void **base) {
     MF_HIP(try_alloc(base));
     return MF_OK;

@@ -382,39 +382,38 @@ static mf_status make_strips(mf_tiled *t, const int *rowptr, bool &no_memory) {
   for (int s = 0; s < nstr; ++s) leads += (P.desc[s].flags & kStripLead) != 0;
   L.leads = 2 * leads >= nstr;
   int *d_safe = nullptr, *d_slot = nullptr, *d_long = nullptr;
+  // (few calls: on a handle of 512 rows the strips' allocations, fills and
+  // launches took 100 of 393 us)
   Slab slab, tmp;
   slab.add(&L.desc, P.desc.size());
+  slab.add(&d_safe, P.safe.size());
   slab.add(&L.words, 128 * np);
-  slab.add(&L.vv, 128 * nf);
-  slab.add(&L.vf, 128 * nf);
   if (P.any_full) slab.add(&L.vc, 128 * nf);
-  if (P.any_near) slab.add(&L.vh, 128 * nf);
   if (P.ndiag) slab.add(&L.dslot, P.ndiag);
-  slab.add(&L.lead64, 64 * (size_t)nstr);
-  slab.add(&L.lead32, 64 * (size_t)nstr);
   if (P.sorted) slab.add(&L.rowmap, P.rowmap.size());
   if (L.nlong > 0) {
     slab.add(&L.lane_long, P.lane_long.size());
     slab.add(&L.lrow, P.lrow.size());
     slab.add(&L.piece_long, P.piece_long.size());
   }
-  tmp.add(&d_safe, P.safe.size());
+  // zero where nothing is stored: from lead64 to the end
+  slab.add(&L.lead64, 64 * (size_t)nstr);
+  slab.add(&L.lead32, 64 * (size_t)nstr);
+  slab.add(&L.vv, 128 * nf);
+  slab.add(&L.vf, 128 * nf);
+  if (P.any_near) slab.add(&L.vh, 128 * nf);
   if (P.sorted) tmp.add(&d_slot, P.slot.size());
   if (L.nlong > 0) tmp.add(&d_long, P.long_of.size());
   void *scratch = nullptr;  // temporaries of the fill
   MF_TRY(alloc(slab, &L.slab));
-  if (!no_memory) MF_TRY(alloc(tmp, &scratch));
+  if (!no_memory && P.sorted) MF_TRY(alloc(tmp, &scratch));
   if (no_memory) return MF_OK;
-  MF_HIP(hipMemset(L.lead64, 0, sizeof(double) * 64 * (size_t)nstr));
-  MF_HIP(hipMemset(L.lead32, 0, sizeof(float) * 64 * (size_t)nstr));
-  if (nf > 0) {
-    MF_HIP(hipMemset(L.vv, 0, sizeof(double) * 128 * nf));
-    MF_HIP(hipMemset(L.vf, 0, sizeof(float) * 128 * nf));
-    if (L.vc) MF_HIP(hipMemset(L.vc, 0xff, sizeof(int) * 128 * nf));
-    if (L.vh) MF_HIP(hipMemset(L.vh, 0, sizeof(uint16_t) * 128 * nf));
-  }
+  bool fill = false;
+  for (const StripDesc &d : P.desc) fill = fill || d.cls != kStripDiag;
+  if (fill) MF_HIP(hipMemset(L.lead64, 0, (size_t)((char *)L.slab + slab.bytes() - (char *)L.lead64)));
+  if (L.vc && nf > 0) MF_HIP(hipMemset(L.vc, 0xff, sizeof(int) * 128 * nf));
   mf_status st = upload(L.desc, P.desc);
-  if (st == MF_OK) st = upload(d_safe, P.safe);
+  if (st == MF_OK && np > 0) st = upload(d_safe, P.safe);
   if (st == MF_OK && P.sorted) st = upload(L.rowmap, P.rowmap);
   if (st == MF_OK && P.sorted) st = upload(d_slot, P.slot);
   if (st == MF_OK && L.nlong > 0) {
@@ -424,16 +423,16 @@ static mf_status make_strips(mf_tiled *t, const int *rowptr, bool &no_memory) {
     if (st == MF_OK) st = upload(d_long, P.long_of);
   }
   if (st == MF_OK) {
-    k_pad_words<<<(unsigned)P.desc.size(), 256>>>(L.desc, d_safe, L.words);
+    if (np > 0) k_pad_words<<<(unsigned)P.desc.size(), 256>>>(L.desc, d_safe, L.words);
     FillArgs a{A, L.desc, d_slot, d_long, L.lrow, L.words, L.vv, L.vf, L.vc, L.vh,
                L.lead64, L.lead32, rows, nstr};
-    k_fill_strips<<<(rows + 3) / 4, 256>>>(a);
+    if (fill) k_fill_strips<<<(rows + 3) / 4, 256>>>(a);
     if (P.ndiag) k_diag_slots<true><<<(nstr + 3) / 4, 256>>>(A, rows, nstr, nullptr, L.desc, L.dslot, L.lead64, L.lead32);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) st = fail(MF_ERR_HIP, std::string("build_strips: ") + hipGetErrorString(e));
   }
-  (void)hipFree(scratch);
+  if (scratch) (void)hipFree(scratch);
   if (st == MF_OK) L.nstrips = nstr;
   return st;
 }

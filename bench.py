@@ -88,7 +88,8 @@ def _iteration_roofline(tm, res, method, levels=None):
     out = {}
     for pol, r in res.items():
         mixed = pol != "fp64" and not r["fell_back"]
-        if pol != "rule" and tm.strips()["lean"]:
+        # (the rule, and learned levels on sorted rows, reach strips only by a fallback)
+        if r["strips_per_wave"] and pol != "rule" and not (pol == "learned" and tm.strips()["sorted"]):
             b_it = spmvs * (tm.strips()["bytes"] + (8 if mixed else 16) * tm.rowA)
             us = 1e3 * r["kernel_ms"] / max(r["iterations"], 1)
             gbs = b_it / (us * 1e-6) / 1e9
@@ -134,6 +135,7 @@ def _timed_solves(tm, solve, policies, args, n, rp, ci, va, b, dx):
         res[pol] = {"ms": round(1e3 * sum(out[pol]) / args.steps, 3),
                     "kernel_ms": round(r["time_ms"], 3), "iterations": r["iterations"],
                     "refreshes": r["refreshes"], "fell_back": r["fell_back"], "status": r["status"],
+                    "strips_per_wave": r["strips_per_wave"],
                     "rel_residual_fp64_cpu": rel[pol], "prec_hist": r["prec_hist"]}
         log(f"{pol}: {res[pol]}")
     return res
@@ -366,7 +368,7 @@ def main():
     dxs, dys = tm.vector(xs), tm.vector()
     tune = None
     strip = None
-    if tm.strips()["lean"]:
+    if tm.spmv_kernel_name().startswith("mf::k_spmv_strip"):
         # the default kernel; its bytes are those of the strip layout, x and y
         timer = mf.Timer()
         for _ in range(10):
@@ -485,9 +487,9 @@ def main():
         "laplace2d_64": small,
         "iteration_roofline": _iteration_roofline(
             tm, {policy: {"kernel_ms": rep["time_ms"], "iterations": rep["iterations"],
-                          "fell_back": rep["fell_back"]},
+                          "fell_back": rep["fell_back"], "strips_per_wave": rep["strips_per_wave"]},
                  "fp64": {"kernel_ms": rep64["time_ms"], "iterations": rep64["iterations"],
-                          "fell_back": 0}}, "cg", levels=lv_mixed),
+                          "fell_back": 0, "strips_per_wave": rep64["strips_per_wave"]}}, "cg", levels=lv_mixed),
     }
     if not (rel_cpu <= 1e-10 and rel64 <= 1e-10):
         out["error"] = "FP64-checked residual above 1e-10"

@@ -183,8 +183,8 @@ mf_status mf_spmv(mf_tiled *t, const double *d_x, const float *d_x32,
  * ranges, LDS row accumulators; any sparsity), MF_SPMV_ROWGROUP (one row per
  * lane, four tile-rows per wave; regular sparsity), MF_SPMV_STRIP (mode 0: a
  * layout of row strips built with the handle, one row per lane; mode 1 runs
- * the streamed kernel) or MF_SPMV_AUTO (the default: strips where they are
- * lean, see mf_tile_strip_info, else streamed).
+ * the streamed kernel) or MF_SPMV_AUTO (the default: strips where the handle
+ * has them and they are not expected to be slower, else streamed).
  * No reference counterpart (one kernel form there, src/Mille-feuille-cg.h:97-166). */
 #define MF_SPMV_AUTO (-1)
 #define MF_SPMV_STREAM 0
@@ -198,8 +198,9 @@ mf_status mf_tile_get_spmv_kernel(const mf_tiled *t, int mode, int *kind);
  * none), pieces of rows too long for a strip, whether rows are sorted by
  * length inside windows, and the entry slots (padding included) stored as one
  * 32-bit word, in full, and as diagonals of one value for the strip; bytes: what
- * an FP64 product reads of the layout; lean: that is little enough next to the
- * tiles for strips to be the default.  No reference counterpart. */
+ * an FP64 product reads of the layout; lean: that is at most 1.2 times what it
+ * reads of the tiles.  (A handle has no strips where memory for them is
+ * wanting.)  No reference counterpart. */
 mf_status mf_tile_strip_info(const mf_tiled *t, int *strips, int *pieces, int *sorted,
                              int64_t *packed_slots, int64_t *full_slots, int64_t *diag_slots,
                              int64_t *bytes, int *lean);
@@ -251,20 +252,24 @@ typedef struct mf_solve_opts {
   int blocks;           /* persistent grid size override (0: about 1024 rows
                            per block, at least 4 blocks, at most one block of
                            16 waves per CU; over row strips 2048 rows per block
-                           from 128 blocks on, 512 with pieces of long rows) */
+                           from 128 blocks on, 512 with pieces of long rows,
+                           fewer where rows are wide) */
   int fixed_iters;      /* >0: run exactly this many iterations, no test
                            (reference timing mode, src/Mille-feuille-cg.h:426) */
   int form;             /* solver SpMV form: MF_FORM_MEMORY (every SpMV reads
                            the tile metadata of each wave's windows from HBM),
                            MF_FORM_RESIDENT or MF_FORM_AUTO (FP64, ERRBOUND
-                           and LEARNED on a handle whose row strips are no
-                           larger than its tiles: strips, each wave's vectors
-                           in registers, up to 8 strips a wave.  Else each wave
+                           and, on unsorted rows, LEARNED: over row strips,
+                           each wave's vectors in registers, where a product
+                           over them costs no more than over tiles and a wave
+                           holds at most 8 strips, 2,097,152 rows on 256
+                           CUs.  Else each wave
                            keeps its share's tile metadata in LDS for the
                            whole solve when every share fits a window of 40
                            tile-rows, 256 tiles and 1024 chunks with no heavy
                            tile-row; else as MEMORY).  The report's form_used
-                           says which ran; strips count as RESIDENT. */
+                           says which ran; strips count as RESIDENT, and
+                           strips_per_wave tells them apart. */
   int batch_waves;      /* mf_batch_cg_solve: waves per (system, right-hand
                            side) item, 4, 8 or 16 (0 -> 16 where the batch
                            runs over row strips, else 8, see

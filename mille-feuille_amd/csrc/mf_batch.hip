@@ -15,8 +15,8 @@
 // one.
 //
 // FP64 and error-bound batches of handles with row strips run k_batch_strip
-// (mf_batch_strip.hip).  k_batch_cg, for the caller's own per-tile levels and
-// for handles without strips: an item's 8 waves own nnz-balanced tile-row
+// (mf_batch_strip.hip; batch_on_strips has the rule).  k_batch_cg, for the
+// caller's own per-tile levels and for the others: an item's 8 waves own nnz-balanced tile-row
 // ranges of the system, the SpMV is the streamed wave SpMV, dot products are
 // deterministic block sums and every phase ends at a block barrier.
 // Precision follows the handle's current tile levels with FP64 scalars, FP64

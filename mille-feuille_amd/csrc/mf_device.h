@@ -1784,27 +1784,6 @@ __device__ __forceinline__ void mbox_post(unsigned long long *mb, unsigned epoch
   }
 }
 
-template <int NV>
-__device__ __forceinline__ bool mbox_take(const unsigned long long *mb, unsigned epoch, GridSync *gs,
-                                          double (&v)[NV]) {
-  unsigned long long w[2 * NV];
-  unsigned n = 0;
-  for (;;) {
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < 2 * NV; ++k) {
-      w[k] = __hip_atomic_load(mb + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      ok = ok && (unsigned)(w[k] >> 32) == epoch;
-    }
-    if (ok) break;
-    if (!spin_on(n, gs)) return false;
-  }
-#pragma unroll
-  for (int i = 0; i < NV; ++i)
-    v[i] = __builtin_bit_cast(double, ((w[2 * i + 1] & 0xffffffffull) << 32) | (w[2 * i] & 0xffffffffull));
-  return true;
-}
-
 // mbox: gridDim.x * kMboxWords words, zero before the launch.  lds: NV *
 // 16 doubles.  Blocks of at most 16 waves.
 template <int NV>

@@ -202,11 +202,13 @@ struct Schedule {
   int *wave_heavy = nullptr;      // device, nwaves+1: heavy tile-rows each wave owns
 };
 
-// Schedule of the strip solvers for one wave count: equal contiguous runs of
-// strips, and the pieces of long rows dealt to the waves with the least work.
+// Schedule of the strip solvers for one wave count: the pieces of long rows
+// dealt to the waves with the least work, and equal runs of tile-rows, one per
+// wave, whose narrow levels the error bound reports as one (a wave's unsorted
+// strips are not such a run, and its arithmetic does not depend on the levels).
 struct StripSchedule {
   int nwaves = 0;
-  std::vector<int> wave_tr;      // tile-rows of each wave's strips, nwaves + 1
+  std::vector<int> wave_tr;      // bounds of those tile-rows, nwaves + 1
   std::vector<int> wave_piece;   // bounds of each wave's pieces, nwaves + 1
   std::vector<int> piece_order;  // npieces
   int *d_wave_tr = nullptr, *d_wave_piece = nullptr, *d_piece_order = nullptr;

@@ -28,8 +28,8 @@
 //     products are those of the FP64 values; 4 bytes an entry instead of 9.
 //   near (kStripNear): FP64 and FP32 values and 16-bit column fields.
 //   full (kStripFull): FP64 and FP32 values and 32-bit columns.
-// Padding never touches x (its product is replaced by 0), so an infinity or
-// NaN in x reaches exactly the rows that have an entry in its column.
+// Padding gathers an entry of x that exists, and its product is replaced by 0,
+// so an infinity or NaN in x reaches exactly the rows that have an entry in its column.
 #pragma once
 
 #include <type_traits>

@@ -195,3 +195,23 @@ def test_batch_of_a_matrix(mf, oracle, name, policy, strips):
         assert rep["batch_waves"] == (waves or (16 if strips else 8)), rep
         for k in range(2):
             assert oracle.rel_residual(*m, bs[k], xs[k][0]) <= TOL
+
+
+def test_learned_levels_over_tiles_move_fewer_bytes_than_the_rule(mf, oracle):
+    """Over tiles the levels are what the product reads (9, 5, 3 and 2 bytes an
+    entry with its column): the learned policy moves at most 60% of the FP64
+    payload per product, and less in all than the rule."""
+    from millefeuille import gen
+    m = gen.laplace3d_scaled(32, seed=2)
+    tm = mf.TiledMatrix(*m)
+    _learned(mf, tm)
+    full = 9.0 * tm.csrsize
+    total = {}
+    for policy in ("rule", "learned"):
+        rep = _solve(mf, oracle, tm, m, "cg", policy=policy, form="memory")
+        assert rep["strips_per_wave"] == 0, rep
+        payload = float(np.dot(rep["prec_hist"], [9, 5, 3, 2, 0])) * tm.csrsize / tm.tilenum
+        total[policy] = payload + full * rep["refreshes"]
+        if policy == "learned":
+            assert rep["fell_back"] == 0 and payload <= 0.6 * full * rep["iterations"], rep
+    assert total["learned"] < total["rule"], total
